@@ -38,10 +38,11 @@ hipError_t launch_elem(int d, int p, const PatchDev *patches, const int *gpatch,
 hipError_t launch_elem_range(int d, int p, const PatchDev *patches, const int *gpatch,
                              const int64_t *gprefix, int ng, int64_t e0, int64_t e1, const GaussTab &gt,
                              double *Kbuf, double *Fbuf, double *detmin, hipStream_t s);
-hipError_t launch_l2err(int d, int p, const PatchDev *patches, const int *gpatch,
-                        const int64_t *gprefix, int ng, int64_t nelem, const GaussTab &gt,
-                        const double *sol, int nfree, double *out, double *out_h1, const double *fixed,
-                        hipStream_t s);
+// Blocks of launch_norms for one patch (each writes one partial per norm).
+int64_t norm_blocks(int d, int p, const int *nel);
+hipError_t launch_norms(int d, int p, const PatchDev *patches, const int *gpatch, const int64_t *bprefix, int ng,
+                        int64_t nblocks, const GaussTab &gt, const double *sol, int nfree, double *out,
+                        double *out_h1, const double *fixed, hipStream_t s);
 hipError_t launch_rowcount(const PatchDev *patches, const int *occ_ptr, const int *occ_patch,
                            const int64_t *occ_local, int nfree, int *counts, int *err,
                            hipStream_t s);
@@ -74,7 +75,7 @@ hipError_t launch_keep(const int *rowptr, const int *col, const double *val,
                        int *ncol, double *nval, long long *bsum, long long *total,
                        unsigned long long *dropped, int phase, hipStream_t s);
 hipError_t launch_min(const double *v, int64_t n, double *out, hipStream_t s);
-hipError_t launch_sum(const double *v, int64_t n, double *out, hipStream_t s);
+hipError_t launch_sum_arrays(const double *v, int narr, int64_t n, int64_t stride, double *out, hipStream_t s);
 
 // solve
 int spmv_lpr(double avg_row);

@@ -247,8 +247,9 @@ struct Group {
     int d, p;
     std::vector<int> patches;
     std::vector<int64_t> prefix;
+    std::vector<int64_t> nprefix;   // blocks of the error norm kernel per patch
     int64_t nelem = 0;
-    DevPtr d_gpatch, d_gprefix;
+    DevPtr d_gpatch, d_gprefix, d_nprefix;
 };
 
 struct gsx_problem {
@@ -798,11 +799,19 @@ gsx_status gsx_problem_create(gsx_ctx *c, int32_t npatch, const gsx_patch_desc *
     }
     for (auto &g : P->groups) {
         g.prefix.assign(1, 0);
-        for (int k : g.patches) g.prefix.push_back(g.prefix.back() + P->hp[k].nelem);
+        g.nprefix.assign(1, 0);
+        for (int k : g.patches) {
+            g.prefix.push_back(g.prefix.back() + P->hp[k].nelem);
+            g.nprefix.push_back(g.nprefix.back() + gsx::norm_blocks(g.d, g.p, P->hp[k].nel));
+        }
         g.nelem = g.prefix.back();
         g.d_gpatch = dalloc(c, sizeof(int) * g.patches.size());
         g.d_gprefix = dalloc(c, sizeof(int64_t) * g.prefix.size());
-        if (!g.d_gpatch || !g.d_gprefix) return fail(c, GSX_ERR_OOM, "device allocation (groups)");
+        g.d_nprefix = dalloc(c, sizeof(int64_t) * g.nprefix.size());
+        if (!g.d_gpatch || !g.d_gprefix || !g.d_nprefix)
+            return fail(c, GSX_ERR_OOM, "device allocation (groups)");
+        HIP_OK(c, hipMemcpyAsync(g.d_nprefix.get(), g.nprefix.data(), sizeof(int64_t) * g.nprefix.size(),
+                                 hipMemcpyHostToDevice, s));
         HIP_OK(c, hipMemcpyAsync(g.d_gpatch.get(), g.patches.data(), sizeof(int) * g.patches.size(),
                                  hipMemcpyHostToDevice, s));
         HIP_OK(c, hipMemcpyAsync(g.d_gprefix.get(), g.prefix.data(), sizeof(int64_t) * g.prefix.size(),
@@ -2539,20 +2548,22 @@ gsx_status gsx_error_norms(gsx_problem *P, const double *sol, double *l2, double
     gsx_ctx *c = P->ctx;
     if (P->geo) return fail(c, GSX_ERR_ARG, "error norms need the problem's own geometry");
     hipStream_t s = c->stream;
-    const int64_t ne = std::max<int64_t>(1, P->nelem);
-    DevPtr per = dalloc(c, sizeof(double) * 2 * (ne + 1));
+    int64_t nblk = 0;   // partial sums: one per block, then the two totals
+    for (auto &g : P->groups) nblk += g.nprefix.back();
+    DevPtr per = dalloc(c, sizeof(double) * (2 * nblk + 2));
     if (!per) return fail(c, GSX_ERR_OOM, "device allocation (error norms)");
-    double *pl2 = dp<double>(per), *ph1 = pl2 + ne + 1;
-    for (auto &g : P->groups)
-        HIP_OK(c, gsx::launch_l2err(g.d, g.p, dp<PatchDev>(P->d_patches), dp<int>(g.d_gpatch),
-                                    dp<int64_t>(g.d_gprefix), (int)g.patches.size(), g.nelem, c->gt,
-                                    sol, P->nfree, pl2, h1semi ? ph1 : nullptr,
+    double *pl2 = dp<double>(per), *ph1 = h1semi ? pl2 + nblk : nullptr, *ptot = pl2 + 2 * nblk;
+    int64_t off = 0;
+    for (auto &g : P->groups) {
+        HIP_OK(c, gsx::launch_norms(g.d, g.p, dp<PatchDev>(P->d_patches), dp<int>(g.d_gpatch),
+                                    dp<int64_t>(g.d_nprefix), (int)g.patches.size(), g.nprefix.back(), c->gt, sol,
+                                    P->nfree, pl2 + off, ph1 ? ph1 + off : nullptr,
                                     P->d_fixed ? dp<double>(P->d_fixed) : nullptr, s));
-    HIP_OK(c, gsx::launch_sum(pl2, P->nelem, pl2 + ne, s));
-    if (h1semi) HIP_OK(c, gsx::launch_sum(ph1, P->nelem, ph1 + ne, s));
+        off += g.nprefix.back();
+    }
+    HIP_OK(c, gsx::launch_sum_arrays(pl2, h1semi ? 2 : 1, nblk, nblk, ptot, s));
     double tot[2] = {0.0, 0.0};
-    HIP_OK(c, hipMemcpyAsync(&tot[0], pl2 + ne, sizeof(double), hipMemcpyDeviceToHost, s));
-    if (h1semi) HIP_OK(c, hipMemcpyAsync(&tot[1], ph1 + ne, sizeof(double), hipMemcpyDeviceToHost, s));
+    HIP_OK(c, hipMemcpyAsync(tot, ptot, sizeof(double) * (h1semi ? 2 : 1), hipMemcpyDeviceToHost, s));
     HIP_OK(c, hipStreamSynchronize(s));
     if (l2) *l2 = std::sqrt(tot[0]);
     if (h1semi) *h1semi = std::sqrt(tot[1]);
