@@ -245,6 +245,21 @@ hipError_t launch_cg2_dot_f32(int n, const float *a, const float *b, double *par
 // direction dir of the m0 x m1 x m2 box (element (a,b,c) of x at
 // xo + a + b xs1 + c xs2, of y at yo + a + b ys1 + c ys2); with l0 != null
 // the result is divided by alpha + l0[a] + l1[b] (+ l2[c])
+// Two mode products per launch on the matrix cores (gsx_fd.hip), where
+// fd_fused says the strips fit the LDS.
+bool fd_fused(int d, int m0, int m1, int m2, size_t esz);
+hipError_t launch_fd_pair_f64(int m0, int m1, int m2, const double *M0, const double *M1, const double *x, int64_t xo,
+                              int64_t xs1, int64_t xs2, double *y, int64_t yo, int64_t ys1, int64_t ys2,
+                              const double *l0, const double *l1, double alpha, const CGState *st, hipStream_t s);
+hipError_t launch_fd_pair_f32(int m0, int m1, int m2, const float *M0, const float *M1, const float *x, int64_t xo,
+                              int64_t xs1, int64_t xs2, float *y, int64_t yo, int64_t ys1, int64_t ys2,
+                              const double *l0, const double *l1, double alpha, const CGState *st, hipStream_t s);
+hipError_t launch_fd_column_f64(int m0, int m1, int m2, const double *Q, const double *QT, const double *x, double *y,
+                                const double *l0, const double *l1, const double *l2, double alpha,
+                                const CGState *st, hipStream_t s);
+hipError_t launch_fd_column_f32(int m0, int m1, int m2, const float *Q, const float *QT, const float *x, float *y,
+                                const double *l0, const double *l1, const double *l2, double alpha,
+                                const CGState *st, hipStream_t s);
 hipError_t launch_fd_mode_f64(int m0, int m1, int m2, int dir, const double *M, const double *x, int64_t xo,
                               int64_t xs1, int64_t xs2, double *y, int64_t yo, int64_t ys1, int64_t ys2,
                               const double *l0, const double *l1, const double *l2, double alpha,

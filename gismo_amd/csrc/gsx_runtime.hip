@@ -1920,8 +1920,42 @@ static hipError_t scms_apply(const gsx_fd *F, const T *x, int64_t xo, int64_t xs
     return first ? hipErrorInvalidValue : hipSuccess;
 }
 
+static hipError_t fd_pair(const gsx_fd *F, bool forward, const double *x, int64_t xo, int64_t xs1, int64_t xs2,
+                          double *y, int64_t yo, int64_t ys1, int64_t ys2, const double *l0, const double *l1,
+                          const gsx::CGState *st, hipStream_t s)
+{
+    return gsx::launch_fd_pair_f64(F->m[0], F->m[1], F->m[2], dp<double>(forward ? F->Q64[0] : F->QT64[0]),
+                                   dp<double>(forward ? F->Q64[1] : F->QT64[1]), x, xo, xs1, xs2, y, yo, ys1, ys2, l0,
+                                   l1, F->alpha, st, s);
+}
+
+static hipError_t fd_pair(const gsx_fd *F, bool forward, const float *x, int64_t xo, int64_t xs1, int64_t xs2,
+                          float *y, int64_t yo, int64_t ys1, int64_t ys2, const double *l0, const double *l1,
+                          const gsx::CGState *st, hipStream_t s)
+{
+    return gsx::launch_fd_pair_f32(F->m[0], F->m[1], F->m[2], dp<float>(forward ? F->Q32[0] : F->QT32[0]),
+                                   dp<float>(forward ? F->Q32[1] : F->QT32[1]), x, xo, xs1, xs2, y, yo, ys1, ys2, l0,
+                                   l1, F->alpha, st, s);
+}
+
+static hipError_t fd_column(const gsx_fd *F, const double *x, double *y, const double *l0, const double *l1,
+                            const double *l2, const gsx::CGState *st, hipStream_t s)
+{
+    return gsx::launch_fd_column_f64(F->m[0], F->m[1], F->m[2], dp<double>(F->Q64[2]), dp<double>(F->QT64[2]), x, y,
+                                     l0, l1, l2, F->alpha, st, s);
+}
+
+static hipError_t fd_column(const gsx_fd *F, const float *x, float *y, const double *l0, const double *l1,
+                            const double *l2, const gsx::CGState *st, hipStream_t s)
+{
+    return gsx::launch_fd_column_f32(F->m[0], F->m[1], F->m[2], dp<float>(F->Q32[2]), dp<float>(F->QT32[2]), x, y,
+                                     l0, l1, l2, F->alpha, st, s);
+}
+
 // y = FD(x): element (a,b,c) of x at xo + a + b xs1 + c xs2 (likewise y); the
-// 2d mode products alternate between the two compact scratch tensors.
+// intermediate tensors are compact.  The directions of a plane commute, so
+// the forward and the backward pass both take direction 1 first.  Boxes too
+// large for the fused kernels take the 2d mode products one by one.
 template <typename T>
 static hipError_t fd_apply(const gsx_fd *F, const T *x, int64_t xo, int64_t xs1, int64_t xs2, T *y, int64_t yo,
                            int64_t ys1, int64_t ys2, const gsx::CGState *st, hipStream_t s)
@@ -1933,6 +1967,14 @@ static hipError_t fd_apply(const gsx_fd *F, const T *x, int64_t xo, int64_t xs1,
     const int D = F->d, m0 = F->m[0], m1 = F->m[1], m2 = F->m[2];
     const double *l0 = dp<double>(F->lam[0]), *l1 = dp<double>(F->lam[1]);
     const double *l2 = D == 3 ? dp<double>(F->lam[2]) : nullptr;
+    if (gsx::fd_fused(D, m0, m1, m2, sizeof(T))) {
+        const int64_t c1 = m0, c2 = (int64_t)m0 * m1;
+        hipError_t e = fd_pair(F, true, x, xo, xs1, xs2, buf[0], 0, c1, c2, D == 2 ? l0 : nullptr, l1, st, s);
+        if (e == hipSuccess && D == 3) e = fd_column(F, buf[0], buf[1], l0, l1, l2, st, s);
+        if (e == hipSuccess)
+            e = fd_pair(F, false, D == 3 ? buf[1] : buf[0], 0, c1, c2, y, yo, ys1, ys2, nullptr, nullptr, st, s);
+        return e;
+    }
     const T *in = x;
     int64_t io = xo, is1 = xs1, is2 = xs2;
     for (int k = 0; k < 2 * D; ++k) {

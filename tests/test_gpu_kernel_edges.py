@@ -38,3 +38,45 @@ def test_error_norms_columns(ctx, d, p, n):
     assert h1 == pytest.approx(O.h1_error(prob.patches, dofs, nfree, sol), rel=1e-11)
     x.close()
     gp.close()
+
+
+# strips and tiles of 16 outputs; the last box exceeds the strips' LDS (one
+# mode product per launch)
+@pytest.mark.parametrize("d,p,n", [(2, 1, (2, 2)), (2, 1, (17, 16)), (2, 2, (15, 33)), (2, 3, (3, 130)),
+                                   (3, 1, (2, 2, 2)), (3, 2, (16, 15, 17)), (3, 3, (5, 31, 2)), (3, 4, (14, 2, 15)),
+                                   (2, 1, (530, 3))])
+def test_fd_apply_tiles(ctx, d, p, n):
+    prob = _noisy_box(d, p, n, kappa=False)
+    sides = [s for _, s in prob.dir_sides]
+    gp = gsx.Problem(ctx, prob)
+    fd = gsx.FastDiag(gp)
+    r = np.random.default_rng(7).standard_normal(gp.nfree)
+    want = O.fd_operator(prob.patches[0], sides)(r)
+    rd, zd = ctx.to_device(r), ctx.array(gp.nfree)
+    fd.apply(rd, zd)
+    # sums of up to 2 (m0 + m1 + m2) terms of both eigenbases in FP64
+    assert np.abs(zd.download() - want).max() <= 1e-11 * np.abs(want).max()
+    for o in (rd, zd, fd, gp):
+        o.close()
+
+
+@pytest.mark.parametrize("d,p,n", [(2, 2, (17, 31)), (3, 2, (16, 5, 15)), (3, 3, (6, 14, 7))])
+def test_fd_pcg_fp32_tiles(ctx, d, p, n):
+    """FP32 iterations (FP32 factors) reach the FP64 solution."""
+    prob = _noisy_box(d, p, n)
+    dofs, nfree = O.mapper(prob.patches, prob.dir_sides, prob.ifaces)
+    Ao, bo = O.assemble(prob.patches, dofs, nfree, 0)
+    gp = gsx.Problem(ctx, prob)
+    A, b = gp.assemble(gsx.PATTERN_EXPR, gsx.MIXED)
+    fd = gsx.FastDiag(gp)
+    its = []
+    for prec in (gsx.FP64, gsx.MIXED):
+        x = ctx.array(gp.nfree).zero()
+        it, rel, ok = gsx.fd_cg_solve(A, fd, b, x, tol=1e-10, maxit=300, precision=prec)
+        xs = x.download()
+        assert ok and np.linalg.norm(bo - Ao @ xs) <= 1.1e-10 * np.linalg.norm(bo)
+        its.append(it)
+        x.close()
+    assert its[1] <= its[0] + 5, its   # wrong FP32 factors would not precondition
+    for o in (A, b, fd, gp):
+        o.close()
