@@ -97,6 +97,23 @@ struct CGState {
     int frozen;
 };
 
+// The scalars of one iteration of the grid-layout CG: iteration k starts from
+// the np partials of (r, r) and (r, z).  restart: 0 test and continue; 1 the
+// residual has just been replaced by the FP64 one (no test); 2 that, and the
+// direction restarts from z.
+struct CGStep {
+    int k, np, restart, mixed;
+    const double *part_rr, *part_rz;
+    double *hist;
+};
+
+// A structured operator's geometry: rows = the free box m0 x m1 x m2, vectors
+// on the padded grid with strides sy, sz; window: sspmv_window.
+struct SpmvGrid {
+    int d, p, nfree, sy, sz, m0, m1, window;
+    const int *f2g;
+};
+
 // One boundary element: the element of `patch` adjacent to side `side`
 // (1..2d) at element index ei, the condition's type (1 Dirichlet, 2
 // Neumann), data kind (0 zero, 1 manufactured, 2 affine) and values.

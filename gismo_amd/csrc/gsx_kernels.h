@@ -210,26 +210,22 @@ hipError_t launch_scatter_f64_to_grid(int nfree, const int *f2g, const double *s
 hipError_t launch_gather_f64_from_grid(int nfree, const int *f2g, const double *src, double *dst,
                                        hipStream_t s);
 // MODE 1 with st: skipped once the solve stopped or paused at iteration k
-hipError_t launch_sspmv_f64(int d, int p, int mode, int nfree, const int *f2g, int sy, int sz,
-                            const double *sv, const double *x, double *y, const double *b,
-                            double *part, CGState *st, int k, hipStream_t s);
-// FP32 operator in the half-stored layout (stencil_half); m0 x m1 x m2 = the
-// free box (rows lexicographic), m0 m1 m2 == nfree.
-hipError_t launch_sspmv_f32(int d, int p, int mode, int nfree, const int *f2g, int sy, int sz, int m0, int m1,
-                            int m2, const float *sv, const float *x, float *y, const float *b,
-                            double *part, CGState *st, int k, hipStream_t s);
+// Grid entries staged for 256 rows: the largest span of a row tile plus its
+// halo in one plane.
+int sspmv_window(int p, int nfree, int m0, int m1, int sy, int sz);
+hipError_t launch_sspmv_residual(const SpmvGrid &G, const double *sv, const double *x, double *y, const double *b,
+                                 double *part, hipStream_t s);
+hipError_t launch_cg2_spmv_f64(const SpmvGrid &G, const double *sv, const double *z, const double *po, double *pn,
+                               double *t, double *part, const CGStep &cs, CGState *st, hipStream_t s);
+hipError_t launch_cg2_spmv_f32(const SpmvGrid &G, const float *sv, const float *x, const float *po, float *pn,
+                               float *y, double *part, const CGStep &cs, CGState *st, hipStream_t s);
+hipError_t launch_cg2_check(const CGStep &cs, CGState *st, hipStream_t s);
 hipError_t launch_cg2_update_f64(int n, double *x, double *r, const double *p, const double *t,
                                  double *z, const double *diag, double tau, const double *pap,
                                  int npap, double *prr, double *prz, CGState *st, int k, hipStream_t s);
 hipError_t launch_cg2_update_f32(int n, float *x, float *r, const float *p, const float *t, float *z,
                                  const float *diag, double tau, const double *pap, int npap,
                                  double *prr, double *prz, CGState *st, int k, hipStream_t s);
-hipError_t launch_cg2_direction_f64(int n, double *p, const double *z, const double *prr,
-                                    const double *prz, int np, CGState *st, int k, double *hist,
-                                    hipStream_t s);
-hipError_t launch_cg2_direction_f32_mixed(int n, float *p, const float *z, const double *prr,
-                                          const double *prz, int np, CGState *st, int k,
-                                          hipStream_t s);
 // Gauss-Seidel: update the cnt rows listed in rows (one level set)
 hipError_t launch_gs_rows_f64(int cnt, const int *rows, const int *rp, const int *ci, const double *va,
                               const double *b, double *x, hipStream_t s);
@@ -279,11 +275,10 @@ hipError_t launch_tensor_mode_f32(int o0, int o1, int o2, int dir, int m_in, con
                                   int64_t xo, int64_t xs1, int64_t xs2, float *y, int64_t yo, int64_t ys1,
                                   int64_t ys2, int scale, double alpha, const double *l0, const double *l1,
                                   const double *l2, int accumulate, const CGState *st, hipStream_t s);
-hipError_t launch_cg2_precond_f64(int n, const double *r, double *z, const double *diag,
-                                  double tau, double *prz, hipStream_t s);
-hipError_t launch_cg2_precond_f32(int n, const float *r, float *z, const float *diag, double tau,
+hipError_t launch_cg2_precond_f64(int n, const double *r, double *z, const double *diag, double tau, double *prr,
                                   double *prz, hipStream_t s);
-hipError_t launch_set_rz(const double *parts, int np, CGState *st, int slot, hipStream_t s);
+hipError_t launch_cg2_precond_f32(int n, const float *r, float *z, const float *diag, double tau, double *prr,
+                                  double *prz, hipStream_t s);
 hipError_t launch_grid_f64_to_f32(int64_t n, const double *a, float *b, hipStream_t s);
 hipError_t launch_accum_grid(int64_t n, double *x, float *xc, hipStream_t s);
 

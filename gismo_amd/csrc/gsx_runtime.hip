@@ -993,8 +993,9 @@ struct StencilOp {
     DevPtr s32full;                   // all slots in FP32 (batch members that ask for it)
     // grid-layout workspace
     DevPtr diag64, diag32;
-    DevPtr xg, rg, bg, zg, pg, tg;            // FP64
-    DevPtr r32, z32, p32, t32, xc32;          // FP32
+    DevPtr xg, rg, bg, zg, pg[2], tg;         // FP64 (directions by iteration parity)
+    DevPtr r32, z32, p32[2], t32, xc32;       // FP32
+    int window = 0;                           // grid entries a row tile's input spans
     DevPtr parts;
 };
 
@@ -1757,29 +1758,33 @@ static gsx_status stencil_prepare(gsx_matrix *A, bool mixed)
         S.rg = dalloc(c, sizeof(double) * N);
         S.bg = dalloc(c, sizeof(double) * N);
         S.zg = dalloc(c, sizeof(double) * N);
-        S.pg = dalloc(c, sizeof(double) * N);
+        S.pg[0] = dalloc(c, sizeof(double) * N);
+        S.pg[1] = dalloc(c, sizeof(double) * N);
         S.tg = dalloc(c, sizeof(double) * N);
         S.parts = dalloc(c, sizeof(double) * 4 * kPartStride);
-        if (!S.diag64 || !S.xg || !S.rg || !S.bg || !S.zg || !S.pg || !S.tg || !S.parts)
+        if (!S.diag64 || !S.xg || !S.rg || !S.bg || !S.zg || !S.pg[0] || !S.pg[1] || !S.tg ||
+            !S.parts)
             return fail(c, GSX_ERR_OOM, "device allocation (grid workspace)");
         // diagonal = centre slot of the structured operator
         HIP_OK(c, gsx::launch_fill_f64(dp<double>(S.diag64), N, 1.0, s));
         HIP_OK(c, gsx::launch_stencil_diag(n, (int)K, dp<int>(S.f2g), dp<double>(S.s64), dp<double>(S.diag64), s));
-        for (DevPtr *v : {&S.xg, &S.rg, &S.bg, &S.zg, &S.pg, &S.tg})
+        for (DevPtr *v : {&S.xg, &S.rg, &S.bg, &S.zg, &S.pg[0], &S.pg[1], &S.tg})
             HIP_OK(c, gsx::launch_fill_f64(dp<double>(*v), N, 0.0, s));
+        S.window = gsx::sspmv_window(S.p, n, S.m[0], S.m[1], S.nx, S.nx * S.ny);
         S.built = true;
     }
     if (mixed && !S.r32) {
         S.diag32 = dalloc(c, sizeof(float) * N);
         S.r32 = dalloc(c, sizeof(float) * N);
         S.z32 = dalloc(c, sizeof(float) * N);
-        S.p32 = dalloc(c, sizeof(float) * N);
+        S.p32[0] = dalloc(c, sizeof(float) * N);
+        S.p32[1] = dalloc(c, sizeof(float) * N);
         S.t32 = dalloc(c, sizeof(float) * N);
         S.xc32 = dalloc(c, sizeof(float) * N);
-        if (!S.diag32 || !S.r32 || !S.z32 || !S.p32 || !S.t32 || !S.xc32)
+        if (!S.diag32 || !S.r32 || !S.z32 || !S.p32[0] || !S.p32[1] || !S.t32 || !S.xc32)
             return fail(c, GSX_ERR_OOM, "device allocation (grid workspace, fp32)");
         HIP_OK(c, gsx::launch_grid_f64_to_f32(N, dp<double>(S.diag64), dp<float>(S.diag32), s));
-        for (DevPtr *v : {&S.r32, &S.z32, &S.p32, &S.t32, &S.xc32})
+        for (DevPtr *v : {&S.r32, &S.z32, &S.p32[0], &S.p32[1], &S.t32, &S.xc32})
             HIP_OK(c, gsx::launch_fill_f32(dp<float>(*v), N, 0.0f, s));
     }
     return GSX_OK;
@@ -2014,9 +2019,9 @@ static gsx_status cg_grid(gsx_matrix *A, int precond, double tau, const double *
     double *hist = mixed ? nullptr : dp<double>(w.hist);
     const bool jac = precond == GSX_PREC_JACOBI;
     const int *f2g = dp<int>(S.f2g);
-    const int sy = S.nx, sz = S.nx * S.ny;
+    const gsx::SpmvGrid G{S.d, S.p, n, S.nx, S.nx * S.ny, S.m[0], S.m[1], S.window, f2g};
     double *xg = dp<double>(S.xg), *rg = dp<double>(S.rg), *bg = dp<double>(S.bg);
-    double *zg = dp<double>(S.zg), *pg = dp<double>(S.pg), *tg = dp<double>(S.tg);
+    double *zg = dp<double>(S.zg), *tg = dp<double>(S.tg);
     const double *sv = dp<double>(S.s64), *dg = dp<double>(S.diag64);
     CGState h{};
     h.tol = tol;
@@ -2028,105 +2033,104 @@ static gsx_status cg_grid(gsx_matrix *A, int precond, double tau, const double *
         KScope k(c, "cg_init");
         HIP_OK(c, gsx::launch_scatter_f64_to_grid(n, f2g, b, bg, s));
         HIP_OK(c, gsx::launch_scatter_f64_to_grid(n, f2g, x, xg, s));
-        HIP_OK(c, gsx::launch_sspmv_f64(S.d, S.p, 2, n, f2g, sy, sz, sv, xg, rg, bg, P1, nullptr, 0, s));
-        HIP_OK(c, gsx::launch_cg2_precond_f64((int)N, bg, zg, nullptr, 1.0, P0, s));   // ||b||^2
+        HIP_OK(c, gsx::launch_sspmv_residual(G, sv, xg, rg, bg, P1, s));
+        HIP_OK(c, gsx::launch_cg2_dot_f64((int)N, bg, bg, P0, nullptr, s));   // ||b||^2
         HIP_OK(c, gsx::launch_cg_scalar(0, P0, nv, P1, nsp, st, hist, s));
     }
     GSX_TRY(read_state(c, w, h));
     if (h.done == 3) HIP_OK(c, gsx::launch_fill_f64(x, n, 0.0, s));
     int k = 0;
+    gsx::CGStep cs{0, nv, 2, mixed ? 1 : 0, P1, P2, hist};
     // the fast diagonalization applies between the update (which then only
     // moves x and r) and the direction, followed by the (r, z) partials
-    auto fd64 = [&](const gsx::CGState *sp, double *part) -> gsx_status {
+    auto fd64 = [&](const gsx::CGState *sp) -> gsx_status {
         KScope kf(c, "fd_apply");
         HIP_OK(c, fd_apply<double>(fd, rg, fd->goff, fd->gs1, fd->gs2, zg, fd->goff, fd->gs1, fd->gs2, sp, s));
-        HIP_OK(c, gsx::launch_cg2_dot_f64((int)N, rg, zg, part, sp, s));
+        HIP_OK(c, gsx::launch_cg2_dot_f64((int)N, rg, zg, P2, sp, s));
         return GSX_OK;
     };
     if (!h.done && !mixed) {
-        if (fd) {
-            GSX_TRY(fd64(nullptr, P0));
-        } else {
-            HIP_OK(c, gsx::launch_cg2_precond_f64((int)N, rg, zg, jac ? dg : nullptr, tau, P0, s));
-        }
-        HIP_OK(c, gsx::launch_set_rz(P0, nv, st, 0, s));
-        HIP_OK(c, hipMemcpyAsync(pg, zg, sizeof(double) * N, hipMemcpyDeviceToDevice, s));
+        HIP_OK(c, gsx::launch_cg2_precond_f64((int)N, rg, zg, jac && !fd ? dg : nullptr, tau, P1, P2, s));
+        if (fd) GSX_TRY(fd64(nullptr));
         const int chunk = 16;
         while (k < maxit) {
             const int kend = std::min(maxit, k + chunk);
             for (; k < kend; ++k) {
+                double *pn = dp<double>(S.pg[k & 1]);
+                cs.k = k;
                 {
                     KScope ks(c, "spmv_f64");
-                    HIP_OK(c, gsx::launch_sspmv_f64(S.d, S.p, 1, n, f2g, sy, sz, sv, pg, tg, nullptr, P0, st, k, s));
+                    HIP_OK(c, gsx::launch_cg2_spmv_f64(G, sv, zg, dp<double>(S.pg[(k + 1) & 1]), pn, tg, P0, cs, st, s));
                 }
+                cs.restart = 0;
                 {
                     KScope kv(c, "cg_vec");
-                    HIP_OK(c, gsx::launch_cg2_update_f64((int)N, xg, rg, pg, tg, zg, jac && !fd ? dg : nullptr, tau,
+                    HIP_OK(c, gsx::launch_cg2_update_f64((int)N, xg, rg, pn, tg, zg, jac && !fd ? dg : nullptr, tau,
                                                          P0, nsp, P1, P2, st, k, s));
                 }
-                if (fd) GSX_TRY(fd64(st, P2));
-                KScope kv(c, "cg_vec");
-                HIP_OK(c, gsx::launch_cg2_direction_f64((int)N, pg, zg, P1, P2, nv, st, k, hist, s));
+                if (fd) GSX_TRY(fd64(st));
             }
+            cs.k = k;
+            HIP_OK(c, gsx::launch_cg2_check(cs, st, s));
             GSX_TRY(read_state(c, w, h));
             if (h.done) break;
         }
         HIP_OK(c, gsx::launch_gather_f64_from_grid(n, f2g, xg, x, s));
     } else if (!h.done && mixed) {
-        float *r32 = dp<float>(S.r32), *z32 = dp<float>(S.z32), *p32 = dp<float>(S.p32);
+        float *r32 = dp<float>(S.r32), *z32 = dp<float>(S.z32);
         float *t32 = dp<float>(S.t32), *xc = dp<float>(S.xc32);
         const float *sv32 = dp<float>(S.s32), *d32 = dp<float>(S.diag32);
-        auto fd32 = [&](const gsx::CGState *sp, double *part) -> gsx_status {
+        auto fd32 = [&](const gsx::CGState *sp) -> gsx_status {
             KScope kf(c, "fd_apply_f32");
             HIP_OK(c, fd_apply<float>(fd, r32, fd->goff, fd->gs1, fd->gs2, z32, fd->goff, fd->gs1, fd->gs2, sp, s));
-            HIP_OK(c, gsx::launch_cg2_dot_f32((int)N, r32, z32, part, sp, s));
+            HIP_OK(c, gsx::launch_cg2_dot_f32((int)N, r32, z32, P2, sp, s));
             return GSX_OK;
         };
-        auto restart = [&](int slot) -> gsx_status {
+        // r32 = fp32(r64), z32 = M r32 and their partials, from which the
+        // next iteration takes its direction
+        auto restart = [&]() -> gsx_status {
             HIP_OK(c, gsx::launch_grid_f64_to_f32(N, rg, r32, s));
-            if (fd) {
-                GSX_TRY(fd32(nullptr, P0));
-            } else {
-                HIP_OK(c, gsx::launch_cg2_precond_f32((int)N, r32, z32, jac ? d32 : nullptr, tau, P0, s));
-            }
-            HIP_OK(c, gsx::launch_set_rz(P0, nv, st, slot, s));
+            HIP_OK(c, gsx::launch_cg2_precond_f32((int)N, r32, z32, jac && !fd ? d32 : nullptr, tau, P1, P2, s));
+            if (fd) GSX_TRY(fd32(nullptr));
             return GSX_OK;
         };
         HIP_OK(c, gsx::launch_fill_f32(xc, N, 0.0f, s));
-        GSX_TRY(restart(0));
-        HIP_OK(c, hipMemcpyAsync(p32, z32, sizeof(float) * N, hipMemcpyDeviceToDevice, s));
+        GSX_TRY(restart());
         const int chunk = 8;
         while (true) {
-            for (int j = 0; j < chunk; ++j, ++k) {
+            const int kend = std::min(maxit, k + chunk);
+            for (; k < kend; ++k) {
+                float *pn = dp<float>(S.p32[k & 1]);
+                cs.k = k;
                 {
                     KScope ks(c, "spmv_f32");
-                    HIP_OK(c, gsx::launch_sspmv_f32(S.d, S.p, 1, n, f2g, sy, sz, S.m[0], S.m[1], S.m[2], sv32, p32,
-                                                    t32, nullptr, P0, st, k, s));
+                    HIP_OK(c, gsx::launch_cg2_spmv_f32(G, sv32, z32, dp<float>(S.p32[(k + 1) & 1]), pn, t32, P0, cs,
+                                                       st, s));
                 }
+                cs.restart = 0;
                 {
                     KScope kv(c, "cg_vec_f32");
-                    HIP_OK(c, gsx::launch_cg2_update_f32((int)N, xc, r32, p32, t32, z32, jac && !fd ? d32 : nullptr,
+                    HIP_OK(c, gsx::launch_cg2_update_f32((int)N, xc, r32, pn, t32, z32, jac && !fd ? d32 : nullptr,
                                                          tau, P0, nsp, P1, P2, st, k, s));
                 }
-                if (fd) GSX_TRY(fd32(st, P2));
-                KScope kv(c, "cg_vec_f32");
-                HIP_OK(c, gsx::launch_cg2_direction_f32_mixed((int)N, p32, z32, P1, P2, nv, st, k, s));
+                if (fd) GSX_TRY(fd32(st));
             }
+            cs.k = k;
+            HIP_OK(c, gsx::launch_cg2_check(cs, st, s));
             GSX_TRY(read_state(c, w, h));
             k = h.it;
             if (h.need_update || h.done == 2 || h.err < tol) {
                 KScope kr(c, "reliable_update");
                 const double rr_rec = h.rr;   // the FP32 recurrence's residual
                 HIP_OK(c, gsx::launch_accum_grid(N, xg, xc, s));
-                HIP_OK(c, gsx::launch_sspmv_f64(S.d, S.p, 2, n, f2g, sy, sz, sv, xg, rg, bg, P1, nullptr, 0, s));
+                HIP_OK(c, gsx::launch_sspmv_residual(G, sv, xg, rg, bg, P1, s));
                 HIP_OK(c, gsx::launch_cg_reliable(P1, nsp, st, nullptr, s));
                 GSX_TRY(read_state(c, w, h));
                 if (h.done == 1 || h.done == 2) break;
-                GSX_TRY(restart(k));
+                GSX_TRY(restart());
                 // a recurrence that has parted from the true residual (it
                 // ran into its FP32 floor) leaves no usable direction
-                if (rr_rec < gsx::kDirectionReset * h.rr)
-                    HIP_OK(c, hipMemcpyAsync(p32, z32, sizeof(float) * N, hipMemcpyDeviceToDevice, s));
+                cs.restart = rr_rec < gsx::kDirectionReset * h.rr ? 2 : 1;
             }
             if (h.it >= maxit) break;
         }

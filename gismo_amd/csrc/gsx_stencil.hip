@@ -12,37 +12,71 @@
 // as the CSR SpMV (columns ascending = grid order).
 //
 // CG (gsConjugateGradient::step, src/gsSolver/gsConjugateGradient.hpp:55-93)
-// in three launches per iteration: SpMV + partial (p, Ap); update
-// (x, r, z = tau r / diag, partial (r,r), (r,z)); direction update
-// (p = z + beta p).  Every block of a launch sums the previous launch's
-// partials itself (bounded counts, fixed order) and derives alpha or beta,
-// so there is no single-block reduction kernel in the loop; block 0 records
-// the scalars.  The (r,z) of iteration k lives in slot k & 1.
+// in two launches per iteration: k_cg2_spmv tests the last residual, forms the
+// direction p = z + beta p where it stages its input, applies the operator and
+// writes partial (p, A p); k_cg2_update moves x and r, applies the Jacobi
+// preconditioner and writes partial (r, r), (r, z).  Every block of a launch
+// sums the previous launch's partials itself (bounded counts, fixed order) and
+// derives alpha or beta, so there is no single-block reduction kernel in the
+// loop; block 0 records the scalars.  The direction of iteration k lives in
+// buffer k & 1 (neighbouring blocks still read the old one while the new one
+// is written), its (r, z) in slot k & 1.
 #include "gsx_common.h"
 #include "gsx_kernels.h"
+
+#include <algorithm>
 
 namespace gsx {
 
 constexpr int kMaxPartials = 2048;
 
-// block sum of 256 threads: wavefront shuffles, then the 4 wave sums in
-// wave order (fixed order: bitwise reproducible)
-__device__ inline double bsum256(double v, double *s)
+constexpr int kVecThreads = 512;   // threads of the vector kernels' blocks
+
+// block sum of NT threads: wavefront shuffles, then the wave sums in wave
+// order (fixed order: bitwise reproducible)
+template <int NT>
+__device__ inline double bsum(double v, double *s)
 {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
     __syncthreads();
-    const double r = (s[0] + s[1]) + (s[2] + s[3]);
+    double r = 0.0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) r += s[w];
     __syncthreads();
     return r;
 }
 
+// two sums with one pair of barriers (s: 2 NT / 64 doubles)
+template <int NT>
+__device__ inline void bsum2(double &a, double &b, double *s)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        a += __shfl_xor(a, off, 64);
+        b += __shfl_xor(b, off, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        s[threadIdx.x >> 6] = a;
+        s[NT / 64 + (threadIdx.x >> 6)] = b;
+    }
+    __syncthreads();
+    a = b = 0.0;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) {
+        a += s[w];
+        b += s[NT / 64 + w];
+    }
+    __syncthreads();
+}
+
+template <int NT>
 __device__ inline double sum_partials(const double *__restrict__ p, int np, double *s)
 {
     double a = 0.0;
-    for (int i = threadIdx.x; i < np; i += 256) a += p[i];
-    return bsum256(a, s);
+    for (int i = threadIdx.x; i < np; i += NT) a += p[i];
+    return bsum<NT>(a, s);
 }
 
 template <typename T>
@@ -100,140 +134,199 @@ __global__ void k_gather_from_grid(int nfree, const int *__restrict__ free2grid,
 }
 
 // ---------------------------------------------------------------------------
-// Stencil SpMV.  MODE 0: y = A x; 1: y = A x, partial (x, y); 2: y = b - A x,
-// partial (y, y).  Vectors on the grid; rows = free functions.
+// Stencil SpMV.  Vectors on the grid; rows = free functions, the free box
+// m0 x m1 x m2 in lexicographic order.  MODE 1, iteration k of CG: stop test,
+// pn = x + beta po (x is the preconditioned residual z), y = A pn, partial
+// (pn, y).  MODE 2: y = b - A x, partial (y, y).
+//
+// KIND 0, the FP32 copy: only the upper slots are stored (stencil_half).
+// KIND 1, 2, the FP64 operator: all slots are stored.  With KIND 0 and 1 an
+// upper slot is read from the row itself and a lower one from the neighbour
+// row at that offset, whose mirrored upper slot holds the same coefficient
+// (the operator is bitwise symmetric): half the bytes of the operator move.
+// Each upper x-line of the stencil, (dz, dy) > 0 lexicographically, is taken
+// together with its mirror line (-dz, -dy): both read the same slot plane, the
+// mirror one at the rows shifted by the offset, so a block reads the plane at
+// the same point of its loop as the blocks that own those rows (up to p
+// z-planes back, on the same XCD through xcd_block) and the second read mostly
+// hits the L2.  Neighbours outside the free box contribute 0 (x is 0 there).
+// KIND 2 reads every slot from the row itself, with fewer index operations.
+//
+// The input of a block's 256 rows is staged in LDS, the window of grid entries
+// around them in planes dz and -dz (a few times the rows' number in entries):
+// it is read from memory once instead of once per coefficient, and in MODE 1
+// the direction is formed there, which saves its own launch.  Windows that do
+// not fit (STAGED = false) are read entry by entry.
+// Bound by the operator's bytes and the mirrored reads that miss the L2.  64^3
+// elements p = 3: FP32 46.1 us with the direction (49 us in two launches
+// before); FP64 residual 109 us (159 us reading all slots).  75^3 p = 2, FP64:
+// 54.5 us with the direction (89 + 7 us reading all slots).
 // ---------------------------------------------------------------------------
-template <int D, int P, typename V, typename T, int MODE>
-__global__ __launch_bounds__(256) void k_sspmv(int nfree, const int *__restrict__ free2grid,
-                                               int sy, int sz, const V *__restrict__ sval,
-                                               const T *__restrict__ x, T *__restrict__ y,
-                                               const T *__restrict__ b,
-                                               double *__restrict__ partial,
-                                               CGState *__restrict__ st, int k)
+template <int D, int P, typename V, typename T, int KIND, int MODE, bool STAGED>
+__global__ __launch_bounds__(256) void k_cg2_spmv(int nfree, const int *__restrict__ free2grid, int sy, int sz,
+                                                  int m0, int m1, const V *__restrict__ sval,
+                                                  const T *__restrict__ x, const T *__restrict__ po,
+                                                  T *__restrict__ pn, T *__restrict__ y, const T *__restrict__ b,
+                                                  double *__restrict__ partial, CGStep cs,
+                                                  CGState *__restrict__ st, int wn)
 {
-    __shared__ double s[4];
-    if (st && (st->done || (st->flag_next && st->flag_next <= k))) return;
+    extern __shared__ double sp_smem[];
+    __shared__ double s[8];
     constexpr int W = 2 * P + 1;
     constexpr int NS = (D == 3) ? W * W * W : W * W;
+    constexpr int C = NS / 2, SL = KIND == 0 ? stencil_half(NS) : NS;   // slots of the stored layout
+    constexpr int UP = KIND == 0 ? 0 : C;                               // stored index of the centre slot
     static_assert(kStencilTile == 256, "one block applies one row tile");
-    double contrib = 0.0;
+    if (MODE == 1 && (st->done || (st->flag_next && st->flag_next <= cs.k))) return;
+    const int halo = P * sy + P;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
-    for (int r = blk * 256 + threadIdx.x; r < nfree; r += gridDim.x * 256) {
-        const int g = free2grid[r];
-        const T *xb = x + g;
-        const V *vb = sval + stencil_index(0, r, NS);
-        T acc = 0;
-        if (D == 3) {
-#pragma unroll 1
-            for (int dz = -P; dz <= P; ++dz) {
+    // the first tile's window is requested before the sums that give beta
+    constexpr int NPRE = MODE == 1 && STAGED ? 4 : 1;
+    T prx[NPRE], prp[NPRE];
+    int w0 = 0, w1 = 0;
+    if (MODE == 1 && STAGED) {
+        w0 = free2grid[blk * 256] - halo;
+        w1 = free2grid[min(blk * 256 + 255, nfree - 1)] + halo + 1;
 #pragma unroll
-                for (int dy = -P; dy <= P; ++dy) {
-                    const int base = dz * sz + dy * sy;
-                    const int slot0 = ((dz + P) * W + (dy + P)) * W;
-#pragma unroll
-                    for (int dx = -P; dx <= P; ++dx)
-                        acc += (T)vb[(slot0 + dx + P) * kStencilTile] * xb[base + dx];
-                }
+        for (int u = 0; u < NPRE; ++u) {
+            const int i = w0 + (int)threadIdx.x + 256 * u;
+            prx[u] = i < w1 ? x[i] : (T)0;
+            prp[u] = i < w1 ? po[i] : (T)0;
+        }
+    }
+    T tb = 0;
+    if (MODE == 1) {
+        double rr = 0.0, rzn = 0.0;
+        for (int i = threadIdx.x; i < cs.np; i += 256) {
+            rr += cs.part_rr[i];
+            rzn += cs.part_rz[i];
+        }
+        bsum2<256>(rr, rzn, s);
+        const double err = sqrt(rr) / st->bnorm;
+        // restart > 0: the residual has just been formed and tested in FP64
+        const bool conv = !cs.restart && !cs.mixed && err < st->tol;
+        const bool due = !cs.restart && cs.mixed && (rr < st->rel_since_update * st->rr_ref || err < st->tol);
+        const double beta = cs.restart == 2 ? 0.0 : rzn / st->rzs[(cs.k + 1) & 1];
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            st->it = cs.k;
+            st->rr = rr;
+            st->err = err;
+            if (cs.hist && !cs.restart) cs.hist[cs.k] = err;
+            if (conv) st->done = 1;
+            if (due) {
+                // iterations from k on wait for the reliable update
+                st->need_update = 1;
+                st->flag_next = cs.k;
             }
-        } else {
+            if (!conv && !due) {
+                st->beta = beta;
+                st->rzs[cs.k & 1] = rzn;
+            }
+        }
+        // every block takes the same decision from the same partials, whether
+        // or not it has seen block 0's record of it
+        if (conv || due) return;
+        tb = (T)beta;
+    }
+    const bool first = MODE == 1 && cs.restart == 2;   // the old direction is not read
+    auto input = [&](int i) -> T {
+        if (MODE == 2) return x[i];
+        return first ? x[i] : x[i] + tb * po[i];
+    };
+    T *sA = reinterpret_cast<T *>(sp_smem), *sB = sA + wn;
+    double contrib = 0.0;
+    for (int r0 = blk * 256; r0 < nfree; r0 += gridDim.x * 256) {
+        const int r = r0 + threadIdx.x;
+        const bool act = r < nfree;
+        const int g = act ? free2grid[r] : 0;
+        const int ia = r % m0, ib = (r / m0) % m1, ic = (D == 3) ? r / (m0 * m1) : 0;
+        const V *vb = sval + stencil_index(UP, r, SL);   // from the centre slot up
+        const bool pre = NPRE > 1 && r0 == blk * 256;
+        int c = 0;
+        if (STAGED) {
+            w0 = free2grid[r0] - halo;
+            w1 = free2grid[min(r0 + 255, nfree - 1)] + halo + 1;
+            c = g - w0;
+        }
+        T acc = 0, own = 0;
+        auto plane = [&](int dz) {
+            if (STAGED) {
+                __syncthreads();   // the readers of the last planes are done
+                int i = w0 + threadIdx.x;
+                if (pre && dz == 0) {
 #pragma unroll
-            for (int dy = -P; dy <= P; ++dy) {
-                const int base = dy * sy;
-                const int slot0 = (dy + P) * W;
+                    for (int u = 0; u < NPRE; ++u, i += 256)
+                        if (i < w1) sA[i - w0] = first ? prx[u] : prx[u] + tb * prp[u];
+                }
+                for (; i < w1; i += 256) {
+                    sA[i - w0] = input(i + dz * sz);
+                    if (D == 3 && dz > 0) sB[i - w0] = input(i - dz * sz);
+                }
+                __syncthreads();
+            }
+        };
+        // entry at grid offset o of plane +dz / -dz
+        auto xa = [&](int dz, int o) -> T { return STAGED ? sA[c + o] : input(g + dz * sz + o); };
+        auto xm = [&](int dz, int o) -> T {
+            return STAGED ? (D == 3 && dz > 0 ? sB[c + o] : sA[c + o]) : input(g - dz * sz + o);
+        };
+        // upper line (dz, dy) and its mirror (-dz, -dy)
+        auto line = [&](int dz, int dy) {
+            const int h0 = (D == 3 ? ((dz + P) * W + (dy + P)) * W : (dy + P) * W) - C;   // (dz, dy, -P) from the centre
+#pragma unroll
+            for (int dx = -P; dx <= P; ++dx) acc += (T)vb[(h0 + dx + P) * kStencilTile] * xa(dz, dy * sy + dx);
+            if (KIND == 2) {
 #pragma unroll
                 for (int dx = -P; dx <= P; ++dx)
-                    acc += (T)vb[(slot0 + dx + P) * kStencilTile] * xb[base + dx];
+                    acc += (T)vb[-(h0 - dx + P) * kStencilTile] * xm(dz, dx - dy * sy);
+            } else {
+                const bool okyz = ib - dy >= 0 && ib - dy < m1 && ic - dz >= 0;
+                const int rm = r - m0 * (dy + m1 * dz);
+#pragma unroll
+                for (int dx = -P; dx <= P; ++dx) {
+                    const bool ok = okyz && ia + dx >= 0 && ia + dx < m0;
+                    acc += (T)(ok ? sval[stencil_index(UP + h0 - dx + P, rm + dx, SL)] : (V)0) * xm(dz, dx - dy * sy);
+                }
             }
-        }
-        if (MODE == 2) {
-            const T v = b[g] - acc;
-            y[g] = v;
-            contrib += (double)v * (double)v;
-        } else {
-            y[g] = acc;
-            if (MODE == 1) contrib += (double)x[g] * (double)acc;
-        }
-    }
-    if (MODE != 0) {
-        const double tot = bsum256(contrib, s);
-        if (threadIdx.x == 0) partial[blockIdx.x] = tot;
-    }
-}
-
-// The same SpMV on the half-stored FP32 operator (stencil_half layout): an
-// upper slot is read from the row itself, a lower slot from the neighbour row
-// at that offset (free box m0 x m1 x m2, rows lexicographic), whose mirrored
-// upper slot holds the same coefficient since the operator is bitwise
-// symmetric.  Neighbours outside the free box contribute 0 (x is 0 there).
-//
-// Order: each upper x-line of the stencil, (dz, dy) > 0 lexicographically
-// (the centre line from dx = 0), is taken together with its mirror line
-// (-dz, -dy).  Both read the same slot plane of the operator, the mirror one
-// at the rows shifted by the offset, so a block reads the plane at the same
-// point of its loop as the blocks that own those rows (up to 3 z-planes back,
-// on the same XCD through xcd_block) and the second read hits the L2.  With
-// the lexicographic order the z-lower mirrors were read at the start of the
-// loop and their owners read them at its end: each was fetched from HBM twice.
-template <int D, int P, typename T, int MODE>
-__global__ __launch_bounds__(256) void k_sspmv_half(int nfree, const int *__restrict__ free2grid,
-                                                    int sy, int sz, int m0, int m1, int m2,
-                                                    const float *__restrict__ sval,
-                                                    const T *__restrict__ x, T *__restrict__ y,
-                                                    const T *__restrict__ b,
-                                                    double *__restrict__ partial,
-                                                    CGState *__restrict__ st, int k)
-{
-    __shared__ double s[4];
-    if (st && (st->done || (st->flag_next && st->flag_next <= k))) return;
-    constexpr int W = 2 * P + 1;
-    constexpr int NS = (D == 3) ? W * W * W : W * W;
-    constexpr int C = NS / 2, NH = stencil_half(NS);
-    // full upper x-lines after the centre one: dz = 0, dy = 1..P, then (3D)
-    // dz = 1..P, dy = -P..P
-    constexpr int NL = (D == 3) ? P + P * W : P;
-    double contrib = 0.0;
-    const int blk = xcd_block(blockIdx.x, gridDim.x);
-    for (int r = blk * 256 + threadIdx.x; r < nfree; r += gridDim.x * 256) {
-        const int g = free2grid[r];
-        const int ia = r % m0, ib = (r / m0) % m1, ic = (D == 3) ? r / (m0 * m1) : 0;
-        const T *xb = x + g;
-        const float *vb = sval + stencil_index(0, r, NH);
-        T acc = 0;
-        // centre line: own slots dx = 0..P (half slots 0..P), mirrors dx = -P..-1
+        };
+        plane(0);
+        if (act) {
+            own = xa(0, 0);
+            // centre line: own slots dx = 0..P, mirrors dx = -P..-1
 #pragma unroll
-        for (int dx = 0; dx <= P; ++dx) acc += (T)vb[dx * kStencilTile] * xb[dx];
+            for (int dx = 0; dx <= P; ++dx) acc += (T)vb[dx * kStencilTile] * xa(0, dx);
 #pragma unroll
-        for (int dx = -P; dx < 0; ++dx)
-            acc += (T)(ia + dx >= 0 ? sval[stencil_index(-dx, r + dx, NH)] : 0.0f) * xb[dx];
+            for (int dx = -P; dx < 0; ++dx) {
+                if (KIND == 2) acc += (T)vb[dx * kStencilTile] * xa(0, dx);
+                else acc += (T)(ia + dx >= 0 ? sval[stencil_index(UP - dx, r + dx, SL)] : (V)0) * xa(0, dx);
+            }
 #pragma unroll 1
-        for (int u = 0; u < NL; ++u) {
-            const int dz = (D == 2 || u < P) ? 0 : 1 + (u - P) / W;
-            const int dy = (D == 2 || u < P) ? u + 1 : (u - P) % W - P;
-            const int h0 = (D == 3 ? ((dz + P) * W + (dy + P)) * W : (dy + P) * W) - C;   // (dz, dy, -P)
-            const int base = dz * sz + dy * sy;
-#pragma unroll
-            for (int dx = -P; dx <= P; ++dx) acc += (T)vb[(h0 + dx + P) * kStencilTile] * xb[base + dx];
-            const bool okyz = ib - dy >= 0 && ib - dy < m1 && ic - dz >= 0;
-            const int rm = r - m0 * (dy + m1 * dz);
-#pragma unroll
-            for (int dx = -P; dx <= P; ++dx) {
-                const bool ok = okyz && ia + dx >= 0 && ia + dx < m0;
-                acc += (T)(ok ? sval[stencil_index(h0 - dx + P, rm + dx, NH)] : 0.0f) * xb[dx - base];
+            for (int dy = 1; dy <= P; ++dy) line(0, dy);
+        }
+        if (D == 3) {
+#pragma unroll 1
+            for (int dz = 1; dz <= P; ++dz) {
+                plane(dz);
+                if (act) {
+#pragma unroll 1
+                    for (int dy = -P; dy <= P; ++dy) line(dz, dy);
+                }
             }
         }
-        if (MODE == 2) {
-            const T v = b[g] - acc;
-            y[g] = v;
-            contrib += (double)v * (double)v;
-        } else {
-            y[g] = acc;
-            if (MODE == 1) contrib += (double)x[g] * (double)acc;
+        if (act) {
+            if (MODE == 2) {
+                const T v = b[g] - acc;
+                y[g] = v;
+                contrib += (double)v * (double)v;
+            } else {
+                pn[g] = own;
+                y[g] = acc;
+                contrib += (double)own * (double)acc;
+            }
         }
     }
-    if (MODE != 0) {
-        const double tot = bsum256(contrib, s);
-        if (threadIdx.x == 0) partial[blockIdx.x] = tot;
-    }
+    const double tot = bsum<256>(contrib, s);
+    if (threadIdx.x == 0) partial[blockIdx.x] = tot;
 }
 
 // ---------------------------------------------------------------------------
@@ -244,17 +337,31 @@ __global__ __launch_bounds__(256) void k_sspmv_half(int nfree, const int *__rest
 // Every block derives alpha = rz_k / (p, A p) from the SpMV's partials
 // itself (a bounded count, summed in a fixed order).
 template <typename T, typename TX>
-__global__ __launch_bounds__(256) void k_cg2_update(int n, TX *__restrict__ x, T *__restrict__ r,
-                                                    const T *__restrict__ p, const T *__restrict__ t,
-                                                    T *__restrict__ z, const T *__restrict__ diag,
-                                                    double tau, const double *__restrict__ pap_parts,
-                                                    int npap, double *__restrict__ part_rr,
-                                                    double *__restrict__ part_rz,
-                                                    CGState *__restrict__ st, int k)
+__global__ __launch_bounds__(kVecThreads) void k_cg2_update(int n, TX *__restrict__ x, T *__restrict__ r,
+                                                            const T *__restrict__ p, const T *__restrict__ t,
+                                                            T *__restrict__ z, const T *__restrict__ diag,
+                                                            double tau, const double *__restrict__ pap_parts,
+                                                            int npap, double *__restrict__ part_rr,
+                                                            double *__restrict__ part_rz,
+                                                            CGState *__restrict__ st, int k)
 {
-    __shared__ double s[4];
+    __shared__ double s[2 * kVecThreads / 64];
     if (st->done || (st->flag_next && st->flag_next <= k)) return;
-    const double pap = sum_partials(pap_parts, npap, s);
+    // the first entries are requested before the sum that gives alpha
+    int i = blockIdx.x * kVecThreads + threadIdx.x;
+    T pi = 0, ti = 0, ri = 0, di = 1;
+    TX xi = 0;
+    auto load = [&]() {
+        if (i < n) {
+            pi = p[i];
+            ti = t[i];
+            ri = r[i];
+            xi = x[i];
+            if (diag) di = diag[i];
+        }
+    };
+    load();
+    const double pap = sum_partials<kVecThreads>(pap_parts, npap, s);
     const double alpha_d = st->rzs[k & 1] / pap;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         st->pap = pap;
@@ -263,102 +370,87 @@ __global__ __launch_bounds__(256) void k_cg2_update(int n, TX *__restrict__ x, T
     const T alpha = (T)alpha_d;
     const T ta = (T)tau;
     double rr = 0.0, rz = 0.0;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        x[i] += (TX)(alpha * p[i]);
-        const T ri = r[i] - alpha * t[i];
-        r[i] = ri;
-        const T zi = diag ? ta * ri / diag[i] : ri;
+    while (i < n) {
+        x[i] = xi + (TX)(alpha * pi);
+        const T rn = ri - alpha * ti;
+        r[i] = rn;
+        const T zi = diag ? ta * rn / di : rn;
+        z[i] = zi;
+        rr += (double)rn * (double)rn;
+        rz += (double)rn * (double)zi;
+        i += gridDim.x * kVecThreads;
+        load();
+    }
+    bsum2<kVecThreads>(rr, rz, s);
+    if (threadIdx.x == 0) {
+        part_rr[blockIdx.x] = rr;
+        part_rz[blockIdx.x] = rz;
+    }
+}
+
+// The stop test of k_cg2_spmv on its own, after the last iteration of a chunk
+// of launches: k iterations are complete.  MIXED == 0: reference stopping rule
+// (err < tol stops).  MIXED == 1: FP32 recurrence of the mixed solver: never
+// stops on its own residual, flags a reliable update instead and pauses until
+// it has run.
+__global__ __launch_bounds__(256) void k_cg2_check(CGStep cs, CGState *__restrict__ st)
+{
+    __shared__ double s[4];
+    if (st->done || (st->flag_next && st->flag_next <= cs.k)) return;
+    const double rr = sum_partials<256>(cs.part_rr, cs.np, s);
+    if (threadIdx.x != 0) return;
+    const double err = sqrt(rr) / st->bnorm;
+    st->it = cs.k;
+    st->rr = rr;
+    st->err = err;
+    if (cs.hist) cs.hist[cs.k] = err;
+    if (!cs.mixed && err < st->tol) {
+        st->done = 1;
+    } else {
+        if (cs.mixed && (rr < st->rel_since_update * st->rr_ref || err < st->tol)) {
+            st->need_update = 1;
+            st->flag_next = cs.k;
+        }
+        if (cs.k >= st->maxit) st->done = 2;
+    }
+}
+
+// z = tau r / diag (or z = r), partials (r, r) and (r, z)
+template <typename T>
+__global__ __launch_bounds__(kVecThreads) void k_cg2_precond(int n, const T *__restrict__ r, T *__restrict__ z,
+                                                             const T *__restrict__ diag, double tau,
+                                                             double *__restrict__ part_rr,
+                                                             double *__restrict__ part_rz)
+{
+    __shared__ double s[2 * kVecThreads / 64];
+    double rr = 0.0, rz = 0.0;
+    for (int i = blockIdx.x * kVecThreads + threadIdx.x; i < n; i += gridDim.x * kVecThreads) {
+        const T ri = r[i];
+        const T zi = diag ? (T)tau * ri / diag[i] : ri;
         z[i] = zi;
         rr += (double)ri * (double)ri;
         rz += (double)ri * (double)zi;
     }
-    const double a = bsum256(rr, s);
-    const double c = bsum256(rz, s);
+    bsum2<kVecThreads>(rr, rz, s);
     if (threadIdx.x == 0) {
-        part_rr[blockIdx.x] = a;
-        part_rz[blockIdx.x] = c;
+        part_rr[blockIdx.x] = rr;
+        part_rz[blockIdx.x] = rz;
     }
-}
-
-// Stop test and p = z + beta p.  MIXED == 0: reference stopping rule (err <
-// tol stops, before the direction update).  MIXED == 1: FP32 recurrence of
-// the mixed solver: never stops on its own residual, flags a reliable
-// update instead and pauses from iteration k + 1 on until it has run.
-template <typename T, int MIXED>
-__global__ __launch_bounds__(256) void k_cg2_direction(int n, T *__restrict__ p, const T *__restrict__ z,
-                                                       const double *__restrict__ part_rr,
-                                                       const double *__restrict__ part_rz, int np,
-                                                       CGState *__restrict__ st, int k,
-                                                       double *__restrict__ hist)
-{
-    __shared__ double s[4];
-    // flag_next is only ever set to k + 1 below, so the blocks of this
-    // launch read the same decision whether or not block 0 has written it
-    if (st->done || (st->flag_next && st->flag_next <= k)) return;
-    const double rr = sum_partials(part_rr, np, s);
-    const double rzn = sum_partials(part_rz, np, s);
-    const double err = sqrt(rr) / st->bnorm;
-    const bool conv = !MIXED && err < st->tol;
-    const double beta = rzn / st->rzs[k & 1];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        st->it = k + 1;
-        st->rr = rr;
-        st->err = err;
-        if (hist) hist[k + 1] = err;
-        if (conv) {
-            st->done = 1;
-        } else {
-            st->beta = beta;
-            st->rzs[(k + 1) & 1] = rzn;
-            if (MIXED && (rr < st->rel_since_update * st->rr_ref || err < st->tol)) {
-                st->need_update = 1;
-                st->flag_next = k + 1;
-            }
-            if (k + 1 >= st->maxit) st->done = 2;
-        }
-    }
-    if (conv) return;
-    const T tb = (T)beta;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) p[i] = z[i] + tb * p[i];
-}
-
-// z = tau r / diag (or z = r), partial (r, z)
-template <typename T>
-__global__ __launch_bounds__(256) void k_cg2_precond(int n, const T *__restrict__ r, T *__restrict__ z,
-                                                     const T *__restrict__ diag, double tau,
-                                                     double *__restrict__ part_rz)
-{
-    __shared__ double s[4];
-    double rz = 0.0;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        const T zi = diag ? (T)tau * r[i] / diag[i] : r[i];
-        z[i] = zi;
-        rz += (double)r[i] * (double)zi;
-    }
-    const double c = bsum256(rz, s);
-    if (threadIdx.x == 0) part_rz[blockIdx.x] = c;
 }
 
 // partial (a, b) in the grid solvers' block layout (a preconditioner that
 // is not fused into the update writes z, then this gives the (r, z) partials)
 template <typename T>
-__global__ __launch_bounds__(256) void k_cg2_dot(int n, const T *__restrict__ a, const T *__restrict__ b,
-                                                 double *__restrict__ part, const CGState *__restrict__ st)
+__global__ __launch_bounds__(kVecThreads) void k_cg2_dot(int n, const T *__restrict__ a, const T *__restrict__ b,
+                                                         double *__restrict__ part, const CGState *__restrict__ st)
 {
-    __shared__ double s[4];
+    __shared__ double s[kVecThreads / 64];
     if (st && st->done) return;
     double v = 0.0;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) v += (double)a[i] * (double)b[i];
-    const double c = bsum256(v, s);
+    for (int i = blockIdx.x * kVecThreads + threadIdx.x; i < n; i += gridDim.x * kVecThreads)
+        v += (double)a[i] * (double)b[i];
+    const double c = bsum<kVecThreads>(v, s);
     if (threadIdx.x == 0) part[blockIdx.x] = c;
-}
-
-__global__ __launch_bounds__(256) void k_set_rz(const double *__restrict__ parts, int np, CGState *__restrict__ st,
-                                                int slot)
-{
-    __shared__ double s[4];
-    const double a = sum_partials(parts, np, s);
-    if (threadIdx.x == 0) st->rzs[slot & 1] = a;
 }
 
 template <typename S, typename Dt>
@@ -381,16 +473,16 @@ __global__ void k_accum_grid(int64_t n, double *__restrict__ x, float *__restric
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-static inline unsigned blocks_for(int64_t n, int cap)
+static inline unsigned blocks_for(int64_t n, int nt, int cap)
 {
-    int64_t b = (n + 255) / 256;
+    int64_t b = (n + nt - 1) / nt;
     if (b > cap) b = cap;
     if (b < 1) b = 1;
     return (unsigned)b;
 }
 
-int sspmv_blocks(int nfree) { return (int)blocks_for(nfree, kMaxPartials); }
-int vec_blocks(int64_t n) { return (int)blocks_for(n, 1024); }
+int sspmv_blocks(int nfree) { return (int)blocks_for(nfree, 256, kMaxPartials); }
+int vec_blocks(int64_t n) { return (int)blocks_for(n, kVecThreads, 512); }
 
 template <typename T>
 hipError_t launch_fill_t(T *a, int64_t n, T v, hipStream_t s)
@@ -436,48 +528,94 @@ hipError_t launch_gather_f64_from_grid(int nfree, const int *f2g, const double *
     return hipGetLastError();
 }
 
-template <typename V, typename T>
-static hipError_t sspmv_dispatch(int d, int p, int mode, int nfree, const int *f2g, int sy, int sz,
-                                 const V *sv, const T *x, T *y, const T *b, double *part,
-                                 CGState *st, int k, hipStream_t s)
+int sspmv_window(int p, int nfree, int m0, int m1, int sy, int sz)
 {
-    const dim3 grid(sspmv_blocks(nfree)), blk(256);
-#define GSX_S(D, P, M) if (d == D && p == P && mode == M) { hipLaunchKernelGGL((k_sspmv<D, P, V, T, M>), grid, blk, 0, s, nfree, f2g, sy, sz, sv, x, y, b, part, st, k); return hipGetLastError(); }
-#define GSX_S3(D, P) GSX_S(D, P, 0) GSX_S(D, P, 1) GSX_S(D, P, 2)
-    GSX_S3(2, 1) GSX_S3(2, 2) GSX_S3(2, 3) GSX_S3(2, 4)
-    GSX_S3(3, 1) GSX_S3(3, 2) GSX_S3(3, 3) GSX_S3(3, 4)
-#undef GSX_S3
-#undef GSX_S
+    auto grid = [&](int r) { return (int64_t)(r % m0) + (int64_t)sy * ((r / m0) % m1) + (int64_t)sz * (r / (m0 * m1)); };
+    int64_t w = 0;
+    for (int r0 = 0; r0 < nfree; r0 += 256) w = std::max(w, grid(std::min(r0 + 255, nfree - 1)) - grid(r0));
+    w += 1 + 2 * (int64_t)(p * sy + p);
+    return (int)std::min<int64_t>(w, INT32_MAX);
+}
+
+// An FP64 operator of at most this many bytes (all slots) is read whole: it
+// stays in the eight 4 MB L2s, where the mirrored reads' index operations cost
+// more than the bytes they save.  Whole solves, all slots against mirrored:
+// 64^2 p = 2 (0.8 MB) 1788 / 1967 us, 18^3 p = 3 (20 MB) 3662 / 4392 us;
+// 75^3 p = 2 (422 MB) 12.5 / 7.4 ms.
+constexpr int64_t kMirrorBytes = (int64_t)24 << 20;
+constexpr size_t kWindowLds = 64 * 1024;
+
+template <int D, int P, typename V, typename T, int KIND, int MODE>
+static hipError_t sspmv_launch(const SpmvGrid &G, const V *sv, const T *x, const T *po, T *pn, T *y, const T *b,
+                               double *part, const CGStep &cs, CGState *st, hipStream_t s)
+{
+    const dim3 grid(sspmv_blocks(G.nfree)), blk(256);
+    const size_t lds = (size_t)G.window * (D == 3 ? 2 : 1) * sizeof(T);
+    if (lds <= kWindowLds)
+        hipLaunchKernelGGL((k_cg2_spmv<D, P, V, T, KIND, MODE, true>), grid, blk, lds, s, G.nfree, G.f2g, G.sy, G.sz,
+                           G.m0, G.m1, sv, x, po, pn, y, b, part, cs, st, G.window);
+    else
+        hipLaunchKernelGGL((k_cg2_spmv<D, P, V, T, KIND, MODE, false>), grid, blk, 0, s, G.nfree, G.f2g, G.sy, G.sz,
+                           G.m0, G.m1, sv, x, po, pn, y, b, part, cs, st, 0);
+    return hipGetLastError();
+}
+
+#define GSX_SALL(KIND, MODE)                                                                                      \
+    GSX_S(2, 1, KIND, MODE) GSX_S(2, 2, KIND, MODE) GSX_S(2, 3, KIND, MODE) GSX_S(2, 4, KIND, MODE)               \
+    GSX_S(3, 1, KIND, MODE) GSX_S(3, 2, KIND, MODE) GSX_S(3, 3, KIND, MODE) GSX_S(3, 4, KIND, MODE)
+#define GSX_S(D, P, KIND, MODE)                                                                                   \
+    if (G.d == D && G.p == P) return sspmv_launch<D, P, SV, ST, KIND, MODE>(G, sv, x, po, pn, y, b, part, cs, st, s);
+
+template <int MODE>
+static hipError_t sspmv_f64(const SpmvGrid &G, const double *sv, const double *x, const double *po, double *pn,
+                            double *y, const double *b, double *part, const CGStep &cs, CGState *st, hipStream_t s)
+{
+    using SV = double;
+    using ST = double;
+    const int w = 2 * G.p + 1, slots = G.d == 3 ? w * w * w : w * w;
+    if ((int64_t)G.nfree * slots * 8 <= kMirrorBytes) {
+        GSX_SALL(2, MODE)
+    } else {
+        GSX_SALL(1, MODE)
+    }
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_sspmv_f64(int d, int p, int mode, int nfree, const int *f2g, int sy, int sz,
-                            const double *sv, const double *x, double *y, const double *b,
-                            double *part, CGState *st, int k, hipStream_t s)
+hipError_t launch_sspmv_residual(const SpmvGrid &G, const double *sv, const double *x, double *y, const double *b,
+                                 double *part, hipStream_t s)
 {
-    return sspmv_dispatch<double, double>(d, p, mode, nfree, f2g, sy, sz, sv, x, y, b, part, st, k, s);
+    return sspmv_f64<2>(G, sv, x, nullptr, nullptr, y, b, part, CGStep{}, nullptr, s);
 }
 
-hipError_t launch_sspmv_f32(int d, int p, int mode, int nfree, const int *f2g, int sy, int sz, int m0, int m1,
-                            int m2, const float *sv, const float *x, float *y, const float *b,
-                            double *part, CGState *st, int k, hipStream_t s)
+hipError_t launch_cg2_spmv_f64(const SpmvGrid &G, const double *sv, const double *z, const double *po, double *pn,
+                               double *t, double *part, const CGStep &cs, CGState *st, hipStream_t s)
 {
-    if ((int64_t)m0 * m1 * m2 != nfree) return hipErrorInvalidValue;
-    const dim3 grid(sspmv_blocks(nfree)), blk(256);
-#define GSX_S(D, P, M) if (d == D && p == P && mode == M) { hipLaunchKernelGGL((k_sspmv_half<D, P, float, M>), grid, blk, 0, s, nfree, f2g, sy, sz, m0, m1, m2, sv, x, y, b, part, st, k); return hipGetLastError(); }
-#define GSX_S3(D, P) GSX_S(D, P, 0) GSX_S(D, P, 1) GSX_S(D, P, 2)
-    GSX_S3(2, 1) GSX_S3(2, 2) GSX_S3(2, 3) GSX_S3(2, 4)
-    GSX_S3(3, 1) GSX_S3(3, 2) GSX_S3(3, 3) GSX_S3(3, 4)
-#undef GSX_S3
-#undef GSX_S
+    return sspmv_f64<1>(G, sv, z, po, pn, t, nullptr, part, cs, st, s);
+}
+
+hipError_t launch_cg2_spmv_f32(const SpmvGrid &G, const float *sv, const float *x, const float *po, float *pn,
+                               float *y, double *part, const CGStep &cs, CGState *st, hipStream_t s)
+{
+    using SV = float;
+    using ST = float;
+    const float *b = nullptr;
+    GSX_SALL(0, 1)
     return hipErrorInvalidValue;
+}
+#undef GSX_S
+#undef GSX_SALL
+
+hipError_t launch_cg2_check(const CGStep &cs, CGState *st, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_cg2_check, dim3(1), dim3(256), 0, s, cs, st);
+    return hipGetLastError();
 }
 
 hipError_t launch_cg2_update_f64(int n, double *x, double *r, const double *p, const double *t,
                                  double *z, const double *diag, double tau, const double *pap,
                                  int npap, double *prr, double *prz, CGState *st, int k, hipStream_t s)
 {
-    hipLaunchKernelGGL((k_cg2_update<double, double>), dim3(vec_blocks(n)), dim3(256), 0, s, n, x, r, p, t, z,
+    hipLaunchKernelGGL((k_cg2_update<double, double>), dim3(vec_blocks(n)), dim3(kVecThreads), 0, s, n, x, r, p, t, z,
                        diag, tau, pap, npap, prr, prz, st, k);
     return hipGetLastError();
 }
@@ -486,60 +624,38 @@ hipError_t launch_cg2_update_f32(int n, float *x, float *r, const float *p, cons
                                  const float *diag, double tau, const double *pap, int npap,
                                  double *prr, double *prz, CGState *st, int k, hipStream_t s)
 {
-    hipLaunchKernelGGL((k_cg2_update<float, float>), dim3(vec_blocks(n)), dim3(256), 0, s, n, x, r, p, t, z,
+    hipLaunchKernelGGL((k_cg2_update<float, float>), dim3(vec_blocks(n)), dim3(kVecThreads), 0, s, n, x, r, p, t, z,
                        diag, tau, pap, npap, prr, prz, st, k);
-    return hipGetLastError();
-}
-
-hipError_t launch_cg2_direction_f64(int n, double *p, const double *z, const double *prr,
-                                    const double *prz, int np, CGState *st, int k, double *hist,
-                                    hipStream_t s)
-{
-    hipLaunchKernelGGL((k_cg2_direction<double, 0>), dim3(vec_blocks(n)), dim3(256), 0, s, n, p, z, prr, prz,
-                       np, st, k, hist);
-    return hipGetLastError();
-}
-
-hipError_t launch_cg2_direction_f32_mixed(int n, float *p, const float *z, const double *prr,
-                                          const double *prz, int np, CGState *st, int k,
-                                          hipStream_t s)
-{
-    hipLaunchKernelGGL((k_cg2_direction<float, 1>), dim3(vec_blocks(n)), dim3(256), 0, s, n, p, z, prr, prz,
-                       np, st, k, nullptr);
     return hipGetLastError();
 }
 
 hipError_t launch_cg2_dot_f64(int n, const double *a, const double *b, double *part, const CGState *st,
                               hipStream_t s)
 {
-    hipLaunchKernelGGL((k_cg2_dot<double>), dim3(vec_blocks(n)), dim3(256), 0, s, n, a, b, part, st);
+    hipLaunchKernelGGL((k_cg2_dot<double>), dim3(vec_blocks(n)), dim3(kVecThreads), 0, s, n, a, b, part, st);
     return hipGetLastError();
 }
 
 hipError_t launch_cg2_dot_f32(int n, const float *a, const float *b, double *part, const CGState *st,
                               hipStream_t s)
 {
-    hipLaunchKernelGGL((k_cg2_dot<float>), dim3(vec_blocks(n)), dim3(256), 0, s, n, a, b, part, st);
+    hipLaunchKernelGGL((k_cg2_dot<float>), dim3(vec_blocks(n)), dim3(kVecThreads), 0, s, n, a, b, part, st);
     return hipGetLastError();
 }
 
-hipError_t launch_cg2_precond_f64(int n, const double *r, double *z, const double *diag, double tau,
+hipError_t launch_cg2_precond_f64(int n, const double *r, double *z, const double *diag, double tau, double *prr,
                                   double *prz, hipStream_t s)
 {
-    hipLaunchKernelGGL((k_cg2_precond<double>), dim3(vec_blocks(n)), dim3(256), 0, s, n, r, z, diag, tau, prz);
+    hipLaunchKernelGGL((k_cg2_precond<double>), dim3(vec_blocks(n)), dim3(kVecThreads), 0, s, n, r, z, diag, tau, prr,
+                       prz);
     return hipGetLastError();
 }
 
-hipError_t launch_cg2_precond_f32(int n, const float *r, float *z, const float *diag, double tau,
+hipError_t launch_cg2_precond_f32(int n, const float *r, float *z, const float *diag, double tau, double *prr,
                                   double *prz, hipStream_t s)
 {
-    hipLaunchKernelGGL((k_cg2_precond<float>), dim3(vec_blocks(n)), dim3(256), 0, s, n, r, z, diag, tau, prz);
-    return hipGetLastError();
-}
-
-hipError_t launch_set_rz(const double *parts, int np, CGState *st, int slot, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_set_rz, dim3(1), dim3(256), 0, s, parts, np, st, slot);
+    hipLaunchKernelGGL((k_cg2_precond<float>), dim3(vec_blocks(n)), dim3(kVecThreads), 0, s, n, r, z, diag, tau, prr,
+                       prz);
     return hipGetLastError();
 }
 

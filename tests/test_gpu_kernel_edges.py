@@ -80,3 +80,45 @@ def test_fd_pcg_fp32_tiles(ctx, d, p, n):
     assert its[1] <= its[0] + 5, its   # wrong FP32 factors would not precondition
     for o in (A, b, fd, gp):
         o.close()
+
+
+# the structured CG: row tiles of 256 with staged windows, all slots read below
+# 24 MB of operator and mirrored upper ones above, direct reads where a window
+# exceeds the LDS (the flat boxes), several tiles a block above 524,288 rows
+@pytest.mark.parametrize("d,p,n", [(2, 1, (2, 2)), (2, 2, (16, 17)), (2, 4, (300, 9)), (2, 1, (740, 731)),
+                                   (3, 1, (9, 8, 7)), (3, 2, (3, 3, 600)), (3, 3, (2, 2, 450)), (3, 3, (19, 18, 19)),
+                                   (3, 3, (21, 19, 20)), (3, 4, (13, 11, 12)), (3, 4, (2, 40, 3))])
+def test_structured_cg_tiles(ctx, d, p, n):
+    """FP64 and mixed solves on the structured operator reach the CSR
+    operator's solution in its iterations."""
+    P = problems.box_patch(d, p, n)
+    P.kappa = problems.lognormal_kappa(P.nelem, 0.3, 5)
+    P.fkind = 1
+    prob = problems.Problem([P], problems.all_sides(d), [])
+    gp = gsx.Problem(ctx, prob)
+    A, b = gp.assemble(gsx.PATTERN_EXPR, gsx.MIXED)
+    # Ten FP64 iterations: the recurrences perturb each step by a few eps and
+    # a perturbation grows at most with the Krylov polynomials, of norm up to
+    # about sqrt(cond) <= 1e5 here before orthogonality is lost, so the two
+    # operators' iterates agree to 10 * 1e-16 * 1e5 = 1e-10.  (After 120 the
+    # flat boxes' iterates differ by 1e-5: orthogonality is gone there.)
+    few = []
+    for structured in (False, True):
+        A.set_operator(structured)
+        x = ctx.array(gp.nfree).zero()
+        it, rel, ok = A.cg_solve(b, x, tol=1e-30, maxit=10)
+        few.append((x.download(), it, A.history()))
+        x.close()
+    assert few[0][1] == few[1][1]
+    assert np.linalg.norm(few[1][0] - few[0][0]) <= 1e-10 * np.linalg.norm(few[0][0])
+    assert np.allclose(few[1][2], few[0][2], rtol=1e-9, atol=1e-13)
+    # solves to 1e-9, the mixed one through FP32 iterations
+    r = b.download()
+    M = A.to_scipy()
+    for prec in (gsx.FP64, gsx.MIXED):
+        x = ctx.array(gp.nfree).zero()
+        it, rel, ok = A.cg_solve(b, x, tol=1e-9, maxit=20000, precision=prec)
+        assert ok and np.linalg.norm(r - M @ x.download()) <= 1.01e-9 * np.linalg.norm(r), (prec, it, rel)
+        x.close()
+    for o in (A, b, gp):
+        o.close()
