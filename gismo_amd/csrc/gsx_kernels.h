@@ -106,6 +106,8 @@ hipError_t launch_jacobi_apply_f64(int n, const double *r, double *z, const doub
                                    double tau, double *prz, const CGState *st, hipStream_t s);
 hipError_t launch_jacobi_apply_f32(int n, const float *r, float *z, const float *diag,
                                    double tau, double *prz, const CGState *st, hipStream_t s);
+hipError_t launch_cg_restart(int n, const double *r64, float *r, float *z, float *p, const float *diag, double tau,
+                             int keep, double *prz, hipStream_t s);
 hipError_t launch_jacobi_step_f64(int lpr, int n, const int *rp, const int *ci, const double *v,
                                   const double *diag, const double *b, const double *xin,
                                   double *xout, double tau, int x_is_zero, hipStream_t s);

@@ -807,23 +807,6 @@ __global__ void k_prolong_add(int n, const int *__restrict__ rp, const int *__re
     y[r] = (T)((double)y[r] + (double)alpha * s);
 }
 
-// r = b - A x (CSR), one wavefront-group per row
-template <int LPR, typename V, typename T>
-__global__ __launch_bounds__(256) void k_residual(int n, const int *__restrict__ rp, const int *__restrict__ ci,
-                                                  const V *__restrict__ v, const T *__restrict__ x,
-                                                  const T *__restrict__ b, T *__restrict__ r)
-{
-    constexpr int RPB = 256 / LPR;
-    const int g = threadIdx.x / LPR, lane = threadIdx.x % LPR;
-    const int row = blockIdx.x * RPB + g;
-    double acc = 0.0;   // FP64 sums whatever the storage type (see k_jacobi_step)
-    if (row < n)
-        for (int k = rp[row] + lane; k < rp[row + 1]; k += LPR) acc += (double)v[k] * (double)x[ci[k]];
-#pragma unroll
-    for (int off = LPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, LPR);
-    if (row < n && lane == 0) r[row] = (T)((double)b[row] - acc);
-}
-
 // y = R x (restriction), kRestrictLanes lanes per coarse row (consecutive
 // lanes read consecutive entries of the row); lane partials summed in FP64
 // by butterfly shuffles (a fixed order), stored in the coarse vector's type TY
@@ -1039,38 +1022,6 @@ hipError_t launch_restrict_v32(int n, const int *rp, const int *ci, const float 
 {
     hipLaunchKernelGGL((k_restrict<float, double, float>), g1((int64_t)n * kRestrictLanes), dim3(256), 0, s, n, rp, ci, v, x, y);
     return hipGetLastError();
-}
-
-template <typename V, typename T>
-static hipError_t residual_dispatch(int lpr, int n, const int *rp, const int *ci, const V *v, const T *x,
-                                    const T *b, T *r, hipStream_t s)
-{
-    const dim3 grid((n + 256 / lpr - 1) / (256 / lpr)), blk(256);
-    switch (lpr) {
-    case 64: hipLaunchKernelGGL((k_residual<64, V, T>), grid, blk, 0, s, n, rp, ci, v, x, b, r); break;
-    case 32: hipLaunchKernelGGL((k_residual<32, V, T>), grid, blk, 0, s, n, rp, ci, v, x, b, r); break;
-    case 16: hipLaunchKernelGGL((k_residual<16, V, T>), grid, blk, 0, s, n, rp, ci, v, x, b, r); break;
-    default: hipLaunchKernelGGL((k_residual<8, V, T>), grid, blk, 0, s, n, rp, ci, v, x, b, r); break;
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_residual_f64(int lpr, int n, const int *rp, const int *ci, const double *v, const double *x,
-                               const double *b, double *r, hipStream_t s)
-{
-    return residual_dispatch<double, double>(lpr, n, rp, ci, v, x, b, r, s);
-}
-
-hipError_t launch_residual_v32(int lpr, int n, const int *rp, const int *ci, const float *v, const double *x,
-                               const double *b, double *r, hipStream_t s)
-{
-    return residual_dispatch<float, double>(lpr, n, rp, ci, v, x, b, r, s);
-}
-
-hipError_t launch_residual_f32(int lpr, int n, const int *rp, const int *ci, const float *v, const float *x,
-                               const float *b, float *r, hipStream_t s)
-{
-    return residual_dispatch<float, float>(lpr, n, rp, ci, v, x, b, r, s);
 }
 
 hipError_t launch_conv_f64_f32(int64_t n, const double *a, float *b, hipStream_t s)

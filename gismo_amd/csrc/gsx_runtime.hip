@@ -1658,23 +1658,15 @@ static gsx_status cg_mixed(gsx_matrix *A, int precond, double tau, const double 
     GSX_TRY(read_state(c, w, h));
     if (h.done == 3) HIP_OK(c, hipMemsetAsync(x, 0, sizeof(double) * n, s));
 
-    // r32 = fp32(r64); z32 = M r32; rz = (r32, z32); the direction p32 is kept
-    auto restart_from_r64 = [&]() -> gsx_status {
-        HIP_OK(c, gsx::launch_f64_to_f32(n, r, r32, s));
-        if (jac) {
-            HIP_OK(c, gsx::launch_jacobi_apply_f32(n, r32, z32, d32, tau, P0, nullptr, s));
-        } else {
-            HIP_OK(c, hipMemcpyAsync(z32, r32, sizeof(float) * n, hipMemcpyDeviceToDevice, s));
-            HIP_OK(c, gsx::launch_dot_f32(n, r32, r32, P0, nullptr, s));
-        }
+    // r32 = fp32(r64); z32 = M r32; rz = (r32, z32)
+    auto restart_from_r64 = [&](bool keep) -> gsx_status {
+        HIP_OK(c, gsx::launch_cg_restart(n, r, r32, z32, p32, jac ? d32 : nullptr, tau, keep ? 1 : 0, P0, s));
         HIP_OK(c, gsx::launch_cg_scalar(1, P0, nv, nullptr, 0, st, nullptr, s));
         return GSX_OK;
     };
     if (!h.done) {
         HIP_OK(c, hipMemsetAsync(xc, 0, sizeof(float) * n, s));
-        gsx_status e = restart_from_r64();
-        if (e != GSX_OK) return e;
-        HIP_OK(c, hipMemcpyAsync(p32, z32, sizeof(float) * n, hipMemcpyDeviceToDevice, s));
+        GSX_TRY(restart_from_r64(false));
         int chunk = 8;
         while (true) {
             for (int k = 0; k < chunk; ++k) {
@@ -1699,12 +1691,9 @@ static gsx_status cg_mixed(gsx_matrix *A, int precond, double tau, const double 
                 HIP_OK(c, gsx::launch_cg_reliable(P1, ns, st, nullptr, s));
                 GSX_TRY(read_state(c, w, h));
                 if (h.done == 1 || h.done == 2) break;
-                gsx_status e2 = restart_from_r64();
-                if (e2 != GSX_OK) return e2;
                 // a recurrence that has parted from the true residual (it
                 // ran into its FP32 floor) leaves no usable direction
-                if (rr_rec < gsx::kDirectionReset * h.rr)
-                    HIP_OK(c, hipMemcpyAsync(p32, jac ? z32 : r32, sizeof(float) * n, hipMemcpyDeviceToDevice, s));
+                GSX_TRY(restart_from_r64(rr_rec >= gsx::kDirectionReset * h.rr));
             }
             if (h.it >= maxit) break;
         }
@@ -2226,7 +2215,8 @@ gsx_status gsx_cg_solve_noalloc(gsx_matrix *A, int32_t precond, double tau, cons
         if (relres) *relres = 0.0;
         return GSX_OK;
     }
-    const int nparts = std::max(gsx::spmv_blocks(n, A->lpr), (n + 255) / 256) + 1;
+    const int rpb = 256 / A->lpr;   // the fixed array's documented share of partial sums: one per rpb rows
+    const int nparts = std::max((n + rpb - 1) / rpb, (n + 255) / 256) + 1;
     size_t off = 0;
     auto take = [&](size_t bytes) {
         const size_t o = off;

@@ -12,16 +12,9 @@
 // them in a fixed order), so results are bitwise reproducible run to run.
 #include "gsx_common.h"
 #include "gsx_kernels.h"
+#include "gsx_csr.h"
 
 namespace gsx {
-
-template <int LPR, typename T>
-__device__ inline T group_sum(T v)
-{
-#pragma unroll
-    for (int off = LPR / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, LPR);
-    return v;
-}
 
 __device__ inline double block_sum256(double v, double *s)
 {
@@ -36,13 +29,13 @@ __device__ inline double block_sum256(double v, double *s)
 }
 
 // ---------------------------------------------------------------------------
-// SpMV, LPR lanes per row, 256 threads per block.
+// CSR SpMV (csr_rows), L lanes summing a row, 256 threads per block.
 //   MODE 0: y = A x
 //   MODE 1: y = A x and partial[block] = sum_rows x_i y_i
 //   MODE 2: y = b - A x and partial[block] = sum_rows y_i^2
 // Skipped entirely when state->done != 0 (state may be null).
 // ---------------------------------------------------------------------------
-template <int LPR, typename V, typename T, int MODE>
+template <int L, typename V, typename T, int MODE>
 __global__ __launch_bounds__(256) void k_spmv(int n, const int *__restrict__ rowptr,
                                               const int *__restrict__ col,
                                               const V *__restrict__ val, const T *__restrict__ x,
@@ -50,28 +43,23 @@ __global__ __launch_bounds__(256) void k_spmv(int n, const int *__restrict__ row
                                               double *__restrict__ partial,
                                               const CGState *__restrict__ state)
 {
-    __shared__ double s[256];
+    __shared__ T buf[4][kCsrCap];
+    __shared__ double s[4];
     if (state && (state->done || state->frozen)) return;
-    constexpr int RPB = 256 / LPR;
-    const int g = threadIdx.x / LPR, lane = threadIdx.x % LPR;
-    const int r = blockIdx.x * RPB + g;
-    T acc = 0;
-    if (r < n) {
-        const int k0 = rowptr[r], k1 = rowptr[r + 1];
-        for (int k = k0 + lane; k < k1; k += LPR) acc += (T)val[k] * x[col[k]];
-    }
-    acc = group_sum<LPR, T>(acc);
     double contrib = 0.0;
-    if (r < n && lane == 0) {
-        if (MODE == 2) {
-            const T v = b[r] - acc;
-            y[r] = v;
-            contrib = (double)v * (double)v;
-        } else {
-            y[r] = acc;
-            if (MODE == 1) contrib = (double)x[r] * (double)acc;
-        }
-    }
+    csr_rows<L, T>(
+        n, rowptr, col, val, x, buf[threadIdx.x >> 6],
+        [&](int r) -> T { return MODE == 2 ? b[r] : (MODE == 1 ? x[r] : (T)0); },
+        [&](int r, T acc, T pv) {
+            if (MODE == 2) {
+                const T v = pv - acc;
+                y[r] = v;
+                contrib += (double)v * (double)v;
+            } else {
+                y[r] = acc;
+                if (MODE == 1) contrib += (double)pv * (double)acc;
+            }
+        });
     if (MODE != 0) {
         const double tot = block_sum256(contrib, s);
         if (threadIdx.x == 0) partial[blockIdx.x] = tot;
@@ -200,45 +188,90 @@ __global__ __launch_bounds__(256) void k_jacobi_apply(int n, const T *__restrict
     }
 }
 
+// Reliable update of the mixed solver: the FP64 residual replaces the FP32
+// recurrence's, z = tau r / diag (z = r without diag), partial (r, z).
+// keep: the direction, z + beta p with the recurrence's z, takes the new z in
+// its place (p += z_new - z_old), so a recurrence at its rounding floor leaves
+// nothing of its residual in it; otherwise the direction is z.
+__global__ __launch_bounds__(256) void k_cg_restart(int n, const double *__restrict__ r64, float *__restrict__ r,
+                                                    float *__restrict__ z, float *__restrict__ p,
+                                                    const float *__restrict__ diag, double tau, int keep,
+                                                    double *__restrict__ part_rz)
+{
+    __shared__ double s[4];
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    double v = 0.0;
+    if (i < n) {
+        const float rn = (float)r64[i];
+        const float zn = diag ? (float)tau * rn / diag[i] : rn;
+        const float zo = diag ? z[i] : r[i];
+        p[i] = keep ? p[i] + (zn - zo) : zn;
+        r[i] = rn;
+        z[i] = zn;
+        v = (double)rn * (double)zn;
+    }
+    const double tot = block_sum256(v, s);
+    if (threadIdx.x == 0) part_rz[blockIdx.x] = tot;
+}
+
 // Damped Jacobi smoothing step x += tau (b - A x) / diag, fused with the
 // SpMV (gsJacobiOp::step).  Reads x_in, writes x_out (x_in != x_out).
-template <int LPR, typename V, typename T>
+template <int L, typename V, typename T>
 __global__ __launch_bounds__(256) void k_jacobi_step(int n, const int *__restrict__ rowptr,
                                                      const int *__restrict__ col,
                                                      const V *__restrict__ val,
                                                      const T *__restrict__ diag,
                                                      const T *__restrict__ b, const T *__restrict__ xin,
-                                                     T *__restrict__ xout, T tau, int x_is_zero)
+                                                     T *__restrict__ xout, T tau)
 {
     // products and sums in FP64 whatever the storage type: an FP32 row sum
     // of a stiffness row cancels to a relative error of eps * cond(A), which
     // costs a multigrid preconditioner outer iterations
-    constexpr int RPB = 256 / LPR;
-    const int g = threadIdx.x / LPR, lane = threadIdx.x % LPR;
-    const int r = blockIdx.x * RPB + g;
-    double acc = 0.0;
-    if (r < n && !x_is_zero) {
-        const int k0 = rowptr[r], k1 = rowptr[r + 1];
-        for (int k = k0 + lane; k < k1; k += LPR) acc += (double)val[k] * (double)xin[col[k]];
-    }
-    acc = group_sum<LPR, double>(acc);
-    if (r < n && lane == 0) {
-        const double xo = x_is_zero ? 0.0 : (double)xin[r];
-        xout[r] = (T)(xo + (double)tau * ((double)b[r] - acc) / (double)diag[r]);
-    }
+    __shared__ double buf[4][kCsrCap];
+    struct Row { T x, b, d; };
+    csr_rows<L, double>(
+        n, rowptr, col, val, xin, buf[threadIdx.x >> 6], [&](int r) { return Row{xin[r], b[r], diag[r]}; },
+        [&](int r, double acc, const Row &q) {
+            xout[r] = (T)((double)q.x + (double)tau * ((double)q.b - acc) / (double)q.d);
+        });
 }
 
-// extract diagonal (value type V -> vector type T)
-template <typename V, typename T>
-__global__ void k_diag(int n, const int *__restrict__ rowptr, const int *__restrict__ col,
-                       const V *__restrict__ val, T *__restrict__ diag)
+// the same from x = 0: no product
+template <typename T>
+__global__ __launch_bounds__(256) void k_jacobi_first(int n, const T *__restrict__ diag, const T *__restrict__ b,
+                                                      T *__restrict__ xout, T tau)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n) return;
-    T d = 0;
-    for (int k = rowptr[r]; k < rowptr[r + 1]; ++k)
-        if (col[k] == r) { d = (T)val[k]; break; }
-    diag[r] = d;
+    const int r = blockIdx.x * 256 + threadIdx.x;
+    if (r < n) xout[r] = (T)((double)tau * (double)b[r] / (double)diag[r]);
+}
+
+// r = b - A x, FP64 sums whatever the storage type (see k_jacobi_step)
+template <int L, typename V, typename T>
+__global__ __launch_bounds__(256) void k_residual(int n, const int *__restrict__ rowptr, const int *__restrict__ col,
+                                                  const V *__restrict__ val, const T *__restrict__ x,
+                                                  const T *__restrict__ b, T *__restrict__ r)
+{
+    __shared__ double buf[4][kCsrCap];
+    csr_rows<L, double>(
+        n, rowptr, col, val, x, buf[threadIdx.x >> 6], [&](int i) -> T { return b[i]; },
+        [&](int i, double acc, T bi) { r[i] = (T)((double)bi - acc); });
+}
+
+// extract diagonal (value type V -> vector type T): kDiagLanes lanes look
+// through a row, its first entry in column r counts
+constexpr int kDiagLanes = 8;
+template <typename V, typename T>
+__global__ __launch_bounds__(256) void k_diag(int n, const int *__restrict__ rowptr, const int *__restrict__ col,
+                                              const V *__restrict__ val, T *__restrict__ diag)
+{
+    const int r = (int)((blockIdx.x * (int64_t)256 + threadIdx.x) / kDiagLanes), lane = threadIdx.x % kDiagLanes;
+    if (r >= n) return;   // the row's lanes leave together
+    int at = INT32_MAX;
+    for (int k = rowptr[r] + lane; k < rowptr[r + 1]; k += kDiagLanes)
+        if (col[k] == r) at = min(at, k);
+#pragma unroll
+    for (int off = kDiagLanes / 2; off > 0; off >>= 1) at = min(at, __shfl_xor(at, off, 64));
+    if (lane == 0) diag[r] = at == INT32_MAX ? (T)0 : (T)val[at];
 }
 
 template <typename S, typename D>
@@ -399,19 +432,20 @@ int spmv_lpr(double avg_row)
     return 8;
 }
 
-int spmv_blocks(int n, int lpr) { return (n + 256 / lpr - 1) / (256 / lpr); }
+int spmv_blocks(int n, int lpr) { return csr_blocks(n, csr_lanes(lpr)); }
 
 template <typename V, typename T, int MODE>
 static hipError_t spmv_dispatch(int lpr, int n, const int *rowptr, const int *col, const V *val,
                                 const T *x, T *y, const T *b, double *partial,
                                 const CGState *st, hipStream_t s)
 {
+    if (n <= 0) return hipSuccess;
     const dim3 grid(spmv_blocks(n, lpr)), block(256);
-    switch (lpr) {
-    case 64: hipLaunchKernelGGL((k_spmv<64, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st); break;
-    case 32: hipLaunchKernelGGL((k_spmv<32, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st); break;
+    switch (csr_lanes(lpr)) {
     case 16: hipLaunchKernelGGL((k_spmv<16, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st); break;
     case 8: hipLaunchKernelGGL((k_spmv<8, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st); break;
+    case 4: hipLaunchKernelGGL((k_spmv<4, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st); break;
+    case 2: hipLaunchKernelGGL((k_spmv<2, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -506,62 +540,99 @@ hipError_t launch_jacobi_apply_f32(int n, const float *r, float *z, const float 
     return hipGetLastError();
 }
 
+hipError_t launch_cg_restart(int n, const double *r64, float *r, float *z, float *p, const float *diag, double tau,
+                             int keep, double *prz, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_cg_restart, vgrid(n), dim3(256), 0, s, n, r64, r, z, p, diag, tau, keep, prz);
+    return hipGetLastError();
+}
+
+template <typename V, typename T>
+static hipError_t jacobi_dispatch(int lpr, int n, const int *rp, const int *ci, const V *v, const T *diag, const T *b,
+                                  const T *xin, T *xout, T tau, int x_is_zero, hipStream_t s)
+{
+    if (n <= 0) return hipSuccess;
+    if (x_is_zero) {
+        hipLaunchKernelGGL((k_jacobi_first<T>), dim3((n + 255) / 256), dim3(256), 0, s, n, diag, b, xout, tau);
+        return hipGetLastError();
+    }
+    const dim3 grid(spmv_blocks(n, lpr)), block(256);
+    switch (csr_lanes(lpr)) {
+    case 16: hipLaunchKernelGGL((k_jacobi_step<16, V, T>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau); break;
+    case 8: hipLaunchKernelGGL((k_jacobi_step<8, V, T>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau); break;
+    case 4: hipLaunchKernelGGL((k_jacobi_step<4, V, T>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau); break;
+    case 2: hipLaunchKernelGGL((k_jacobi_step<2, V, T>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 hipError_t launch_jacobi_step_f64(int lpr, int n, const int *rp, const int *ci, const double *v,
                                   const double *diag, const double *b, const double *xin,
                                   double *xout, double tau, int x_is_zero, hipStream_t s)
 {
-    const dim3 grid(spmv_blocks(n, lpr)), block(256);
-    switch (lpr) {
-    case 64: hipLaunchKernelGGL((k_jacobi_step<64, double, double>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero); break;
-    case 32: hipLaunchKernelGGL((k_jacobi_step<32, double, double>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero); break;
-    case 16: hipLaunchKernelGGL((k_jacobi_step<16, double, double>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero); break;
-    case 8: hipLaunchKernelGGL((k_jacobi_step<8, double, double>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    return jacobi_dispatch(lpr, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero, s);
 }
 
 hipError_t launch_jacobi_step_v32(int lpr, int n, const int *rp, const int *ci, const float *v,
                                   const double *diag, const double *b, const double *xin,
                                   double *xout, double tau, int x_is_zero, hipStream_t s)
 {
-    const dim3 grid(spmv_blocks(n, lpr)), block(256);
-    switch (lpr) {
-    case 64: hipLaunchKernelGGL((k_jacobi_step<64, float, double>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero); break;
-    case 32: hipLaunchKernelGGL((k_jacobi_step<32, float, double>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero); break;
-    case 16: hipLaunchKernelGGL((k_jacobi_step<16, float, double>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero); break;
-    case 8: hipLaunchKernelGGL((k_jacobi_step<8, float, double>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    return jacobi_dispatch(lpr, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero, s);
 }
 
 hipError_t launch_jacobi_step_f32(int lpr, int n, const int *rp, const int *ci, const float *v,
                                   const float *diag, const float *b, const float *xin,
                                   float *xout, float tau, int x_is_zero, hipStream_t s)
 {
+    return jacobi_dispatch(lpr, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero, s);
+}
+
+template <typename V, typename T>
+static hipError_t residual_dispatch(int lpr, int n, const int *rp, const int *ci, const V *v, const T *x, const T *b,
+                                    T *r, hipStream_t s)
+{
+    if (n <= 0) return hipSuccess;
     const dim3 grid(spmv_blocks(n, lpr)), block(256);
-    switch (lpr) {
-    case 64: hipLaunchKernelGGL((k_jacobi_step<64, float, float>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero); break;
-    case 32: hipLaunchKernelGGL((k_jacobi_step<32, float, float>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero); break;
-    case 16: hipLaunchKernelGGL((k_jacobi_step<16, float, float>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero); break;
-    case 8: hipLaunchKernelGGL((k_jacobi_step<8, float, float>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau, x_is_zero); break;
+    switch (csr_lanes(lpr)) {
+    case 16: hipLaunchKernelGGL((k_residual<16, V, T>), grid, block, 0, s, n, rp, ci, v, x, b, r); break;
+    case 8: hipLaunchKernelGGL((k_residual<8, V, T>), grid, block, 0, s, n, rp, ci, v, x, b, r); break;
+    case 4: hipLaunchKernelGGL((k_residual<4, V, T>), grid, block, 0, s, n, rp, ci, v, x, b, r); break;
+    case 2: hipLaunchKernelGGL((k_residual<2, V, T>), grid, block, 0, s, n, rp, ci, v, x, b, r); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
+hipError_t launch_residual_f64(int lpr, int n, const int *rp, const int *ci, const double *v, const double *x,
+                               const double *b, double *r, hipStream_t s)
+{
+    return residual_dispatch<double, double>(lpr, n, rp, ci, v, x, b, r, s);
+}
+
+hipError_t launch_residual_v32(int lpr, int n, const int *rp, const int *ci, const float *v, const double *x,
+                               const double *b, double *r, hipStream_t s)
+{
+    return residual_dispatch<float, double>(lpr, n, rp, ci, v, x, b, r, s);
+}
+
+hipError_t launch_residual_f32(int lpr, int n, const int *rp, const int *ci, const float *v, const float *x,
+                               const float *b, float *r, hipStream_t s)
+{
+    return residual_dispatch<float, float>(lpr, n, rp, ci, v, x, b, r, s);
+}
+
 hipError_t launch_diag_f64(int n, const int *rp, const int *ci, const double *v, double *diag,
                            hipStream_t s)
 {
-    hipLaunchKernelGGL((k_diag<double, double>), dim3((n + 255) / 256), dim3(256), 0, s, n, rp, ci, v, diag);
+    hipLaunchKernelGGL((k_diag<double, double>), dim3((unsigned)(((int64_t)n * kDiagLanes + 255) / 256)), dim3(256), 0, s, n, rp, ci, v, diag);
     return hipGetLastError();
 }
 
 hipError_t launch_diag_f32(int n, const int *rp, const int *ci, const float *v, float *diag,
                            hipStream_t s)
 {
-    hipLaunchKernelGGL((k_diag<float, float>), dim3((n + 255) / 256), dim3(256), 0, s, n, rp, ci, v, diag);
+    hipLaunchKernelGGL((k_diag<float, float>), dim3((unsigned)(((int64_t)n * kDiagLanes + 255) / 256)), dim3(256), 0, s, n, rp, ci, v, diag);
     return hipGetLastError();
 }
 

@@ -122,3 +122,30 @@ def test_structured_cg_tiles(ctx, d, p, n):
         x.close()
     for o in (A, b, gp):
         o.close()
+
+
+# CSR row sums: waves of 64 / L rows, entries in pairs, LDS chunks of 512
+@pytest.mark.parametrize("n,lo,hi", [(1, 1, 1), (3, 0, 2), (65, 1, 9), (513, 0, 40), (1000, 30, 60), (301, 90, 420),
+                                     (37, 700, 1300), (70000, 0, 12)])
+def test_csr_products(ctx, n, lo, hi):
+    """gsx_spmv on matrices with ragged, empty and long rows, and Jacobi
+    sweeps of a multigrid hierarchy over them."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(n)
+    m = max(n, 1400)   # distinct columns for the longest rows come from a window
+    lens = rng.integers(lo, hi + 1, n)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    ci = np.concatenate([np.sort(rng.choice(min(n, m), min(k, n), replace=False)) if k else np.zeros(0, int)
+                         for k in lens]).astype(np.int32)
+    rp = np.concatenate([[0], np.cumsum(np.minimum(lens, n))]).astype(np.int32)
+    va = rng.standard_normal(rp[-1])
+    M = sp.csr_matrix((va, ci, rp), shape=(n, n))
+    A = gsx.Matrix.from_csr(ctx, rp, ci, va)
+    x = rng.standard_normal(n)
+    xd, yd = ctx.to_device(x), ctx.array(n)
+    A.spmv(xd, yd)
+    # each row sum rounds by at most its length times eps of its absolute sum
+    bound = 1e-16 * (1 + np.minimum(lens, n)) * (abs(M) @ abs(x)) + 1e-300
+    assert np.all(np.abs(yd.download() - M @ x) <= 4 * bound)
+    for o in (xd, yd, A):
+        o.close()
