@@ -114,6 +114,14 @@ struct SpmvGrid {
     const int *f2g;
 };
 
+// A matrix in slices of 64 rows (gsx_sell.hip): entry k of row r of slice s at
+// (sptr[s] + k) 64 + r of the value array; columns likewise, or for a uniform
+// slice the offsets col - row at sptr[s] 64 + k.
+struct SellOp {
+    int n;
+    const int *sptr, *uniform, *col;
+};
+
 // One boundary element: the element of `patch` adjacent to side `side`
 // (1..2d) at element index ei, the condition's type (1 Dirichlet, 2
 // Neumann), data kind (0 zero, 1 manufactured, 2 affine) and values.

@@ -330,4 +330,24 @@ hipError_t launch_scatter_add_idx(int n, const int *idx, const double *z, double
 // val(row r) *= 1 / L(r); err[0] = 1 on L(r) == 0
 hipError_t launch_scale_rows(int nrows, const int *rowptr, const double *L, double *val, int *err, hipStream_t s);
 
+// Sliced ELL level operators (gsx_sell.hip).
+int sell_blocks(int n);
+hipError_t launch_sell_width(int n, const int *rowptr, int *width, hipStream_t s);
+hipError_t launch_sell_fill(int n, const int *rowptr, const int *col, const double *val, const int *sptr, int *uniform,
+                            int *scol, float *sval32, double *sval64, hipStream_t s);
+hipError_t launch_sell_jacobi_f64(const SellOp &S, const double *v, const double *diag, const double *b,
+                                  const double *xin, double *xout, double tau, hipStream_t s);
+hipError_t launch_sell_jacobi_v32(const SellOp &S, const float *v, const double *diag, const double *b,
+                                  const double *xin, double *xout, double tau, hipStream_t s);
+hipError_t launch_sell_jacobi_f32(const SellOp &S, const float *v, const float *diag, const float *b,
+                                  const float *xin, float *xout, float tau, hipStream_t s);
+hipError_t launch_sell_residual_f64(const SellOp &S, const double *v, const double *x, const double *b, double *y,
+                                    hipStream_t s);
+hipError_t launch_sell_residual_v32(const SellOp &S, const float *v, const double *x, const double *b, double *y,
+                                    hipStream_t s);
+hipError_t launch_sell_residual_f32(const SellOp &S, const float *v, const float *x, const float *b, float *y,
+                                    hipStream_t s);
+hipError_t launch_sell_spmv(const SellOp &S, const double *v, const double *x, double *y, double *partial,
+                            const CGState *st, hipStream_t s);
+
 }  // namespace gsx

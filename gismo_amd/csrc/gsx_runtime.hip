@@ -1471,7 +1471,7 @@ static gsx_status cg_workspace(gsx_matrix *A, int maxit, bool mixed, bool grid =
     if (w.n != n || !w.r) {
         w = CGWork();
         w.n = n;
-        w.nparts = std::max(gsx::spmv_blocks(n, A->lpr), (n + 255) / 256) + 1;
+        w.nparts = std::max({gsx::spmv_blocks(n, A->lpr), gsx::sell_blocks(n), (n + 255) / 256}) + 1;
         w.r = dalloc(c, sizeof(double) * n);
         w.z = dalloc(c, sizeof(double) * n);
         w.p = dalloc(c, sizeof(double) * n);
@@ -2676,6 +2676,9 @@ struct MGLevel {
     DevPtr x, b, r, t;                 // FP64
     DevPtr x32, b32, r32, t32;         // FP32
     DevPtr d, d32;                     // polynomial smoother direction
+    // the operator in slices of 64 rows (mg_sell); null: CSR kernels
+    DevPtr sl_ptr, sl_uni, sl_col, sl_val, sl_val32;
+    gsx::SellOp sell() const { return gsx::SellOp{n, dp<int>(sl_ptr), dp<int>(sl_uni), dp<int>(sl_col)}; }
     double lmax = 0.0;                 // Chebyshev: bound of lambda(D^-1 A)
     // Gauss-Seidel: rows by level set, forward and reverse sweep
     DevPtr gs_fwd, gs_rev;
@@ -2888,6 +2891,38 @@ static int rcm_order(int n, const std::vector<int> &rp, const std::vector<int> &
 // Per-level diagonals, FP32 copies and vectors, then the exact coarse solve
 // (the dense inverse of the coarsest operator or, above the context's
 // coarse_dense_max rows, its banded FP64 Cholesky factor).
+// Slices of level l's operator, unless padding would add more than a quarter
+// of its entries (very uneven rows): FP32 values for the levels a mixed cycle
+// reads in FP32, FP64 values otherwise and on the finest level (the outer CG).
+static gsx_status mg_sell(gsx_mg *mg, int l)
+{
+    gsx_ctx *c = mg->ctx;
+    hipStream_t s = c->stream;
+    MGLevel &V = mg->L[l];
+    const bool mixed = mg->precision == GSX_MIXED, finest = l == (int)mg->L.size() - 1;
+    if (V.n <= 0 || V.nnz <= 0) return GSX_OK;
+    const int nsl = (V.n + 63) / 64;
+    DevPtr width = dalloc(c, sizeof(int) * nsl);
+    if (!width) return fail(c, GSX_ERR_OOM, "device allocation (level slices)");
+    HIP_OK(c, gsx::launch_sell_width(V.n, dp<int>(V.rowptr), dp<int>(width), s));
+    DevPtr ptr;
+    int64_t total = 0;
+    GSX_TRY(scan_counts(c, dp<int>(width), nsl, ptr, total));
+    if ((double)total * 64 > 1.25 * (double)V.nnz + 65536.0) return GSX_OK;
+    const size_t slots = (size_t)std::max<int64_t>(1, total) * 64;
+    V.sl_uni = dalloc(c, sizeof(int) * nsl);
+    V.sl_col = dalloc(c, sizeof(int) * slots);
+    if (mixed) V.sl_val32 = dalloc(c, sizeof(float) * slots);
+    if (!mixed || finest) V.sl_val = dalloc(c, sizeof(double) * slots);
+    if (!V.sl_uni || !V.sl_col || (mixed && !V.sl_val32) || ((!mixed || finest) && !V.sl_val))
+        return fail(c, GSX_ERR_OOM, "device allocation (level slices)");
+    HIP_OK(c, gsx::launch_sell_fill(V.n, dp<int>(V.rowptr), dp<int>(V.col), dp<double>(V.val), dp<int>(ptr),
+                                    dp<int>(V.sl_uni), dp<int>(V.sl_col), dp<float>(V.sl_val32), dp<double>(V.sl_val),
+                                    s));
+    V.sl_ptr = ptr;
+    return GSX_OK;
+}
+
 static gsx_status mg_finish(gsx_mg *mg)
 {
     gsx_ctx *c = mg->ctx;
@@ -2916,6 +2951,7 @@ static gsx_status mg_finish(gsx_mg *mg)
             }
         }
         GSX_TRY(mg_level_vectors(c, V, mixed));
+        if (l > 0) GSX_TRY(mg_sell(mg, l));
     }
     // exact coarse solve: the dense inverse up to coarse_dense_max rows (one
     // GEMV per solve); above, a banded FP64 Cholesky factor in reverse
@@ -3786,6 +3822,46 @@ static SmoothCoef smooth_coef(const gsx_mg *mg, const MGLevel &V, int k, double 
 // m smoothing sweeps on level V with FP64 vectors (matrix values FP64, or
 // FP32 when v32: the finest level of a mixed cycle).  Jacobi ping-pongs x
 // and t (x may come back as t); the polynomial smoothers update x in place.
+// r = b - A x and one damped Jacobi step of a level, on its slices or its CSR
+// arrays; v32: FP64 vectors on the FP32 values
+static hipError_t level_residual64(const MGLevel &V, bool v32, const double *x, const double *b, double *r,
+                                   hipStream_t s)
+{
+    if (V.sl_ptr)
+        return v32 ? gsx::launch_sell_residual_v32(V.sell(), dp<float>(V.sl_val32), x, b, r, s)
+                   : gsx::launch_sell_residual_f64(V.sell(), dp<double>(V.sl_val), x, b, r, s);
+    const int *rp = dp<int>(V.rowptr), *ci = dp<int>(V.col);
+    return v32 ? gsx::launch_residual_v32(V.lpr, V.n, rp, ci, dp<float>(V.val32), x, b, r, s)
+               : gsx::launch_residual_f64(V.lpr, V.n, rp, ci, dp<double>(V.val), x, b, r, s);
+}
+
+static hipError_t level_residual32(const MGLevel &V, const float *x, const float *b, float *r, hipStream_t s)
+{
+    if (V.sl_ptr) return gsx::launch_sell_residual_f32(V.sell(), dp<float>(V.sl_val32), x, b, r, s);
+    return gsx::launch_residual_f32(V.lpr, V.n, dp<int>(V.rowptr), dp<int>(V.col), dp<float>(V.val32), x, b, r, s);
+}
+
+static hipError_t level_jacobi64(const MGLevel &V, bool v32, const double *b, const double *x, double *xn, bool zero,
+                                 hipStream_t s)
+{
+    const double *dg = dp<double>(V.diag);
+    if (V.sl_ptr && !zero)
+        return v32 ? gsx::launch_sell_jacobi_v32(V.sell(), dp<float>(V.sl_val32), dg, b, x, xn, V.tau, s)
+                   : gsx::launch_sell_jacobi_f64(V.sell(), dp<double>(V.sl_val), dg, b, x, xn, V.tau, s);
+    const int *rp = dp<int>(V.rowptr), *ci = dp<int>(V.col);
+    return v32 ? gsx::launch_jacobi_step_v32(V.lpr, V.n, rp, ci, dp<float>(V.val32), dg, b, x, xn, V.tau, zero, s)
+               : gsx::launch_jacobi_step_f64(V.lpr, V.n, rp, ci, dp<double>(V.val), dg, b, x, xn, V.tau, zero, s);
+}
+
+static hipError_t level_jacobi32(const MGLevel &V, const float *b, const float *x, float *xn, bool zero, hipStream_t s)
+{
+    const float *dg = dp<float>(V.diag32);
+    if (V.sl_ptr && !zero)
+        return gsx::launch_sell_jacobi_f32(V.sell(), dp<float>(V.sl_val32), dg, b, x, xn, (float)V.tau, s);
+    return gsx::launch_jacobi_step_f32(V.lpr, V.n, dp<int>(V.rowptr), dp<int>(V.col), dp<float>(V.val32), dg, b, x, xn,
+                                       (float)V.tau, zero, s);
+}
+
 static gsx_status smooth64(gsx_mg *mg, MGLevel &V, double *&x, double *&t, const double *b, bool &zero, int m,
                            bool v32, bool post)
 {
@@ -3794,10 +3870,7 @@ static gsx_status smooth64(gsx_mg *mg, MGLevel &V, double *&x, double *&t, const
     const int *rp = dp<int>(V.rowptr), *ci = dp<int>(V.col);
     const double *va = dp<double>(V.val), *dg = dp<double>(V.diag);
     const float *va32 = v32 ? dp<float>(V.val32) : nullptr;
-    auto residual = [&](const double *xx, double *rr) {
-        return v32 ? gsx::launch_residual_v32(V.lpr, V.n, rp, ci, va32, xx, b, rr, s)
-                   : gsx::launch_residual_f64(V.lpr, V.n, rp, ci, va, xx, b, rr, s);
-    };
+    auto residual = [&](const double *xx, double *rr) { return level_residual64(V, v32, xx, b, rr, s); };
     if (V.smoother == GSX_SMOOTH_GAUSS_SEIDEL) {
         if (m > 0 && zero) HIP_OK(c, gsx::launch_fill_f64(x, V.n, 0.0, s));
         const int *rows = dp<int>(post ? V.gs_rev : V.gs_fwd);
@@ -3852,10 +3925,7 @@ static gsx_status smooth64(gsx_mg *mg, MGLevel &V, double *&x, double *&t, const
     }
     if (V.smoother == GSX_SMOOTH_JACOBI) {
         for (int i = 0; i < m; ++i) {
-            if (v32)
-                HIP_OK(c, gsx::launch_jacobi_step_v32(V.lpr, V.n, rp, ci, va32, dg, b, x, t, V.tau, zero ? 1 : 0, s));
-            else
-                HIP_OK(c, gsx::launch_jacobi_step_f64(V.lpr, V.n, rp, ci, va, dg, b, x, t, V.tau, zero ? 1 : 0, s));
+            HIP_OK(c, level_jacobi64(V, v32, b, x, t, zero, s));
             std::swap(x, t);
             zero = false;
         }
@@ -3896,7 +3966,7 @@ static gsx_status smooth32(gsx_mg *mg, MGLevel &V, float *&x, float *&t, const f
         float *r = dp<float>(V.r32), *d = dp<float>(V.d32);
         const gsx_fd *F = V.scms.get();
         for (int k = 0; k < m; ++k) {
-            HIP_OK(c, gsx::launch_residual_f32(V.lpr, V.n, rp, ci, va, x, b, r, s));
+            HIP_OK(c, level_residual32(V, x, b, r, s));
             HIP_OK(c, fd_apply<float>(F, r, 0, F->m[0], (int64_t)F->m[0] * F->m[1], d, 0, F->m[0],
                                       (int64_t)F->m[0] * F->m[1], nullptr, s));
             HIP_OK(c, gsx::launch_smooth_update_f32(V.n, x, d, d, nullptr, 0.0f, (float)V.scms_tau, 1, s));
@@ -3906,7 +3976,7 @@ static gsx_status smooth32(gsx_mg *mg, MGLevel &V, float *&x, float *&t, const f
     }
     if (V.smoother == GSX_SMOOTH_JACOBI) {
         for (int i = 0; i < m; ++i) {
-            HIP_OK(c, gsx::launch_jacobi_step_f32(V.lpr, V.n, rp, ci, va, dg, b, x, t, (float)V.tau, zero ? 1 : 0, s));
+            HIP_OK(c, level_jacobi32(V, b, x, t, zero, s));
             std::swap(x, t);
             zero = false;
         }
@@ -3916,7 +3986,7 @@ static gsx_status smooth32(gsx_mg *mg, MGLevel &V, float *&x, float *&t, const f
     float *r = dp<float>(V.r32), *d = dp<float>(V.d32);
     double rho = 0.0;
     for (int k = 0; k < m; ++k) {
-        HIP_OK(c, gsx::launch_residual_f32(V.lpr, V.n, rp, ci, va, x, b, r, s));
+        HIP_OK(c, level_residual32(V, x, b, r, s));
         const SmoothCoef cf = smooth_coef(mg, V, k, rho);
         HIP_OK(c, gsx::launch_smooth_update_f32(V.n, x, d, r, V.smoother == GSX_SMOOTH_CHEBYSHEV ? dg : nullptr,
                                                 (float)cf.c1, (float)cf.c2, k == 0 ? 1 : 0, s));
@@ -3948,8 +4018,6 @@ static gsx_status mg_cycle64(gsx_mg *mg, int l, bool mixed = false)
             HIP_OK(c, gsx::launch_dense_gemv_f64(V.n, mg->npad, dp<double>(mg->Dinv), b, x, s));
         return GSX_OK;
     }
-    const int *rp = dp<int>(V.rowptr), *ci = dp<int>(V.col);
-    const double *va = dp<double>(V.val);
     bool zero = true;
     {
         KScope k(c, "mg_smooth");
@@ -3959,8 +4027,7 @@ static gsx_status mg_cycle64(gsx_mg *mg, int l, bool mixed = false)
     {
         KScope k(c, "mg_transfer");
         if (zero) HIP_OK(c, hipMemcpyAsync(r, b, sizeof(double) * V.n, hipMemcpyDeviceToDevice, s));
-        else if (mixed) HIP_OK(c, gsx::launch_residual_v32(V.lpr, V.n, rp, ci, dp<float>(V.val32), x, b, r, s));
-        else HIP_OK(c, gsx::launch_residual_f64(V.lpr, V.n, rp, ci, va, x, b, r, s));
+        else HIP_OK(c, level_residual64(V, mixed, x, b, r, s));
         if (mixed)
             HIP_OK(c, gsx::launch_restrict_v32(C.n, dp<int>(C.rrp), dp<int>(C.rci), dp<float>(C.rv32), r,
                                                dp<float>(C.b32), s));
@@ -4009,8 +4076,6 @@ static gsx_status mg_cycle32(gsx_mg *mg, int l)
         HIP_OK(c, gsx::launch_conv_f64_f32(V.n, dp<double>(V.x), x, s));
         return GSX_OK;
     }
-    const int *rp = dp<int>(V.rowptr), *ci = dp<int>(V.col);
-    const float *va = dp<float>(V.val32);
     bool zero = true;
     {
         KScope k(c, "mg_smooth");
@@ -4020,7 +4085,7 @@ static gsx_status mg_cycle32(gsx_mg *mg, int l)
     {
         KScope k(c, "mg_transfer");
         if (zero) HIP_OK(c, hipMemcpyAsync(r, b, sizeof(float) * V.n, hipMemcpyDeviceToDevice, s));
-        else HIP_OK(c, gsx::launch_residual_f32(V.lpr, V.n, rp, ci, va, x, b, r, s));
+        else HIP_OK(c, level_residual32(V, x, b, r, s));
         HIP_OK(c, gsx::launch_restrict_f32(C.n, dp<int>(C.rrp), dp<int>(C.rci), dp<float>(C.rv32), r, dp<float>(C.b32), s));
     }
     GSX_TRY(mg_cycle32(mg, l - 1));
@@ -4479,6 +4544,10 @@ static gsx_status cg_mg(gsx_matrix *A, gsx_mg *mg, const double *b, double *x, d
     CGWork &w = A->ws;
     const int n = A->n, np = w.nparts;
     const int ns = gsx::spmv_blocks(n, A->lpr), nv = (n + 255) / 256;
+    // the hierarchy's slices of its finest operator, if that is A
+    const MGLevel &F = mg->L.back();
+    const bool sell = F.sl_ptr && F.sl_val && F.val == A->val && F.rowptr == A->rowptr && F.n == n;
+    const int nsp = sell ? gsx::sell_blocks(n) : ns;
     double *P0 = dp<double>(w.parts), *P1 = P0 + np;
     CGState *st = dp<CGState>(w.state);
     double *hist = dp<double>(w.hist);
@@ -4502,9 +4571,10 @@ static gsx_status cg_mg(gsx_matrix *A, gsx_mg *mg, const double *b, double *x, d
         while (true) {
             {
                 KScope k(c, "spmv_f64");
-                HIP_OK(c, gsx::launch_spmv_f64(A->lpr, n, rp, ci, va, p, t, nullptr, P0, 1, st, s));
+                if (sell) HIP_OK(c, gsx::launch_sell_spmv(F.sell(), dp<double>(F.sl_val), p, t, P0, st, s));
+                else HIP_OK(c, gsx::launch_spmv_f64(A->lpr, n, rp, ci, va, p, t, nullptr, P0, 1, st, s));
             }
-            HIP_OK(c, gsx::launch_cg_scalar(2, P0, ns, nullptr, 0, st, hist, s));
+            HIP_OK(c, gsx::launch_cg_scalar(2, P0, nsp, nullptr, 0, st, hist, s));
             HIP_OK(c, gsx::launch_cg_xr_f64(n, x, r, p, t, P1, st, s));
             HIP_OK(c, gsx::launch_cg_scalar(5, P1, nv, nullptr, 0, st, hist, s));
             GSX_TRY(read_state(c, w, h));

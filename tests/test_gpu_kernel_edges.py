@@ -149,3 +149,47 @@ def test_csr_products(ctx, n, lo, hi):
     assert np.all(np.abs(yd.download() - M @ x) <= 4 * bound)
     for o in (xd, yd, A):
         o.close()
+
+
+# level operators in slices of 64 rows: several slices per wave block, four
+# waves per slice below 131,072 rows, uniform slices (inside a patch), a last
+# slice of one row, interface rows; against the cycle written out in scipy
+@pytest.mark.parametrize("gx,gy,n,p,levels", [(1, 1, 16, 2, 2), (2, 1, 12, 3, 2), (3, 2, 24, 3, 3), (2, 2, 8, 4, 2),
+                                              (1, 1, 374, 2, 2)])
+@pytest.mark.parametrize("prec", [gsx.FP64, gsx.MIXED])
+def test_multigrid_level_slices(ctx, gx, gy, n, p, levels, prec):
+    prob = problems.square_grid(gx, gy, n, p)
+    for k, P in enumerate(prob.patches):
+        problems.perturb_interior(P, 0.1 / n, 30 + k)
+    gp = gsx.Problem(ctx, prob)
+    A, b = gp.assemble(gsx.PATTERN_FULL | gsx.ASM_KEEP_ELEMENTS, prec)
+    mg = gsx.Multigrid(gp, A, levels, 2, 1, 0.7, precision=prec)
+    ops = [mg.level(l) for l in range(levels)]
+    import scipy.sparse.linalg as spla
+
+    def cycle(l, rhs):
+        M = ops[l][0]
+        if l == 0:
+            return spla.spsolve(M.tocsc(), rhs)
+        d = M.diagonal()
+        x = np.zeros_like(rhs)
+        for _ in range(2):
+            x = x + 0.7 * (rhs - M @ x) / d
+        P = ops[l - 1][1]
+        x = x + P @ cycle(l - 1, P.T @ (rhs - M @ x))
+        return x + 0.7 * (rhs - M @ x) / d
+    r = np.random.default_rng(4).standard_normal(gp.nfree)
+    want = cycle(levels - 1, r)
+    rd, zd = ctx.to_device(r), ctx.array(gp.nfree)
+    mg.apply(rd, zd)
+    # FP64: sums of at most 81 entries per smoothing step, cond(A_0) < 1e4;
+    # mixed: level values and coarse vectors rounded to FP32 (6e-8), amplified
+    # by the cycle's bounded operators
+    tol = 1e-10 if prec == gsx.FP64 else 2e-5
+    assert np.linalg.norm(zd.download() - want) <= tol * np.linalg.norm(want)
+    x = ctx.array(gp.nfree).zero()
+    it, rel, ok = gsx.mg_cg_solve(A, mg, b, x, tol=1e-9)
+    bb = b.download()
+    assert ok and np.linalg.norm(bb - A.to_scipy() @ x.download()) <= 1.01e-9 * np.linalg.norm(bb)
+    for o in (rd, zd, x, mg, A, b, gp):
+        o.close()
