@@ -54,7 +54,7 @@ __device__ inline double source_value(int fkind, int d, const double *x, const d
     if (fkind == 1) {
         const double pi = 3.14159265358979323846;
         double v = (double)d * pi * pi;
-        for (int r = 0; r < d; ++r) v *= sin(pi * x[r]);
+        for (int r = 0; r < d; ++r) v *= sinpi(x[r]);
         return v;
     }
     return felem ? felem[e] : 0.0;

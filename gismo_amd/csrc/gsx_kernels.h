@@ -22,13 +22,15 @@ int64_t sf_dq_doubles(int p, const int *nel);
 // tables, element load vectors + det check (+ D), stencil rows (FP64, all
 // slots of free rows whose column is in the patch); the tiling (nty, ntz)
 // is chosen here
-hipError_t launch_sf_assemble(int p, const PatchDev *patches, const GaussTab &gt, double *tab, SfBox bx,
-                              double *Fbuf, double *detmin, double *Dq, double *s64, int64_t nelem, hipStream_t s);
-// CSR values, FP32 half stencil (may be null), rhs; zeroes the slots of
-// columns outside the free box; err |= 1 on a CSR row length mismatch
-hipError_t launch_sf_finish(int p, const SfBox &bx, int nfree, const int *rowptr, double *s64, float *s32,
-                            double *val, double *rhs, const double *Fbuf, const int *dofs, const double *fixed,
-                            int *err, hipStream_t s);
+// raw rows, z sums of the load and per-block determinant minima (doubles)
+int64_t sf_raw_doubles(int p, const int *nb);
+int64_t sf_load_doubles(int p, const int *nel);
+int64_t sf_det_count(int p, const int *nel);
+hipError_t launch_sf_assemble(int p, const PatchDev *patches, const GaussTab &gt, double *tab, SfBox bx, double *R1,
+                              double *detmin, double *Dq, double *raw, double *rhs, hipStream_t s);
+hipError_t launch_sf_finish(int p, const SfBox &bx, int nfree, const int *rowptr, const double *raw, double *s64,
+                            float *s32, double *val, double *rhs, const int *dofs, const double *fixed, int *err,
+                            hipStream_t s);
 
 // assembly
 hipError_t launch_elem(int d, int p, const PatchDev *patches, const int *gpatch,

@@ -1146,7 +1146,7 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
     const int64_t kcap = use_sf ? 0
                          : single ? std::min<int64_t>(h0.nel[sd], slab_rows + h0.p[0]) * layer_elems * nb0 * nb0
                                   : P->kdoubles;
-    const int64_t fcap = use_sf ? P->nelem * nb0
+    const int64_t fcap = use_sf ? gsx::sf_load_doubles(h0.p[0], h0.nel)   // z sums of the load
                          : single ? std::min<int64_t>(h0.nel[sd], slab_rows + h0.p[0]) * layer_elems * nb0
                                   : P->fdoubles;
     DevPtr Kbuf = dalloc(c, sizeof(double) * std::max<int64_t>(1, kcap));
@@ -1226,27 +1226,22 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
             sb.ntz = (h.nb[2] + 1) / 2;
             DevPtr tab = dalloc(c, sizeof(double) * gsx::sf_table_doubles(p, h.nel));
             DevPtr dq = dalloc(c, sizeof(double) * std::max<int64_t>(1, gsx::sf_dq_doubles(p, h.nel)));
-            DevPtr s64tmp;
-            double *s64 = dp<double>(S.s64);
-            if (!s64) {
-                s64tmp = dalloc(c, sizeof(double) * gsx::stencil_size(A->n, (int)S.slots));
-                s64 = dp<double>(s64tmp);
-            }
+            DevPtr raw = dalloc(c, sizeof(double) * gsx::sf_raw_doubles(p, h.nb));
             DevPtr errf = dalloc(c, sizeof(int));
-            if (!tab || !dq || !s64 || !errf) return fail(c, GSX_ERR_OOM, "device allocation (row assembly)");
+            if (!tab || !dq || !raw || !errf) return fail(c, GSX_ERR_OOM, "device allocation (row assembly)");
             HIP_OK(c, hipMemsetAsync(errf.get(), 0, sizeof(int), s));
             {
                 KScope k(c, "sf_assemble");
                 HIP_OK(c, gsx::launch_sf_assemble(p, dp<PatchDev>(P->d_patches), c->gt, dp<double>(tab), sb,
-                                                  dp<double>(Fbuf), dp<double>(P->d_detmin), dp<double>(dq), s64,
-                                                  P->nelem, s));
+                                                  dp<double>(Fbuf), dp<double>(P->d_detmin), dp<double>(dq),
+                                                  dp<double>(raw), rhs, s));
             }
             {
                 KScope k(c, "sf_finish");
-                HIP_OK(c, gsx::launch_sf_finish(p, sb, P->nfree, dp<int>(P->d_rowptr), s64,
-                                                S.s32 ? dp<float>(S.s32) : nullptr, dp<double>(A->val), rhs,
-                                                dp<double>(Fbuf), dp<int>(P->d_dofs),
-                                                P->d_fixed ? dp<double>(P->d_fixed) : nullptr, dp<int>(errf), s));
+                HIP_OK(c, gsx::launch_sf_finish(p, sb, P->nfree, dp<int>(P->d_rowptr), dp<double>(raw),
+                                                dp<double>(S.s64), dp<float>(S.s32), dp<double>(A->val), rhs,
+                                                dp<int>(P->d_dofs), P->d_fixed ? dp<double>(P->d_fixed) : nullptr,
+                                                dp<int>(errf), s));
             }
             int errh = 0;
             HIP_OK(c, hipMemcpyAsync(&errh, errf.get(), sizeof(int), hipMemcpyDeviceToHost, s));
@@ -1304,7 +1299,8 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
     Kbuf.reset();
     Fbuf.reset();
     double *dmin_slot = dp<double>(P->d_detmin) + std::max<int64_t>(1, P->nelem);
-    HIP_OK(c, gsx::launch_min(dp<double>(P->d_detmin), P->nelem, dmin_slot, s));
+    HIP_OK(c, gsx::launch_min(dp<double>(P->d_detmin),
+                              use_sf ? gsx::sf_det_count(h0.p[0], h0.nel) : P->nelem, dmin_slot, s));
     double mind = 0.0;
     HIP_OK(c, hipMemcpyAsync(&mind, dmin_slot, sizeof(double), hipMemcpyDeviceToHost, s));
     if (mode == GSX_PATTERN_EXPR && keep) {

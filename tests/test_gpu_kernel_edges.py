@@ -193,3 +193,45 @@ def test_multigrid_level_slices(ctx, gx, gy, n, p, levels, prec):
     assert ok and np.linalg.norm(bb - A.to_scipy() @ x.download()) <= 1.01e-9 * np.linalg.norm(bb)
     for o in (rd, zd, x, mg, A, b, gp):
         o.close()
+
+
+# the row assembly: tiles of 4 x 4 (2 x 3) rows in (y, z) split along x, Gauss
+# point columns in chunks along z, x-line segments of 64 and of 16 (8) rows;
+# boxes thinner than a chunk, a tile or the stencil, and eliminated columns
+# moved to the right-hand side
+@pytest.mark.parametrize("p,n", [(1, (1, 2, 3)), (1, (70, 4, 5)), (2, (1, 1, 1)), (2, (2, 5, 17)), (2, (67, 3, 2)),
+                                 (3, (1, 1, 9)), (3, (17, 5, 4)), (3, (4, 18, 3)), (4, (1, 2, 1)), (4, (9, 2, 5)),
+                                 (4, (2, 7, 9))])
+@pytest.mark.parametrize("sides", [(1, 2, 3, 4, 5, 6), (2, 5)])
+def test_row_assembly_tiles(ctx, p, n, sides):
+    P = problems.box_patch(3, p, n)
+    problems.perturb_interior(P, 0.1 / max(n), 9)
+    P.kappa = problems.lognormal_kappa(P.nelem, 0.5, 9)
+    P.fkind = 1
+    prob = problems.Problem([P], [(0, s) for s in sides], [])
+    gp = gsx.Problem(ctx, prob)
+    if gp.nfree == 0:
+        gp.close()
+        pytest.skip("no free functions")
+    gp.set_bc([(0, s, gsx.BC_DIRICHLET, gsx.BCF_AFFINE, (0.5, 1.0, -2.0, 0.25)) for s in sides])
+    out = []
+    for mode in (gsx.ASM_ROWWISE, gsx.ASM_ELEMENTWISE):
+        A, b = gp.assemble(gsx.PATTERN_FULL | mode, gsx.MIXED)
+        rp, ci, va = A.download()
+        x = ctx.array(gp.nfree).zero()
+        it, rel, ok = A.cg_solve(b, x, tol=1e-10, maxit=5000, precision=gsx.MIXED)   # on the stencils
+        assert ok
+        out.append((rp, ci, va, b.download()[:gp.nfree], gp.min_detj(), A.to_scipy(), x.download()))
+        for o in (x, A, b):
+            o.close()
+    r, e = out
+    assert np.array_equal(r[0], e[0]) and np.array_equal(r[1], e[1])
+    # the same products grouped differently: up to (p+1)^3 27 9 terms per entry
+    # at eps, judged against the row's largest entry
+    scale = np.maximum.reduceat(np.abs(e[2]), e[0][:-1])
+    assert np.all(np.abs(r[2] - e[2]) <= 1e-12 * np.repeat(scale, np.diff(e[0])))
+    assert np.abs(r[3] - e[3]).max() <= 1e-12 * np.abs(e[3]).max()
+    assert r[4] == pytest.approx(e[4], rel=1e-12)
+    assert (r[5] != r[5].T).nnz == 0   # bitwise symmetric
+    assert np.linalg.norm(r[3] - r[5] @ r[6]) <= 1.01e-10 * np.linalg.norm(r[3])
+    gp.close()
