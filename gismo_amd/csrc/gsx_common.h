@@ -31,6 +31,8 @@ struct PatchDev {
     int64_t kmat_off;       // element matrices: doubles offset of element 0
     int64_t fvec_off;       // element load vectors: doubles offset
     int64_t elem_off;       // global element id of element 0
+    int64_t b_off;          // basis functions of the patches before
+    int64_t r_off;          // raw rows (2D): doubles offset of function 0
 };
 
 // Gauss-Legendre nodes/weights for n = 1..kMaxQ1 points, ascending.

@@ -352,4 +352,21 @@ hipError_t launch_sell_residual_f32(const SellOp &S, const float *v, const float
 hipError_t launch_sell_spmv(const SellOp &S, const double *v, const double *x, double *y, double *partial,
                             const CGState *st, hipStream_t s);
 
+// Sum-factorised rows of 2D patches (gsx_sf2.hip); cy: rows iy per chunk, the
+// block prefix counts sf2_blocks per patch.  err |= 1 where a CSR row does not
+// hold the window's columns.
+bool sf2_supported(int p);
+int64_t sf2_raw_doubles(int p, int64_t nbasis);
+int64_t sf2_blocks(int p, const int *nb, int cy);
+hipError_t launch_sf2_rows(int p, const PatchDev *patches, const int *gpatch, const int64_t *bprefix, int ng,
+                           int64_t nblocks, int cy, const GaussTab &gt, double *raw, double *rawf, double *detmin,
+                           hipStream_t s);
+hipError_t launch_sf2_finish(int p, const SfBox &bx, int nfree, const int *rowptr, const double *raw,
+                             const double *rawf, double *s64, float *s32, double *val, double *rhs, const int *dofs,
+                             const double *fixed, int *err, hipStream_t s);
+hipError_t launch_sf2_gather(int p, const PatchDev *patches, const int *occ_ptr, const int *occ_patch,
+                             const int64_t *occ_local, int nfree, const int *rowptr, const int *col,
+                             const double *raw, const double *rawf, double *val, double *rhs, int maxrow,
+                             const double *fixed, int *err, hipStream_t s);
+
 }  // namespace gsx

@@ -250,6 +250,9 @@ struct Group {
     std::vector<int64_t> nprefix;   // blocks of the error norm kernel per patch
     int64_t nelem = 0;
     DevPtr d_gpatch, d_gprefix, d_nprefix;
+    std::vector<int64_t> rprefix;   // blocks of the 2D row assembly per patch
+    int rows_cy = 16;               // and its rows per chunk
+    DevPtr d_rprefix;
 };
 
 struct gsx_problem {
@@ -281,7 +284,7 @@ struct gsx_problem {
     int box_lo[3] = {0, 0, 0}, box_hi[3] = {0, 0, 0};   // free functions per direction
     // element scratch
     DevPtr d_detmin, d_scan_bsum, d_scan_total;
-    int64_t kdoubles = 0, fdoubles = 0;
+    int64_t kdoubles = 0, fdoubles = 0, rdoubles = 0;
     double min_det = 0.0;
     // boundary data: values of the eliminated DOFs (global index - nfree;
     // null: homogeneous) and the Neumann load over the free DOFs (null: none)
@@ -291,6 +294,7 @@ struct gsx_problem {
     DevPtr kept_K;
     uint64_t asm_serial = 0, kept_serial = 0;
     bool zero_kappa = false;        // some element has kappa exactly 0
+    bool odd_glue = false;          // an interface joins a patch to itself or to one of another degree
     // geometry, kappa and source of another problem (a level of a
     // p-multigrid hierarchy): this problem's patches give only the basis
     gsx_problem *geo = nullptr;
@@ -700,7 +704,7 @@ gsx_status gsx_problem_create(gsx_ctx *c, int32_t npatch, const gsx_patch_desc *
     HIP_OK(c, hipMemcpyAsync(P->d_dofs.get(), P->dofs.data(), sizeof(int) * P->nbasis,
                              hipMemcpyHostToDevice, s));
     eoff = 0;
-    int64_t kdoubles = 0, fdoubles = 0;
+    int64_t kdoubles = 0, fdoubles = 0, rdoubles = 0;
     for (int k = 0; k < npatch; ++k) {
         const gsx_patch_desc &D = patches[k];
         const HostPatch &h = P->hp[k];
@@ -767,6 +771,9 @@ gsx_status gsx_problem_create(gsx_ctx *c, int32_t npatch, const gsx_patch_desc *
         pd.dofs = dp<int>(P->d_dofs) + P->boff[k];
         pd.nelem = h.nelem;
         pd.elem_off = eoff;
+        pd.b_off = P->boff[k];
+        pd.r_off = rdoubles;
+        if (h.d == 2 && gsx::sf2_supported(h.p[0])) rdoubles += gsx::sf2_raw_doubles(h.p[0], h.nbasis);
         int nb1 = h.p[0] + 1;
         int NB = (h.d == 2) ? nb1 * nb1 : nb1 * nb1 * nb1;
         pd.kmat_off = kdoubles;
@@ -778,6 +785,7 @@ gsx_status gsx_problem_create(gsx_ctx *c, int32_t npatch, const gsx_patch_desc *
     }
     P->kdoubles = kdoubles;
     P->fdoubles = fdoubles;
+    P->rdoubles = rdoubles;
     P->d_patches = dalloc(c, sizeof(PatchDev) * npatch);
     if (!P->d_patches) return fail(c, GSX_ERR_OOM, "device allocation (patches)");
     HIP_OK(c, hipMemcpyAsync(P->d_patches.get(), P->pdev.data(), sizeof(PatchDev) * npatch,
@@ -797,7 +805,24 @@ gsx_status gsx_problem_create(gsx_ctx *c, int32_t npatch, const gsx_patch_desc *
         }
         g->patches.push_back(k);
     }
+    for (int f = 0; f < nif; ++f) {
+        const int p1 = ifaces[8 * f], p2 = ifaces[8 * f + 2];
+        P->odd_glue = P->odd_glue || p1 == p2 || P->hp[p1].p[0] != P->hp[p2].p[0];
+    }
     for (auto &g : P->groups) {
+        if (g.d == 2 && gsx::sf2_supported(g.p)) {
+            // shorter chunks (p elements more each) until the blocks fill the CUs
+            for (g.rows_cy = 16;; g.rows_cy /= 2) {
+                g.rprefix.assign(1, 0);
+                for (int k : g.patches)
+                    g.rprefix.push_back(g.rprefix.back() + gsx::sf2_blocks(g.p, P->hp[k].nb, g.rows_cy));
+                if (g.rows_cy <= 2 || g.rprefix.back() >= 512) break;
+            }
+            g.d_rprefix = dalloc(c, sizeof(int64_t) * g.rprefix.size());
+            if (!g.d_rprefix) return fail(c, GSX_ERR_OOM, "device allocation (groups)");
+            HIP_OK(c, hipMemcpyAsync(g.d_rprefix.get(), g.rprefix.data(), sizeof(int64_t) * g.rprefix.size(),
+                                     hipMemcpyHostToDevice, s));
+        }
         g.prefix.assign(1, 0);
         g.nprefix.assign(1, 0);
         for (int k : g.patches) {
@@ -1089,7 +1114,8 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
     const bool csr_only = (mode & GSX_ASM_CSR_ONLY) != 0;
     const bool keep_elements = (mode & GSX_ASM_KEEP_ELEMENTS) != 0;
     const bool rowwise_forced = (mode & GSX_ASM_ROWWISE) != 0;
-    bool elementwise = (mode & GSX_ASM_ELEMENTWISE) != 0;
+    const bool elementwise_asked = (mode & GSX_ASM_ELEMENTWISE) != 0;
+    bool elementwise = elementwise_asked;
     mode &= ~(GSX_ASM_REBUILD_PATTERN | GSX_ASM_CSR_ONLY | GSX_ASM_KEEP_ELEMENTS | GSX_ASM_ELEMENTWISE |
               GSX_ASM_ROWWISE);
     P->kept_K.reset();
@@ -1115,6 +1141,11 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
         elementwise = true;
         if (P->geo->npatch != P->npatch) return fail(c, GSX_ERR_ARG, "geometry problem changed");
     }
+    // 2D patches of degrees 2 to 4: sum-factorised rows likewise (a row of a
+    // patch glued to itself could meet a column twice in its window)
+    bool use_sf2 = P->d == 2 && P->nfree > 0 && !(elementwise_asked || P->geo) && !keep_elements &&
+                   !P->zero_kappa && !P->odd_glue;
+    for (const Group &g : P->groups) use_sf2 = use_sf2 && gsx::sf2_supported(g.p);
     const bool use_sf = single && !elementwise && !keep_elements && !P->zero_kappa && P->hp[0].d == 3 &&
                         P->hp[0].p[0] == P->hp[0].p[1] && P->hp[0].p[0] == P->hp[0].p[2] &&
                         gsx::sf_supported(3, P->hp[0].p[0]);
@@ -1143,16 +1174,32 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
         return fail(c, GSX_ERR_BUDGET, "element matrices of a multipatch assembly exceed the element budget "
                                        "(gsx_ctx_set_elem_budget)");
     }
-    const int64_t kcap = use_sf ? 0
+    const int64_t kcap = use_sf || use_sf2 ? 0
                          : single ? std::min<int64_t>(h0.nel[sd], slab_rows + h0.p[0]) * layer_elems * nb0 * nb0
                                   : P->kdoubles;
     const int64_t fcap = use_sf ? gsx::sf_load_doubles(h0.p[0], h0.nel)   // z sums of the load
+                         : use_sf2 ? P->nbasis                            // loads of the raw rows
                          : single ? std::min<int64_t>(h0.nel[sd], slab_rows + h0.p[0]) * layer_elems * nb0
                                   : P->fdoubles;
     DevPtr Kbuf = dalloc(c, sizeof(double) * std::max<int64_t>(1, kcap));
     DevPtr Fbuf = dalloc(c, sizeof(double) * std::max<int64_t>(1, fcap));
     if (!Kbuf || !Fbuf) return fail(c, GSX_ERR_OOM, "device allocation (element matrices)");
-    if (!single && P->geo) {
+    DevPtr raw2, err2;   // 2D row assembly
+    int64_t ndet2 = 0;   // and its determinant minima, one per block
+    if (use_sf2) {
+        raw2 = dalloc(c, sizeof(double) * P->rdoubles);
+        err2 = dalloc(c, sizeof(int));
+        if (!raw2 || !err2) return fail(c, GSX_ERR_OOM, "device allocation (row assembly)");
+        KScope k(c, "sf_assemble");
+        HIP_OK(c, hipMemsetAsync(err2.get(), 0, sizeof(int), s));
+        for (const Group &g : P->groups) {
+            HIP_OK(c, gsx::launch_sf2_rows(g.p, dp<PatchDev>(P->d_patches), dp<int>(g.d_gpatch),
+                                           dp<int64_t>(g.d_rprefix), (int)g.patches.size(), g.rprefix.back(),
+                                           g.rows_cy, c->gt, dp<double>(raw2), dp<double>(Fbuf),
+                                           dp<double>(P->d_detmin) + ndet2, s));
+            ndet2 += g.rprefix.back();
+        }
+    } else if (!single && P->geo) {
         KScope k(c, "geo_elem");
         for (int ip = 0; ip < P->npatch; ++ip)
             HIP_OK(c, gsx::launch_geo_elem(P->d, dp<PatchDev>(P->d_patches), dp<PatchDev>(P->geo->d_patches), ip, 0,
@@ -1181,8 +1228,9 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
         rhs = dp<double>(rhs_tmp);
     }
     DevPtr keep;
-    if (mode == GSX_PATTERN_EXPR && !use_sf) keep = dalloc(c, std::max<int64_t>(1, P->nnz));
-    if (!A->val || !rhs || (mode == GSX_PATTERN_EXPR && !use_sf && !keep))
+    const bool rows = use_sf || use_sf2;   // no exact-zero flags
+    if (mode == GSX_PATTERN_EXPR && !rows) keep = dalloc(c, std::max<int64_t>(1, P->nnz));
+    if (!A->val || !rhs || (mode == GSX_PATTERN_EXPR && !rows && !keep))
         return fail(c, GSX_ERR_OOM, "device allocation (values)");
     if (single) {
         // structured operator filled by the same gather (unless CSR only)
@@ -1208,8 +1256,8 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
         }
         S.s64_ready = !csr_only;
         S.s32_ready = !csr_only && precision == GSX_MIXED;
-        if (use_sf) {
-            gsx::SfBox sb;
+        gsx::SfBox sb;
+        if (rows) {
             const int p = h.p[0];
             for (int k = 0; k < 3; ++k) {
                 sb.nb[k] = h.nb[k];
@@ -1219,6 +1267,16 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
                 sb.m[k] = P->box_hi[k] - P->box_lo[k] + 1;
                 sb.g[k] = h.nel[k] * (p + 1);
             }
+        }
+        if (use_sf2) {
+            KScope k(c, "sf_finish");
+            HIP_OK(c, gsx::launch_sf2_finish(h.p[0], sb, P->nfree, dp<int>(P->d_rowptr), dp<double>(raw2),
+                                             dp<double>(Fbuf), dp<double>(S.s64), dp<float>(S.s32), dp<double>(A->val),
+                                             rhs, dp<int>(P->d_dofs), P->d_fixed ? dp<double>(P->d_fixed) : nullptr,
+                                             dp<int>(err2), s));
+        }
+        if (use_sf) {
+            const int p = h.p[0];
             sb.toff[0] = 0;
             sb.toff[1] = (int64_t)sb.g[0] * (2 * (p + 1) + 1);
             sb.toff[2] = sb.toff[1] + (int64_t)sb.g[1] * (2 * (p + 1) + 1);
@@ -1253,7 +1311,7 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
         int64_t plane = 1;
         for (int k = 0; k < sd; ++k) plane *= P->box_hi[k] - P->box_lo[k] + 1;
         const Group &g = P->groups[0];
-        for (int L0 = P->box_lo[sd]; !use_sf && L0 <= P->box_hi[sd]; L0 += slab_rows) {
+        for (int L0 = P->box_lo[sd]; !rows && L0 <= P->box_hi[sd]; L0 += slab_rows) {
             const int L1 = std::min(L0 + slab_rows, P->box_hi[sd] + 1);
             const int64_t E0 = std::max(0, L0 - h.p[0]), E1 = std::min(h.nel[sd], L1);
             if (P->geo) {
@@ -1281,6 +1339,14 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
                                                S.s32 ? dp<float>(S.s32) : nullptr, dp<int>(P->d_dofs),
                                                P->d_fixed ? dp<double>(P->d_fixed) : nullptr, s));
         }
+    } else if (use_sf2) {
+        KScope k(c, "gather");
+        for (const Group &g : P->groups)
+            HIP_OK(c, gsx::launch_sf2_gather(g.p, dp<PatchDev>(P->d_patches), dp<int>(P->d_occ_ptr),
+                                             dp<int>(P->d_occ_patch), dp<int64_t>(P->d_occ_local), P->nfree,
+                                             dp<int>(P->d_rowptr), dp<int>(P->d_col), dp<double>(raw2),
+                                             dp<double>(Fbuf), dp<double>(A->val), rhs, P->maxrow,
+                                             P->d_fixed ? dp<double>(P->d_fixed) : nullptr, dp<int>(err2), s));
     } else {
         KScope k(c, "gather");
         HIP_OK(c, gsx::launch_gather(dp<PatchDev>(P->d_patches), dp<int>(P->d_occ_ptr),
@@ -1300,8 +1366,13 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
     Fbuf.reset();
     double *dmin_slot = dp<double>(P->d_detmin) + std::max<int64_t>(1, P->nelem);
     HIP_OK(c, gsx::launch_min(dp<double>(P->d_detmin),
-                              use_sf ? gsx::sf_det_count(h0.p[0], h0.nel) : P->nelem, dmin_slot, s));
+                              use_sf    ? gsx::sf_det_count(h0.p[0], h0.nel)
+                              : use_sf2 ? ndet2
+                                        : P->nelem,
+                              dmin_slot, s));
     double mind = 0.0;
+    int errh2 = 0;
+    if (use_sf2) HIP_OK(c, hipMemcpyAsync(&errh2, err2.get(), sizeof(int), hipMemcpyDeviceToHost, s));
     HIP_OK(c, hipMemcpyAsync(&mind, dmin_slot, sizeof(double), hipMemcpyDeviceToHost, s));
     if (mode == GSX_PATTERN_EXPR && keep) {
         DevPtr dropped = dalloc(c, sizeof(unsigned long long));
@@ -1334,6 +1405,7 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
         }
     }
     HIP_OK(c, hipStreamSynchronize(s));
+    if (errh2) return fail(c, GSX_ERR_ARG, "row assembly: CSR row does not match the stencil window");
     P->min_det = mind;
     if (!(mind > 0.0)) {
         char buf[128];

@@ -235,3 +235,45 @@ def test_row_assembly_tiles(ctx, p, n, sides):
     assert (r[5] != r[5].T).nnz == 0   # bitwise symmetric
     assert np.linalg.norm(r[3] - r[5] @ r[6]) <= 1.01e-10 * np.linalg.norm(r[3])
     gp.close()
+
+
+# the 2D row assembly: blocks of 83 / 61 / 47 rows along x, chunks of 2 to 16
+# rows along y, x-line segments of 32 rows, thin patches, glued patches with
+# interface and corner rows, eliminated columns moved to the right-hand side
+@pytest.mark.parametrize("p,n,gx,gy", [(2, (1, 1), 1, 1), (2, (82, 3), 1, 1), (2, (84, 17), 1, 1), (3, (59, 2), 1, 1),
+                                       (3, (1, 40), 1, 1), (4, (44, 5), 1, 1), (4, (48, 1), 1, 1), (2, 9, 2, 2),
+                                       (3, 63, 2, 1), (3, 5, 3, 3), (4, 7, 1, 2), (2, 90, 4, 4)])
+def test_row_assembly_2d(ctx, p, n, gx, gy):
+    if gx * gy == 1:
+        P = problems.box_patch(2, p, n)
+        P.kappa = problems.lognormal_kappa(P.nelem, 0.5, 9)
+        prob = problems.Problem([P], problems.all_sides(2)[1:], [])
+    else:
+        prob = problems.square_grid(gx, gy, n, p)
+    for k, P in enumerate(prob.patches):
+        problems.perturb_interior(P, 0.1 / np.max(n), 40 + k)
+        P.fkind = 1
+    gp = gsx.Problem(ctx, prob)
+    assert gp.nfree > 0
+    gp.set_bc([(k, s, gsx.BC_DIRICHLET, gsx.BCF_AFFINE, (0.5, 1.0, -2.0, 0.25)) for k, s in prob.dir_sides])
+    out = []
+    for mode in (0, gsx.ASM_ELEMENTWISE):
+        A, b = gp.assemble(gsx.PATTERN_FULL | mode, gsx.MIXED)
+        rp, ci, va = A.download()
+        x = ctx.array(gp.nfree).zero()
+        it, rel, ok = A.cg_solve(b, x, tol=1e-10, maxit=20000, precision=gsx.MIXED)
+        assert ok
+        out.append((rp, ci, va, b.download()[:gp.nfree], gp.min_detj(), A.to_scipy(), x.download()))
+        for o in (x, A, b):
+            o.close()
+    r, e = out
+    assert np.array_equal(r[0], e[0]) and np.array_equal(r[1], e[1])
+    # the same products grouped differently: up to (p+1)^2 16 4 terms per entry
+    # at eps, judged against the row's largest entry (coordinates up to 4)
+    scale = np.maximum.reduceat(np.abs(e[2]), e[0][:-1])
+    assert np.all(np.abs(r[2] - e[2]) <= 1e-12 * np.repeat(scale, np.diff(e[0])))
+    assert np.abs(r[3] - e[3]).max() <= 1e-12 * np.abs(e[3]).max()
+    assert r[4] == pytest.approx(e[4], rel=1e-12)
+    assert (r[5] != r[5].T).nnz == 0   # bitwise symmetric
+    assert np.linalg.norm(r[3] - r[5] @ r[6]) <= 1.01e-10 * np.linalg.norm(r[3])
+    gp.close()
