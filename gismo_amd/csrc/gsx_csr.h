@@ -7,9 +7,11 @@
 // form the products with the gathered input and put them into the wave's LDS
 // buffer; then L lanes per row sum the row's part of the buffer.  Bound by the
 // matrix bytes.  Waves work without block barriers, several loads in flight
-// each.  The other way, L lanes reading their row directly, keeps two loads per
+// each.  The other way (DIRECT), L lanes reading their row, keeps two loads per
 // lane in flight at 49 entries per row, idles a quarter of the lanes in the
-// last one and spends five shuffles per row.
+// last one and spends five shuffles per row, but it is the shorter chain and
+// needs no buffer: it is taken where all rows are on the chip at once, and for
+// rows longer than the buffer serves well (csr_direct).
 // 1.06 M rows of 49 entries (16 patches of 256^2 elements, p = 3): FP64 SpMV
 // 157 us (4.0 TB/s of matrix bytes; direct rows 249 us), damped Jacobi step on
 // FP32 values with FP64 vectors 142 us (225 us).  69 K rows: 11.7 us (14.9 us).
@@ -22,14 +24,30 @@ namespace gsx {
 constexpr int kCsrCap = 512;         // products a wave buffers
 constexpr int kCsrMaxBlocks = 2048;  // blocks of 4 waves; more rows: more groups per wave
 
-// lanes summing one row, from the class of the mean row length (spmv_lpr)
+// lpr: the class of the mean row length (spmv_lpr), kCsrLong for the longest.
+// A wave's buffer sums a row with lpr / 4 lanes, direct rows take lpr (64 for
+// long ones).
+constexpr int kCsrLong = 128;
+
+// Direct rows where a lane per lpr entries' worth of rows fits the chip (256
+// CUs x 2048 lanes), or for long rows.  Direct / buffered, FP64 SpMV: 36 rows
+// 3.3 / 4.2 us, 4096 rows of 25 3.4 / 4.2, 14 K rows of 81 5.8 / 6.4, 8 K rows
+// of 125 4.6 / 4.3 (512 K lanes); beyond the line 66 K rows of 25 7.6 / 6.2.
+// Long rows: 39 K rows of 729 69 / 81 us, 16 K of 280 12.6 / 13.2; 262 K of 330
+// 262 / 258.
+__host__ __device__ inline bool csr_direct(int n, int lpr)
+{
+    return lpr == kCsrLong || (int64_t)n * lpr <= 256 * 2048;
+}
+
 constexpr int csr_lanes(int lpr) { return lpr / 4; }
 
-__host__ __device__ inline int csr_blocks(int n, int lanes)
+__host__ __device__ inline int csr_blocks(int n, int lpr)
 {
-    const int rows = 4 * (64 / lanes);
+    const bool direct = csr_direct(n, lpr);
+    const int rows = direct ? 256 / (lpr > 64 ? 64 : lpr) : 4 * (64 / csr_lanes(lpr));
     const int nb = (n + rows - 1) / rows;
-    return nb < 1 ? 1 : (nb > kCsrMaxBlocks ? kCsrMaxBlocks : nb);
+    return nb < 1 ? 1 : (nb > kCsrMaxBlocks && !direct ? kCsrMaxBlocks : nb);
 }
 
 template <typename V> struct CsrPair;
@@ -38,11 +56,23 @@ template <> struct CsrPair<float> { using type = float2; };
 
 // epi(r, sum, pre(r)) once per row, in the row's first lane (pre's loads are
 // issued with the row's entries); buf: kCsrCap entries of the calling wave.
-// All blocks of 256 threads of the grid take part.
-template <int L, typename Acc, typename V, typename T, typename Pre, typename Epi>
+// All blocks of 256 threads of the grid take part (csr_blocks).
+template <int L, bool DIRECT, typename Acc, typename V, typename T, typename Pre, typename Epi>
 __device__ inline void csr_rows(int n, const int *__restrict__ rowptr, const int *__restrict__ col,
                                 const V *__restrict__ val, const T *__restrict__ x, Acc *buf, Pre pre, Epi epi)
 {
+    if constexpr (DIRECT) {
+        const int r = blockIdx.x * (256 / L) + threadIdx.x / L;
+        Acc acc = 0;
+        if (r < n) {
+            const int k1 = rowptr[r + 1];
+            for (int k = rowptr[r] + threadIdx.x % L; k < k1; k += L) acc += (Acc)val[k] * (Acc)x[col[k]];
+        }
+#pragma unroll
+        for (int off = L / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+        if (r < n && threadIdx.x % L == 0) epi(r, acc, pre(r));
+        return;
+    }
     constexpr int RW = 64 / L, NU = kCsrCap / 128;
     using V2 = typename CsrPair<V>::type;
     const int lane = threadIdx.x & 63;

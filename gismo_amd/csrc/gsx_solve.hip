@@ -35,7 +35,7 @@ __device__ inline double block_sum256(double v, double *s)
 //   MODE 2: y = b - A x and partial[block] = sum_rows y_i^2
 // Skipped entirely when state->done != 0 (state may be null).
 // ---------------------------------------------------------------------------
-template <int L, typename V, typename T, int MODE>
+template <int L, bool DIRECT, typename V, typename T, int MODE>
 __global__ __launch_bounds__(256) void k_spmv(int n, const int *__restrict__ rowptr,
                                               const int *__restrict__ col,
                                               const V *__restrict__ val, const T *__restrict__ x,
@@ -43,11 +43,11 @@ __global__ __launch_bounds__(256) void k_spmv(int n, const int *__restrict__ row
                                               double *__restrict__ partial,
                                               const CGState *__restrict__ state)
 {
-    __shared__ T buf[4][kCsrCap];
+    __shared__ T buf[4][DIRECT ? 1 : kCsrCap];
     __shared__ double s[4];
     if (state && (state->done || state->frozen)) return;
     double contrib = 0.0;
-    csr_rows<L, T>(
+    csr_rows<L, DIRECT, T>(
         n, rowptr, col, val, x, buf[threadIdx.x >> 6],
         [&](int r) -> T { return MODE == 2 ? b[r] : (MODE == 1 ? x[r] : (T)0); },
         [&](int r, T acc, T pv) {
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256) void k_cg_restart(int n, const double *__restr
 
 // Damped Jacobi smoothing step x += tau (b - A x) / diag, fused with the
 // SpMV (gsJacobiOp::step).  Reads x_in, writes x_out (x_in != x_out).
-template <int L, typename V, typename T>
+template <int L, bool DIRECT, typename V, typename T>
 __global__ __launch_bounds__(256) void k_jacobi_step(int n, const int *__restrict__ rowptr,
                                                      const int *__restrict__ col,
                                                      const V *__restrict__ val,
@@ -227,9 +227,9 @@ __global__ __launch_bounds__(256) void k_jacobi_step(int n, const int *__restric
     // products and sums in FP64 whatever the storage type: an FP32 row sum
     // of a stiffness row cancels to a relative error of eps * cond(A), which
     // costs a multigrid preconditioner outer iterations
-    __shared__ double buf[4][kCsrCap];
+    __shared__ double buf[4][DIRECT ? 1 : kCsrCap];
     struct Row { T x, b, d; };
-    csr_rows<L, double>(
+    csr_rows<L, DIRECT, double>(
         n, rowptr, col, val, xin, buf[threadIdx.x >> 6], [&](int r) { return Row{xin[r], b[r], diag[r]}; },
         [&](int r, double acc, const Row &q) {
             xout[r] = (T)((double)q.x + (double)tau * ((double)q.b - acc) / (double)q.d);
@@ -246,13 +246,13 @@ __global__ __launch_bounds__(256) void k_jacobi_first(int n, const T *__restrict
 }
 
 // r = b - A x, FP64 sums whatever the storage type (see k_jacobi_step)
-template <int L, typename V, typename T>
+template <int L, bool DIRECT, typename V, typename T>
 __global__ __launch_bounds__(256) void k_residual(int n, const int *__restrict__ rowptr, const int *__restrict__ col,
                                                   const V *__restrict__ val, const T *__restrict__ x,
                                                   const T *__restrict__ b, T *__restrict__ r)
 {
-    __shared__ double buf[4][kCsrCap];
-    csr_rows<L, double>(
+    __shared__ double buf[4][DIRECT ? 1 : kCsrCap];
+    csr_rows<L, DIRECT, double>(
         n, rowptr, col, val, x, buf[threadIdx.x >> 6], [&](int i) -> T { return b[i]; },
         [&](int i, double acc, T bi) { r[i] = (T)((double)bi - acc); });
 }
@@ -426,13 +426,14 @@ __global__ __launch_bounds__(256) void k_cg_reliable(const double *__restrict__ 
 // ---------------------------------------------------------------------------
 int spmv_lpr(double avg_row)
 {
+    if (avg_row > 240) return kCsrLong;
     if (avg_row > 96) return 64;
     if (avg_row > 40) return 32;
     if (avg_row > 16) return 16;
     return 8;
 }
 
-int spmv_blocks(int n, int lpr) { return csr_blocks(n, csr_lanes(lpr)); }
+int spmv_blocks(int n, int lpr) { return csr_blocks(n, lpr); }
 
 template <typename V, typename T, int MODE>
 static hipError_t spmv_dispatch(int lpr, int n, const int *rowptr, const int *col, const V *val,
@@ -441,13 +442,18 @@ static hipError_t spmv_dispatch(int lpr, int n, const int *rowptr, const int *co
 {
     if (n <= 0) return hipSuccess;
     const dim3 grid(spmv_blocks(n, lpr)), block(256);
-    switch (csr_lanes(lpr)) {
-    case 16: hipLaunchKernelGGL((k_spmv<16, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st); break;
-    case 8: hipLaunchKernelGGL((k_spmv<8, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st); break;
-    case 4: hipLaunchKernelGGL((k_spmv<4, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st); break;
-    case 2: hipLaunchKernelGGL((k_spmv<2, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st); break;
+#define GSX_L(LPR)                                                                                                    \
+    case LPR:                                                                                                         \
+        if (csr_direct(n, lpr))                                                                                       \
+            hipLaunchKernelGGL((k_spmv<LPR, true, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st);  \
+        else                                                                                                          \
+            hipLaunchKernelGGL((k_spmv<LPR / 4, false, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st); \
+        break;
+    switch (lpr == kCsrLong ? 64 : lpr) {
+        GSX_L(8) GSX_L(16) GSX_L(32) GSX_L(64)
     default: return hipErrorInvalidValue;
     }
+#undef GSX_L
     return hipGetLastError();
 }
 
@@ -557,13 +563,18 @@ static hipError_t jacobi_dispatch(int lpr, int n, const int *rp, const int *ci, 
         return hipGetLastError();
     }
     const dim3 grid(spmv_blocks(n, lpr)), block(256);
-    switch (csr_lanes(lpr)) {
-    case 16: hipLaunchKernelGGL((k_jacobi_step<16, V, T>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau); break;
-    case 8: hipLaunchKernelGGL((k_jacobi_step<8, V, T>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau); break;
-    case 4: hipLaunchKernelGGL((k_jacobi_step<4, V, T>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau); break;
-    case 2: hipLaunchKernelGGL((k_jacobi_step<2, V, T>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau); break;
+#define GSX_L(LPR)                                                                                                    \
+    case LPR:                                                                                                         \
+        if (csr_direct(n, lpr))                                                                                       \
+            hipLaunchKernelGGL((k_jacobi_step<LPR, true, V, T>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau);  \
+        else                                                                                                          \
+            hipLaunchKernelGGL((k_jacobi_step<LPR / 4, false, V, T>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau); \
+        break;
+    switch (lpr == kCsrLong ? 64 : lpr) {
+        GSX_L(8) GSX_L(16) GSX_L(32) GSX_L(64)
     default: return hipErrorInvalidValue;
     }
+#undef GSX_L
     return hipGetLastError();
 }
 
@@ -594,13 +605,18 @@ static hipError_t residual_dispatch(int lpr, int n, const int *rp, const int *ci
 {
     if (n <= 0) return hipSuccess;
     const dim3 grid(spmv_blocks(n, lpr)), block(256);
-    switch (csr_lanes(lpr)) {
-    case 16: hipLaunchKernelGGL((k_residual<16, V, T>), grid, block, 0, s, n, rp, ci, v, x, b, r); break;
-    case 8: hipLaunchKernelGGL((k_residual<8, V, T>), grid, block, 0, s, n, rp, ci, v, x, b, r); break;
-    case 4: hipLaunchKernelGGL((k_residual<4, V, T>), grid, block, 0, s, n, rp, ci, v, x, b, r); break;
-    case 2: hipLaunchKernelGGL((k_residual<2, V, T>), grid, block, 0, s, n, rp, ci, v, x, b, r); break;
+#define GSX_L(LPR)                                                                                                    \
+    case LPR:                                                                                                         \
+        if (csr_direct(n, lpr))                                                                                       \
+            hipLaunchKernelGGL((k_residual<LPR, true, V, T>), grid, block, 0, s, n, rp, ci, v, x, b, r);  \
+        else                                                                                                          \
+            hipLaunchKernelGGL((k_residual<LPR / 4, false, V, T>), grid, block, 0, s, n, rp, ci, v, x, b, r); \
+        break;
+    switch (lpr == kCsrLong ? 64 : lpr) {
+        GSX_L(8) GSX_L(16) GSX_L(32) GSX_L(64)
     default: return hipErrorInvalidValue;
     }
+#undef GSX_L
     return hipGetLastError();
 }
 

@@ -162,8 +162,8 @@ __global__ void k_gather_from_grid(int nfree, const int *__restrict__ free2grid,
 // before); FP64 residual 109 us (159 us reading all slots).  75^3 p = 2, FP64:
 // 54.5 us with the direction (89 + 7 us reading all slots).
 // ---------------------------------------------------------------------------
-template <int D, int P, typename V, typename T, int KIND, int MODE, bool STAGED>
-__global__ __launch_bounds__(256) void k_cg2_spmv(int nfree, const int *__restrict__ free2grid, int sy, int sz,
+template <int D, int P, typename V, typename T, int KIND, int MODE, bool STAGED, int Q>
+__global__ __launch_bounds__(256 * Q) void k_cg2_spmv(int nfree, const int *__restrict__ free2grid, int sy, int sz,
                                                   int m0, int m1, const V *__restrict__ sval,
                                                   const T *__restrict__ x, const T *__restrict__ po,
                                                   T *__restrict__ pn, T *__restrict__ y, const T *__restrict__ b,
@@ -171,7 +171,10 @@ __global__ __launch_bounds__(256) void k_cg2_spmv(int nfree, const int *__restri
                                                   CGState *__restrict__ st, int wn)
 {
     extern __shared__ double sp_smem[];
-    __shared__ double s[8];
+    __shared__ double s[8 * Q];
+    __shared__ T sq[Q > 1 ? Q - 1 : 1][256];
+    constexpr int NT = 256 * Q;
+    const int t = threadIdx.x & 255, q = Q > 1 ? threadIdx.x >> 8 : 0;   // row, group
     constexpr int W = 2 * P + 1;
     constexpr int NS = (D == 3) ? W * W * W : W * W;
     constexpr int C = NS / 2, SL = KIND == 0 ? stencil_half(NS) : NS;   // slots of the stored layout
@@ -181,15 +184,15 @@ __global__ __launch_bounds__(256) void k_cg2_spmv(int nfree, const int *__restri
     const int halo = P * sy + P;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     // the first tile's window is requested before the sums that give beta
-    constexpr int NPRE = MODE == 1 && STAGED ? 4 : 1;
-    T prx[NPRE], prp[NPRE];
+    constexpr int NPRE = MODE == 1 && STAGED ? (Q > 1 ? 1 : 4) : 0, NPA = NPRE ? NPRE : 1;
+    T prx[NPA], prp[NPA];
     int w0 = 0, w1 = 0;
     if (MODE == 1 && STAGED) {
         w0 = free2grid[blk * 256] - halo;
         w1 = free2grid[min(blk * 256 + 255, nfree - 1)] + halo + 1;
 #pragma unroll
         for (int u = 0; u < NPRE; ++u) {
-            const int i = w0 + (int)threadIdx.x + 256 * u;
+            const int i = w0 + (int)threadIdx.x + NT * u;
             prx[u] = i < w1 ? x[i] : (T)0;
             prp[u] = i < w1 ? po[i] : (T)0;
         }
@@ -197,11 +200,11 @@ __global__ __launch_bounds__(256) void k_cg2_spmv(int nfree, const int *__restri
     T tb = 0;
     if (MODE == 1) {
         double rr = 0.0, rzn = 0.0;
-        for (int i = threadIdx.x; i < cs.np; i += 256) {
+        for (int i = threadIdx.x; i < cs.np; i += NT) {
             rr += cs.part_rr[i];
             rzn += cs.part_rz[i];
         }
-        bsum2<256>(rr, rzn, s);
+        bsum2<NT>(rr, rzn, s);
         const double err = sqrt(rr) / st->bnorm;
         // restart > 0: the residual has just been formed and tested in FP64
         const bool conv = !cs.restart && !cs.mixed && err < st->tol;
@@ -236,12 +239,12 @@ __global__ __launch_bounds__(256) void k_cg2_spmv(int nfree, const int *__restri
     T *sA = reinterpret_cast<T *>(sp_smem), *sB = sA + wn;
     double contrib = 0.0;
     for (int r0 = blk * 256; r0 < nfree; r0 += gridDim.x * 256) {
-        const int r = r0 + threadIdx.x;
+        const int r = r0 + t;
         const bool act = r < nfree;
         const int g = act ? free2grid[r] : 0;
         const int ia = r % m0, ib = (r / m0) % m1, ic = (D == 3) ? r / (m0 * m1) : 0;
         const V *vb = sval + stencil_index(UP, r, SL);   // from the centre slot up
-        const bool pre = NPRE > 1 && r0 == blk * 256;
+        const bool pre = NPRE > 0 && r0 == blk * 256;
         int c = 0;
         if (STAGED) {
             w0 = free2grid[r0] - halo;
@@ -255,10 +258,10 @@ __global__ __launch_bounds__(256) void k_cg2_spmv(int nfree, const int *__restri
                 int i = w0 + threadIdx.x;
                 if (pre && dz == 0) {
 #pragma unroll
-                    for (int u = 0; u < NPRE; ++u, i += 256)
+                    for (int u = 0; u < NPRE; ++u, i += NT)
                         if (i < w1) sA[i - w0] = first ? prx[u] : prx[u] + tb * prp[u];
                 }
-                for (; i < w1; i += 256) {
+                for (; i < w1; i += NT) {
                     sA[i - w0] = input(i + dz * sz);
                     if (D == 3 && dz > 0) sB[i - w0] = input(i - dz * sz);
                 }
@@ -293,15 +296,17 @@ __global__ __launch_bounds__(256) void k_cg2_spmv(int nfree, const int *__restri
         if (act) {
             own = xa(0, 0);
             // centre line: own slots dx = 0..P, mirrors dx = -P..-1
+            if (q == 0) {
 #pragma unroll
-            for (int dx = 0; dx <= P; ++dx) acc += (T)vb[dx * kStencilTile] * xa(0, dx);
+                for (int dx = 0; dx <= P; ++dx) acc += (T)vb[dx * kStencilTile] * xa(0, dx);
 #pragma unroll
-            for (int dx = -P; dx < 0; ++dx) {
-                if (KIND == 2) acc += (T)vb[dx * kStencilTile] * xa(0, dx);
-                else acc += (T)(ia + dx >= 0 ? sval[stencil_index(UP - dx, r + dx, SL)] : (V)0) * xa(0, dx);
+                for (int dx = -P; dx < 0; ++dx) {
+                    if (KIND == 2) acc += (T)vb[dx * kStencilTile] * xa(0, dx);
+                    else acc += (T)(ia + dx >= 0 ? sval[stencil_index(UP - dx, r + dx, SL)] : (V)0) * xa(0, dx);
+                }
             }
 #pragma unroll 1
-            for (int dy = 1; dy <= P; ++dy) line(0, dy);
+            for (int dy = Q > 1 && q == 0 ? Q : (Q > 1 ? q : 1); dy <= P; dy += Q) line(0, dy);
         }
         if (D == 3) {
 #pragma unroll 1
@@ -309,11 +314,18 @@ __global__ __launch_bounds__(256) void k_cg2_spmv(int nfree, const int *__restri
                 plane(dz);
                 if (act) {
 #pragma unroll 1
-                    for (int dy = -P; dy <= P; ++dy) line(dz, dy);
+                    for (int dy = -P + (q + dz) % Q; dy <= P; dy += Q) line(dz, dy);
                 }
             }
         }
-        if (act) {
+        if (Q > 1) {
+            if (q) sq[q - 1][t] = acc;
+            __syncthreads();
+            if (q == 0)
+#pragma unroll
+                for (int u = 0; u + 1 < Q; ++u) acc += sq[u][t];
+        }
+        if (act && q == 0) {
             if (MODE == 2) {
                 const T v = b[g] - acc;
                 y[g] = v;
@@ -325,7 +337,7 @@ __global__ __launch_bounds__(256) void k_cg2_spmv(int nfree, const int *__restri
             }
         }
     }
-    const double tot = bsum<256>(contrib, s);
+    const double tot = bsum<NT>(contrib, s);
     if (threadIdx.x == 0) partial[blockIdx.x] = tot;
 }
 
@@ -545,18 +557,34 @@ int sspmv_window(int p, int nfree, int m0, int m1, int sy, int sz)
 constexpr int64_t kMirrorBytes = (int64_t)24 << 20;
 constexpr size_t kWindowLds = 64 * 1024;
 
+// A 3D operator of at most a tile per CU leaves most of the chip idle: four
+// groups of 256 threads then share a tile's stencil lines and one sums the
+// parts.  CG solves, one group / four: 12^3 p = 4 mixed 25.5 / 16.3 ms, 32^3 p =
+// 4 mixed 30.1 / 18.0 and FP64 31.5 / 22.6, 30^3 p = 3 mixed 5.3 / 3.9, 40^3 p =
+// 2 mixed (250 tiles) 1.76 / 1.66; beyond the line 40^3 p = 3 FP64 (270 tiles)
+// 6.5 / 7.5, 60^3 p = 3 mixed 8.6 / 12.0.  2D stencils have too few lines: 64^2
+// p = 2 1.50 / 1.66 ms, 300^2 p = 4 mixed 8.4 / 10.4.
+constexpr int kSplit = 4, kSplitTiles = 256;
+
 template <int D, int P, typename V, typename T, int KIND, int MODE>
 static hipError_t sspmv_launch(const SpmvGrid &G, const V *sv, const T *x, const T *po, T *pn, T *y, const T *b,
                                double *part, const CGStep &cs, CGState *st, hipStream_t s)
 {
-    const dim3 grid(sspmv_blocks(G.nfree)), blk(256);
+    const dim3 grid(sspmv_blocks(G.nfree));
     const size_t lds = (size_t)G.window * (D == 3 ? 2 : 1) * sizeof(T);
-    if (lds <= kWindowLds)
-        hipLaunchKernelGGL((k_cg2_spmv<D, P, V, T, KIND, MODE, true>), grid, blk, lds, s, G.nfree, G.f2g, G.sy, G.sz,
-                           G.m0, G.m1, sv, x, po, pn, y, b, part, cs, st, G.window);
-    else
-        hipLaunchKernelGGL((k_cg2_spmv<D, P, V, T, KIND, MODE, false>), grid, blk, 0, s, G.nfree, G.f2g, G.sy, G.sz,
-                           G.m0, G.m1, sv, x, po, pn, y, b, part, cs, st, 0);
+    const bool staged = lds <= kWindowLds;
+#define GSX_Q(STAGED, Q)                                                                                              \
+    hipLaunchKernelGGL((k_cg2_spmv<D, P, V, T, KIND, MODE, STAGED, Q>), grid, dim3(256 * Q), STAGED ? lds : 0, s,     \
+                       G.nfree, G.f2g, G.sy, G.sz, G.m0, G.m1, sv, x, po, pn, y, b, part, cs, st, STAGED ? G.window : 0)
+    if (D == 3 && (int)grid.x <= kSplitTiles) {
+        constexpr int Q = D == 3 ? kSplit : 1;
+        if (staged) GSX_Q(true, Q);
+        else GSX_Q(false, Q);
+    } else {
+        if (staged) GSX_Q(true, 1);
+        else GSX_Q(false, 1);
+    }
+#undef GSX_Q
     return hipGetLastError();
 }
 

@@ -84,10 +84,12 @@ def test_fd_pcg_fp32_tiles(ctx, d, p, n):
 
 # the structured CG: row tiles of 256 with staged windows, all slots read below
 # 24 MB of operator and mirrored upper ones above, direct reads where a window
-# exceeds the LDS (the flat boxes), several tiles a block above 524,288 rows
+# exceeds the LDS (the flat boxes), several tiles a block above 524,288 rows,
+# four groups of threads a tile for 3D operators of up to 256 tiles
 @pytest.mark.parametrize("d,p,n", [(2, 1, (2, 2)), (2, 2, (16, 17)), (2, 4, (300, 9)), (2, 1, (740, 731)),
                                    (3, 1, (9, 8, 7)), (3, 2, (3, 3, 600)), (3, 3, (2, 2, 450)), (3, 3, (19, 18, 19)),
-                                   (3, 3, (21, 19, 20)), (3, 4, (13, 11, 12)), (3, 4, (2, 40, 3))])
+                                   (3, 3, (21, 19, 20)), (3, 4, (13, 11, 12)), (3, 4, (2, 40, 3)),
+                                   (3, 1, (42, 41, 43)), (3, 2, (42, 40, 41))])
 def test_structured_cg_tiles(ctx, d, p, n):
     """FP64 and mixed solves on the structured operator reach the CSR
     operator's solution in its iterations."""
@@ -126,7 +128,8 @@ def test_structured_cg_tiles(ctx, d, p, n):
 
 # CSR row sums: waves of 64 / L rows, entries in pairs, LDS chunks of 512
 @pytest.mark.parametrize("n,lo,hi", [(1, 1, 1), (3, 0, 2), (65, 1, 9), (513, 0, 40), (1000, 30, 60), (301, 90, 420),
-                                     (37, 700, 1300), (70000, 0, 12)])
+                                     (37, 700, 1300), (70000, 0, 12), (20000, 30, 60), (9000, 90, 300),
+                                     (1500, 450, 900)])
 def test_csr_products(ctx, n, lo, hi):
     """gsx_spmv on matrices with ragged, empty and long rows, and Jacobi
     sweeps of a multigrid hierarchy over them."""
