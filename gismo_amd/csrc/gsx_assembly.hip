@@ -16,6 +16,8 @@
 #include "gsx_kernels.h"
 #include "gsx_basis.h"
 
+#include <algorithm>
+
 namespace gsx {
 
 __device__ inline int find_patch(const int64_t *__restrict__ prefix, int np, int64_t e)
@@ -386,6 +388,7 @@ __global__ __launch_bounds__(256) void k_elem3d(const PatchDev *__restrict__ pat
 // ascending, as Eigen keeps them after makeCompressed().
 // ---------------------------------------------------------------------------
 constexpr int kMaxMultiCols = 768;
+constexpr int kMaxMulti2D = (2 * kMaxDeg + 1) * (2 * kMaxDeg + 1);   // a 2D window
 
 __device__ inline void local_coords(const PatchDev &pd, int64_t l, int *c)
 {
@@ -395,102 +398,172 @@ __device__ inline void local_coords(const PatchDev &pd, int64_t l, int *c)
     c[2] = (int)(r / pd.nb[1]);
 }
 
-template <bool WRITE>
-__device__ int row_columns(const PatchDev *__restrict__ patches, const int *__restrict__ occ_ptr,
-                           const int *__restrict__ occ_patch, const int64_t *__restrict__ occ_local,
-                           int nfree, int r, int *__restrict__ out)
+// the window of function l, per direction, and its size
+__device__ inline int row_window(const PatchDev &pd, int64_t loc, int *lo, int *wd)
 {
-    const int o0 = occ_ptr[r], o1 = occ_ptr[r + 1];
-    if (o1 - o0 == 1) {
-        const PatchDev &pd = patches[occ_patch[o0]];
-        int l[3];
-        local_coords(pd, occ_local[o0], l);
-        int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-        for (int k = 0; k < pd.d; ++k) {
-            lo[k] = max(0, l[k] - pd.p[k]);
-            hi[k] = min(pd.nb[k] - 1, l[k] + pd.p[k]);
-        }
-        int cnt = 0, last = -1;
-        bool sorted = true;
-        for (int z = lo[2]; z <= hi[2]; ++z)
-            for (int y = lo[1]; y <= hi[1]; ++y)
-                for (int x = lo[0]; x <= hi[0]; ++x) {
-                    const int64_t m = x + (int64_t)pd.nb[0] * (y + (int64_t)pd.nb[1] * z);
-                    const int g = pd.dofs[m];
-                    if (g < nfree) {
-                        if (WRITE) out[cnt] = g;
-                        if (g < last) sorted = false;
-                        last = g;
-                        ++cnt;
-                    }
-                }
-        if (WRITE && !sorted) {
-            for (int i = 1; i < cnt; ++i) {
-                const int v = out[i];
-                int j = i - 1;
-                while (j >= 0 && out[j] > v) { out[j + 1] = out[j]; --j; }
-                out[j + 1] = v;
-            }
-        }
-        return cnt;
+    int l[3];
+    local_coords(pd, loc, l);
+    int n = 1;
+    for (int k = 0; k < 3; ++k) {
+        lo[k] = k < pd.d ? max(0, l[k] - pd.p[k]) : 0;
+        wd[k] = k < pd.d ? min(pd.nb[k] - 1, l[k] + pd.p[k]) - lo[k] + 1 : 1;
+        n *= wd[k];
     }
-    int buf[kMaxMultiCols];
-    int cnt = 0;
-    for (int o = o0; o < o1; ++o) {
+    return n;
+}
+
+__device__ inline int window_dof(const PatchDev &pd, const int *lo, const int *wd, int s)
+{
+    const int x = lo[0] + s % wd[0], y = lo[1] + (s / wd[0]) % wd[1], z = lo[2] + s / (wd[0] * wd[1]);
+    return pd.dofs[x + (int64_t)pd.nb[0] * (y + (int64_t)pd.nb[1] * z)];
+}
+
+// Rows of one occurrence: G lanes per row, a lane per window function (16 in
+// 2D, where a row has 25 to 81 of them, 64 in 3D).  The free columns mostly
+// ascend along the window and go to their rank among the free lanes; a row
+// next to an interface (coupled functions are numbered last) ranks its columns
+// by counting.  WRITE = 0 counts them.  Bound by the chain of dependent loads
+// (occurrence, patch, functions).  295 K rows of 25 on 9 patches: count 39 us,
+// columns 51 us (a thread per row: 88 and 222 us).
+template <int WRITE, int G>
+__global__ __launch_bounds__(256) void k_row_single(const PatchDev *__restrict__ patches,
+                                                    const int *__restrict__ occ_ptr, const int *__restrict__ occ_patch,
+                                                    const int64_t *__restrict__ occ_local, int nfree, int n,
+                                                    int *__restrict__ counts,
+                                                    const int *__restrict__ rowptr, int *__restrict__ col)
+{
+    constexpr int RB = 256 / G;
+    __shared__ int sG[RB][WRITE ? (G == 64 ? kMaxMultiCols : kMaxMulti2D) : 1];
+    const int w = threadIdx.x / G, lane = threadIdx.x % G, shift = threadIdx.x % kWave - lane;
+    const int r = blockIdx.x * RB + w;
+    const bool act = r < n;   // inactive groups of a wave stay for its ballots
+    const int o = act ? occ_ptr[r] : 0;
+    const PatchDev &pd = patches[act ? occ_patch[o] : 0];
+    int lo[3], wd[3];
+    const int ns = row_window(pd, act ? occ_local[o] : 0, lo, wd);
+    constexpr unsigned long long GM = G == 64 ? ~0ull : (1ull << (G & 63)) - 1;
+    int cnt = 0, last = -1;
+    bool up = true;
+    for (int s0 = 0; __any(s0 < ns); s0 += G) {
+        const int g = act && s0 + lane < ns ? window_dof(pd, lo, wd, s0 + lane) : nfree;
+        const bool fr = g < nfree;
+        const unsigned long long m = (__ballot(fr) >> shift) & GM, below = m & ((1ull << lane) - 1);
+        if (WRITE) {
+            const int prev = __shfl(g, below ? 63 - __clzll(below) : 0, G);
+            const int top = __shfl(g, m ? 63 - __clzll(m) : 0, G);
+            up = up && (!fr || g > (below ? prev : last));
+            if (m) last = top;
+            if (fr) sG[w][cnt + __popcll(below)] = g;
+        }
+        cnt += __popcll(m);
+    }
+    if (!WRITE) {
+        if (act && lane == 0) counts[r] = cnt;
+        return;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const bool sorted = ((__ballot(up) >> shift) & GM) == GM;
+    if (!act) return;
+    int *out = col + rowptr[r];
+    for (int k = lane; k < cnt; k += G) {
+        const int g = sG[w][k];
+        int rank = k;
+        if (!sorted) {
+            rank = 0;
+            for (int j = 0; j < cnt; ++j) rank += sG[w][j] < g || (sG[w][j] == g && j < k);
+        }
+        out[rank] = g;
+    }
+}
+
+// Rows of several occurrences (coupled functions, rows [r0, nfree)): a block
+// per row keeps the sorted union in LDS and merges one occurrence's window at
+// a time; every thread ranks its columns by counting and bisection.  Bound by
+// latency: 2.2 K rows 18 us.
+template <int WRITE>
+__global__ __launch_bounds__(256) void k_row_multi(const PatchDev *__restrict__ patches,
+                                                   const int *__restrict__ occ_ptr, const int *__restrict__ occ_patch,
+                                                   const int64_t *__restrict__ occ_local, int nfree, int r0,
+                                                   int *__restrict__ counts, int *__restrict__ overflow,
+                                                   const int *__restrict__ rowptr, int *__restrict__ col)
+{
+    __shared__ int sU[2][kMaxMultiCols], sN[kMaxMultiCols], nnew;
+    const int r = r0 + blockIdx.x, t = threadIdx.x;
+    int cur = 0, cnt = 0;
+    bool over = false;
+    for (int o = occ_ptr[r]; o < occ_ptr[r + 1]; ++o) {
         const PatchDev &pd = patches[occ_patch[o]];
-        int l[3];
-        local_coords(pd, occ_local[o], l);
-        int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-        for (int k = 0; k < pd.d; ++k) {
-            lo[k] = max(0, l[k] - pd.p[k]);
-            hi[k] = min(pd.nb[k] - 1, l[k] + pd.p[k]);
+        int lo[3], wd[3];
+        const int ns = row_window(pd, occ_local[o], lo, wd);
+        if (t == 0) nnew = 0;
+        __syncthreads();
+        // columns not in the union yet, in any order (their ranks follow from
+        // their values)
+        for (int s = t; s < ns; s += 256) {
+            const int g = window_dof(pd, lo, wd, s);
+            if (g >= nfree) continue;
+            int a = 0, b = cnt;
+            while (a < b) {
+                const int mid = (a + b) >> 1;
+                if (sU[cur][mid] < g) a = mid + 1; else b = mid;
+            }
+            if (a < cnt && sU[cur][a] == g) continue;
+            sN[atomicAdd(&nnew, 1)] = g;   // at most 9^3 entries
         }
-        for (int z = lo[2]; z <= hi[2]; ++z)
-            for (int y = lo[1]; y <= hi[1]; ++y)
-                for (int x = lo[0]; x <= hi[0]; ++x) {
-                    const int64_t m = x + (int64_t)pd.nb[0] * (y + (int64_t)pd.nb[1] * z);
-                    const int g = pd.dofs[m];
-                    if (g >= nfree) continue;
-                    // sorted insert with dedup
-                    int lo2 = 0, hi2 = cnt;
-                    while (lo2 < hi2) {
-                        const int mid = (lo2 + hi2) >> 1;
-                        if (buf[mid] < g) lo2 = mid + 1; else hi2 = mid;
-                    }
-                    if (lo2 < cnt && buf[lo2] == g) continue;
-                    if (cnt >= kMaxMultiCols) return -1;
-                    for (int i = cnt; i > lo2; --i) buf[i] = buf[i - 1];
-                    buf[lo2] = g;
-                    ++cnt;
+        __syncthreads();
+        const int nn = nnew;
+        // a patch glued to itself can show a column twice: its copies count once
+        int dup = 0;
+        for (int k = t; k < nn; k += 256)
+            for (int j = 0; j < k; ++j)
+                if (sN[j] == sN[k]) {
+                    dup = 1;
+                    break;
                 }
+        dup = __syncthreads_count(dup);
+        if (dup) {
+            if (t == 0) {
+                int m = 0;
+                for (int k = 0; k < nn; ++k) {
+                    bool seen = false;
+                    for (int j = 0; j < m; ++j) seen = seen || sN[j] == sN[k];
+                    if (!seen) sN[m++] = sN[k];
+                }
+                nnew = m;
+            }
+            __syncthreads();
+        }
+        const int add = nnew;
+        if (cnt + add > kMaxMultiCols) {
+            over = true;
+            break;   // uniform
+        }
+        for (int k = t; k < cnt; k += 256) {
+            int below = 0;
+            for (int j = 0; j < add; ++j) below += sN[j] < sU[cur][k];
+            sU[1 - cur][k + below] = sU[cur][k];
+        }
+        for (int k = t; k < add; k += 256) {
+            const int g = sN[k];
+            int a = 0, b = cnt, below = 0;
+            while (a < b) {
+                const int mid = (a + b) >> 1;
+                if (sU[cur][mid] < g) a = mid + 1; else b = mid;
+            }
+            for (int j = 0; j < add; ++j) below += sN[j] < g;
+            sU[1 - cur][a + below] = g;
+        }
+        cnt += add;
+        cur = 1 - cur;
+        __syncthreads();
     }
-    if (WRITE)
-        for (int i = 0; i < cnt; ++i) out[i] = buf[i];
-    return cnt;
-}
-
-__global__ void k_rowcount(const PatchDev *__restrict__ patches, const int *__restrict__ occ_ptr,
-                           const int *__restrict__ occ_patch, const int64_t *__restrict__ occ_local,
-                           int nfree, int *__restrict__ counts, int *__restrict__ err)
-{
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nfree) return;
-    const int c = row_columns<false>(patches, occ_ptr, occ_patch, occ_local, nfree, r, nullptr);
-    if (c < 0) {
-        err[0] = 1;
-        counts[r] = 0;
-    } else {
-        counts[r] = c;
+    if (WRITE) {
+        for (int k = t; k < cnt; k += 256) col[rowptr[r] + k] = sU[cur][k];
+    } else if (t == 0) {
+        counts[r] = over ? 0 : cnt;
+        if (over) overflow[0] = 1;
     }
-}
-
-__global__ void k_rowfill(const PatchDev *__restrict__ patches, const int *__restrict__ occ_ptr,
-                          const int *__restrict__ occ_patch, const int64_t *__restrict__ occ_local,
-                          int nfree, const int *__restrict__ rowptr, int *__restrict__ col)
-{
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nfree) return;
-    row_columns<true>(patches, occ_ptr, occ_patch, occ_local, nfree, r, col + rowptr[r]);
 }
 
 // ---------------------------------------------------------------------------
@@ -500,9 +573,11 @@ constexpr int kScanBlock = 1024;
 
 __global__ __launch_bounds__(kScanBlock) void k_scan_local(const int *__restrict__ in, int n,
                                                            int *__restrict__ out,
-                                                           long long *__restrict__ bsum)
+                                                           long long *__restrict__ bsum,
+                                                           int *__restrict__ longest)
 {
     __shared__ long long s[kScanBlock];
+    __shared__ int sm[kScanBlock / kWave];
     const int i = blockIdx.x * kScanBlock + threadIdx.x;
     long long v = (i < n) ? in[i] : 0;
     s[threadIdx.x] = v;
@@ -515,19 +590,40 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_local(const int *__restrict
     }
     if (i < n) out[i] = (int)(s[threadIdx.x] - v);
     if (threadIdx.x == kScanBlock - 1) bsum[blockIdx.x] = s[threadIdx.x];
+    if (!longest) return;
+    int m = (int)v;
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off, kWave));
+    if (threadIdx.x % kWave == 0) sm[threadIdx.x / kWave] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kScanBlock / kWave; ++w) m = max(m, sm[w]);
+        atomicMax(longest, m);
+    }
 }
 
-__global__ void k_scan_blocks(long long *__restrict__ bsum, int nb, long long *__restrict__ total)
+// exclusive scan of the block sums, one block
+__global__ __launch_bounds__(kScanBlock) void k_scan_blocks(long long *__restrict__ bsum, int nb,
+                                                            long long *__restrict__ total)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        long long acc = 0;
-        for (int b = 0; b < nb; ++b) {
-            const long long v = bsum[b];
-            bsum[b] = acc;
-            acc += v;
+    __shared__ long long s[kScanBlock];
+    long long carry = 0;
+    for (int b0 = 0; b0 < nb; b0 += kScanBlock) {
+        const int b = b0 + threadIdx.x;
+        const long long v = b < nb ? bsum[b] : 0;
+        s[threadIdx.x] = v;
+        __syncthreads();
+        for (int off = 1; off < kScanBlock; off <<= 1) {
+            const long long a = threadIdx.x >= off ? s[threadIdx.x - off] : 0;
+            __syncthreads();
+            s[threadIdx.x] += a;
+            __syncthreads();
         }
-        total[0] = acc;
+        if (b < nb) bsum[b] = carry + s[threadIdx.x] - v;
+        carry += s[kScanBlock - 1];
+        __syncthreads();
     }
+    if (threadIdx.x == 0) total[0] = carry;
 }
 
 __global__ void k_scan_add(int *__restrict__ out, int n, const long long *__restrict__ bsum,
@@ -851,53 +947,90 @@ __global__ __launch_bounds__(256) void k_gather_patch(PatchBox bx, int nfree, in
     }
 }
 
-// Single-patch pattern: row r's columns are the free functions of the
-// window [i - P, i + P] clipped to the free box, lexicographic (= ascending
-// free index).  One wavefront per row, lanes write consecutive columns.
-template <int D, int P>
-__global__ __launch_bounds__(256) void k_rowfill_patch(PatchBox bx, int nfree, const int *__restrict__ f2g,
-                                                       const int *__restrict__ rowptr,
-                                                       int *__restrict__ col)
+// Pattern of a single patch whose free functions form a box of m per direction:
+// row a of a direction has c(a) = min(m - 1, a + p) - max(0, a - p) + 1 columns,
+// and the row pointers follow from the sums S(a) = c(0) + .. + c(a - 1).
+__host__ __device__ inline int64_t band_sum(int a, int m, int p)
 {
-    const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int r = blockIdx.x * 4 + w;
-    if (r >= nfree) return;
-    const int g = f2g[r];
-    int ic[3];
-    ic[0] = g % bx.padded[0] - P;
-    ic[1] = (g / bx.padded[0]) % bx.padded[1] - P;
-    ic[2] = (D == 3) ? g / (bx.padded[0] * bx.padded[1]) - P : 0;
-    int lo[3] = {0, 0, 0}, wd[3] = {1, 1, 1}, fw[3] = {1, 1, 1};
-#pragma unroll
-    for (int k = 0; k < D; ++k) {
-        lo[k] = max(bx.flo[k], ic[k] - P);
-        wd[k] = min(bx.fhi[k], ic[k] + P) - lo[k] + 1;
-        fw[k] = bx.fhi[k] - bx.flo[k] + 1;
+    const int64_t t = a - 1 - p > 0 ? a - 1 - p : 0, e = m - 1 - p > 0 ? m - 1 - p : 0;   // c is full below e
+    const int64_t u = a < e ? a : e;
+    return u * (u - 1) / 2 + u * p + (a - u) * (int64_t)(m - 1) - t * (t + 1) / 2 + a;
+}
+
+struct BoxRows {
+    int m[3], p;
+    __host__ __device__ inline int64_t start(int i, int j, int k) const
+    {
+        const int64_t nx = band_sum(m[0], m[0], p), ny = band_sum(m[1], m[1], p);
+        const int64_t cy = band_sum(j + 1, m[1], p) - band_sum(j, m[1], p);
+        const int64_t cz = m[2] > 1 ? band_sum(k + 1, m[2], p) - band_sum(k, m[2], p) : 1;
+        const int64_t sz = m[2] > 1 ? band_sum(k, m[2], p) : k;
+        return sz * nx * ny + cz * (band_sum(j, m[1], p) * nx + cy * band_sum(i, m[0], p));
     }
-    const int rb = rowptr[r], len = rowptr[r + 1] - rb;
-    for (int q = lane; q < len; q += kWave) {
-        const int qx = q % wd[0], qy = (q / wd[0]) % wd[1], qz = (D == 3) ? q / (wd[0] * wd[1]) : 0;
-        const int jx = lo[0] + qx - bx.flo[0], jy = lo[1] + qy - bx.flo[1];
-        const int jz = (D == 3) ? lo[2] + qz - bx.flo[2] : 0;
-        col[rb + q] = jx + fw[0] * (jy + fw[1] * jz);
+};
+
+// Row pointers and columns by row segments of an x-line; a thread keeps its
+// stencil offsets over the segment's rows.  Bound by the bytes written: 64^3
+// elements p = 3 (346 MB) 78 us; counted, scanned and filled row by row 270 us
+// and a copy of the counts to the host.
+template <int D, int P>
+__global__ __launch_bounds__(256) void k_box_pattern(BoxRows B, int nfree, int *__restrict__ rowptr,
+                                                     int *__restrict__ col)
+{
+    constexpr int W = 2 * P + 1, NS = D == 3 ? W * W * W : W * W, R = 32;
+    __shared__ int sBase[R];
+    const int t = threadIdx.x;
+    const int nseg = (B.m[0] + R - 1) / R, seg = blockIdx.x % nseg, j = (blockIdx.x / nseg) % B.m[1];
+    const int k = blockIdx.x / nseg / B.m[1];
+    const int i0 = (int)((int64_t)B.m[0] * seg / nseg), nr = (int)((int64_t)B.m[0] * (seg + 1) / nseg) - i0;
+    const int r0 = i0 + B.m[0] * (j + B.m[1] * k);
+    if (t < nr) {
+        const int b = (int)B.start(i0 + t, j, k);
+        sBase[t] = b;
+        rowptr[r0 + t] = b;
+    }
+    if (blockIdx.x == 0 && t == 0)
+        rowptr[nfree] = (int)(band_sum(B.m[0], B.m[0], P) * band_sum(B.m[1], B.m[1], P) *
+                              (D == 3 ? band_sum(B.m[2], B.m[2], P) : 1));
+    __syncthreads();
+    const int ylo = max(-P, -j), ny = min(P, B.m[1] - 1 - j) - ylo + 1;
+    const int zlo = D == 3 ? max(-P, -k) : 0, nz = D == 3 ? min(P, B.m[2] - 1 - k) - zlo + 1 : 1;
+    constexpr int G = NS < 256 ? 256 / NS : 1;   // rows at a time
+    const int g = NS < 256 ? t / NS : 0;
+    if (g >= G) return;
+#pragma unroll
+    for (int s0 = 0; s0 < NS; s0 += 256) {
+        const int sl = NS < 256 ? t % NS : s0 + t;
+        const int ox = sl % W - P, oy = (sl / W) % W - P, oz = D == 3 ? sl / (W * W) - P : 0;
+        if (sl >= NS || oy < ylo || oy >= ylo + ny || oz < zlo || oz >= zlo + nz) continue;
+        const int yz = (oz - zlo) * ny + oy - ylo, off = ox + B.m[0] * (oy + B.m[1] * oz);
+        for (int rr = g; rr < nr; rr += G) {
+            const int i = i0 + rr, lo = max(-P, -i), nx = min(P, B.m[0] - 1 - i) - lo + 1;
+            if (ox >= lo && ox < lo + nx) col[sBase[rr] + yz * nx + ox - lo] = r0 + rr + off;
+        }
     }
 }
 
-hipError_t launch_rowfill_patch(int d, int p, const int *flo, const int *fhi, const int *nb,
-                                const int *nel, const int *padded, int nfree, const int *f2g,
-                                const int *rowptr, int *col, hipStream_t s)
+// entries of the box's pattern, and of its longest row
+int64_t box_pattern_nnz(int d, int p, const int *m, int *maxrow)
+{
+    int64_t n = 1;
+    *maxrow = 1;
+    for (int k = 0; k < d; ++k) {
+        n *= band_sum(m[k], m[k], p);
+        *maxrow *= std::min(m[k], 2 * p + 1);
+    }
+    return n;
+}
+
+hipError_t launch_box_pattern(int d, int p, const int *m, int nfree, int *rowptr, int *col, hipStream_t s)
 {
     if (nfree <= 0) return hipSuccess;
-    PatchBox bx;
-    for (int k = 0; k < 3; ++k) {
-        bx.flo[k] = flo[k];
-        bx.fhi[k] = fhi[k];
-        bx.nb[k] = nb[k];
-        bx.nel[k] = nel[k];
-        bx.padded[k] = padded[k];
-    }
-    const dim3 grid((nfree + 3) / 4), blk(256);
-#define GSX_F(D, P) if (d == D && p == P) { hipLaunchKernelGGL((k_rowfill_patch<D, P>), grid, blk, 0, s, bx, nfree, f2g, rowptr, col); return hipGetLastError(); }
+    BoxRows B;
+    for (int k = 0; k < 3; ++k) B.m[k] = k < d ? m[k] : 1;
+    B.p = p;
+    const dim3 grid((unsigned)((int64_t)((m[0] + 31) / 32) * B.m[1] * B.m[2])), blk(256);
+#define GSX_F(D, P) if (d == D && p == P) { hipLaunchKernelGGL((k_box_pattern<D, P>), grid, blk, 0, s, B, nfree, rowptr, col); return hipGetLastError(); }
     GSX_F(2, 1) GSX_F(2, 2) GSX_F(2, 3) GSX_F(2, 4)
     GSX_F(3, 1) GSX_F(3, 2) GSX_F(3, 3) GSX_F(3, 4)
 #undef GSX_F
@@ -1458,33 +1591,34 @@ hipError_t launch_norms(int d, int p, const PatchDev *patches, const int *gpatch
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_rowcount(const PatchDev *patches, const int *occ_ptr, const int *occ_patch,
-                           const int64_t *occ_local, int nfree, int *counts, int *err,
-                           hipStream_t s)
+hipError_t launch_row_pattern(const PatchDev *patches, const int *occ_ptr, const int *occ_patch,
+                              const int64_t *occ_local, int nfree, int nsingle, bool flat, int *counts, int *overflow,
+                              const int *rowptr, int *col, hipStream_t s)
 {
-    if (nfree <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_rowcount, dim3((nfree + 127) / 128), dim3(128), 0, s, patches, occ_ptr,
-                       occ_patch, occ_local, nfree, counts, err);
+    const bool write = col != nullptr;
+    if (nsingle > 0) {
+#define GSX_R(W, G) hipLaunchKernelGGL((k_row_single<W, G>), dim3((nsingle + 256 / G - 1) / (256 / G)), dim3(256), 0, s, patches, occ_ptr, occ_patch, occ_local, nfree, nsingle, counts, rowptr, col)
+        if (flat && write) GSX_R(1, 16);
+        else if (flat) GSX_R(0, 16);
+        else if (write) GSX_R(1, 64);
+        else GSX_R(0, 64);
+#undef GSX_R
+    }
+    if (nfree > nsingle) {
+        const dim3 grid(nfree - nsingle), blk(256);
+        if (write) hipLaunchKernelGGL((k_row_multi<1>), grid, blk, 0, s, patches, occ_ptr, occ_patch, occ_local, nfree, nsingle, counts, overflow, rowptr, col);
+        else hipLaunchKernelGGL((k_row_multi<0>), grid, blk, 0, s, patches, occ_ptr, occ_patch, occ_local, nfree, nsingle, counts, overflow, rowptr, col);
+    }
     return hipGetLastError();
 }
 
-hipError_t launch_rowfill(const PatchDev *patches, const int *occ_ptr, const int *occ_patch,
-                          const int64_t *occ_local, int nfree, const int *rowptr, int *col,
-                          hipStream_t s)
-{
-    if (nfree <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_rowfill, dim3((nfree + 127) / 128), dim3(128), 0, s, patches, occ_ptr,
-                       occ_patch, occ_local, nfree, rowptr, col);
-    return hipGetLastError();
-}
-
-hipError_t launch_scan(const int *counts, int n, int *rowptr, long long *bsum, long long *total,
+hipError_t launch_scan(const int *counts, int n, int *rowptr, long long *bsum, long long *total, int *longest,
                        hipStream_t s)
 {
     const int nb = (n + kScanBlock - 1) / kScanBlock;
     if (nb > 0)
-        hipLaunchKernelGGL(k_scan_local, dim3(nb), dim3(kScanBlock), 0, s, counts, n, rowptr, bsum);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(64), 0, s, bsum, nb, total);
+        hipLaunchKernelGGL(k_scan_local, dim3(nb), dim3(kScanBlock), 0, s, counts, n, rowptr, bsum, longest);
+    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(kScanBlock), 0, s, bsum, nb, total);
     hipLaunchKernelGGL(k_scan_add, dim3((n + 1 + 255) / 256), dim3(256), 0, s, rowptr, n, bsum, total);
     return hipGetLastError();
 }
@@ -1536,7 +1670,7 @@ hipError_t launch_keep(const int *rowptr, const int *col, const double *val,
         return hipGetLastError();
     }
     hipLaunchKernelGGL(k_keep_count, dim3((n + 127) / 128), dim3(128), 0, s, rowptr, keep, n, counts);
-    hipError_t e = launch_scan(counts, n, nrowptr, bsum, total, s);
+    hipError_t e = launch_scan(counts, n, nrowptr, bsum, total, nullptr, s);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_keep_copy, dim3((n + 127) / 128), dim3(128), 0, s, rowptr, col, val, keep, n,
                        nrowptr, ncol, nval);

@@ -45,13 +45,16 @@ int64_t norm_blocks(int d, int p, const int *nel);
 hipError_t launch_norms(int d, int p, const PatchDev *patches, const int *gpatch, const int64_t *bprefix, int ng,
                         int64_t nblocks, const GaussTab &gt, const double *sol, int nfree, double *out,
                         double *out_h1, const double *fixed, hipStream_t s);
-hipError_t launch_rowcount(const PatchDev *patches, const int *occ_ptr, const int *occ_patch,
-                           const int64_t *occ_local, int nfree, int *counts, int *err,
-                           hipStream_t s);
-hipError_t launch_rowfill(const PatchDev *patches, const int *occ_ptr, const int *occ_patch,
-                          const int64_t *occ_local, int nfree, const int *rowptr, int *col,
-                          hipStream_t s);
-hipError_t launch_scan(const int *counts, int n, int *rowptr, long long *bsum, long long *total,
+// CSR pattern: row counts (col null; overflow set where a row is too long) or
+// columns; rows [nsingle, nfree) have several occurrences; flat: 2D windows
+hipError_t launch_row_pattern(const PatchDev *patches, const int *occ_ptr, const int *occ_patch,
+                              const int64_t *occ_local, int nfree, int nsingle, bool flat, int *counts, int *overflow,
+                              const int *rowptr, int *col, hipStream_t s);
+// pattern of a single patch whose free functions form a box of m per direction
+int64_t box_pattern_nnz(int d, int p, const int *m, int *maxrow);
+hipError_t launch_box_pattern(int d, int p, const int *m, int nfree, int *rowptr, int *col, hipStream_t s);
+// longest (may be null, starts at 0): the largest count
+hipError_t launch_scan(const int *counts, int n, int *rowptr, long long *bsum, long long *total, int *longest,
                        hipStream_t s);
 int gather_maxrow_bucket(int maxrow);
 // boundary element terms (k_bdry): per item, the boundary-layer mass matrix
@@ -62,9 +65,6 @@ hipError_t launch_gather(const PatchDev *patches, const int *occ_ptr, const int 
                          const int64_t *occ_local, int nfree, const int *rowptr, const int *col,
                          const double *Kbuf, const double *Fbuf, double *val, double *rhs,
                          unsigned char *keep, int maxrow, const double *fixed, hipStream_t s);
-hipError_t launch_rowfill_patch(int d, int p, const int *flo, const int *fhi, const int *nb,
-                                const int *nel, const int *padded, int nfree, const int *f2g,
-                                const int *rowptr, int *col, hipStream_t s);
 // rows [r0, r1) of the free box; Kbuf/Fbuf hold the elements from global
 // element id elbase on
 hipError_t launch_gather_patch(int d, int p, const int *flo, const int *fhi, const int *nb,

@@ -267,6 +267,7 @@ struct gsx_problem {
     DevPtr d_patches, d_dofs;
     std::vector<DevPtr> keep;      // knots, ctrl, kappa, felem
     DevPtr d_occ_ptr, d_occ_patch, d_occ_local;
+    int nsingle = 0;               // rows [0, nsingle) have one occurrence each
     std::vector<Group> groups;
     // pattern cache
     bool have_pattern = false;
@@ -847,6 +848,7 @@ gsx_status gsx_problem_create(gsx_ctx *c, int32_t npatch, const gsx_patch_desc *
     std::vector<int> occ_cnt(nfree + 1, 0);
     for (int64_t i = 0; i < P->nbasis; ++i)
         if (P->dofs[i] < nfree) occ_cnt[P->dofs[i] + 1]++;
+    while (P->nsingle < nfree && occ_cnt[P->nsingle + 1] == 1) ++P->nsingle;
     for (int r = 0; r < nfree; ++r) occ_cnt[r + 1] += occ_cnt[r];
     std::vector<int> occ_patch(occ_cnt[nfree]);
     std::vector<int64_t> occ_local(occ_cnt[nfree]);
@@ -1044,53 +1046,58 @@ static gsx_status pattern_build(gsx_problem *P)
     gsx_ctx *c = P->ctx;
     hipStream_t s = c->stream;
     const int n = P->nfree;
-    DevPtr counts = dalloc(c, sizeof(int) * (n + 1));
-    DevPtr errf = dalloc(c, sizeof(int));
     P->d_rowptr = dalloc(c, sizeof(int) * (n + 1));
     const int nblk = (n + 1023) / 1024 + 1;
     P->d_scan_bsum = dalloc(c, sizeof(long long) * nblk);
     P->d_scan_total = dalloc(c, sizeof(long long));
-    if (!counts || !errf || !P->d_rowptr || !P->d_scan_bsum || !P->d_scan_total)
+    if (!P->d_rowptr || !P->d_scan_bsum || !P->d_scan_total)
         return fail(c, GSX_ERR_OOM, "device allocation (pattern)");
-    HIP_OK(c, hipMemsetAsync(errf.get(), 0, sizeof(int), s));
+    if (n > 0 && P->npatch == 1 && P->d_f2g) {
+        // a box of free functions: the pattern in closed form
+        const HostPatch &h = P->hp[0];
+        int m[3] = {1, 1, 1};
+        for (int k = 0; k < h.d; ++k) m[k] = P->box_hi[k] - P->box_lo[k] + 1;
+        const int64_t total = gsx::box_pattern_nnz(h.d, h.p[0], m, &P->maxrow);
+        if (total >= (int64_t)INT32_MAX) return fail(c, GSX_ERR_ARG, "nnz exceeds int32 indexing");
+        P->nnz = total;
+        P->d_col = dalloc(c, sizeof(int) * std::max<int64_t>(1, total));
+        if (!P->d_col) return fail(c, GSX_ERR_OOM, "device allocation (col)");
+        KScope k(c, "pattern_fill");
+        HIP_OK(c, gsx::launch_box_pattern(h.d, h.p[0], m, n, dp<int>(P->d_rowptr), dp<int>(P->d_col), s));
+        P->have_pattern = true;
+        return GSX_OK;
+    }
+    DevPtr counts = dalloc(c, sizeof(int) * (n + 1));
+    DevPtr info = dalloc(c, sizeof(int) * 2);
+    if (!counts || !info) return fail(c, GSX_ERR_OOM, "device allocation (pattern)");
+    HIP_OK(c, hipMemsetAsync(info.get(), 0, sizeof(int) * 2, s));
     {
         KScope k(c, "pattern_count");
-        HIP_OK(c, gsx::launch_rowcount(dp<PatchDev>(P->d_patches), dp<int>(P->d_occ_ptr),
-                                       dp<int>(P->d_occ_patch), dp<int64_t>(P->d_occ_local), n,
-                                       dp<int>(counts), dp<int>(errf), s));
+        HIP_OK(c, gsx::launch_row_pattern(dp<PatchDev>(P->d_patches), dp<int>(P->d_occ_ptr), dp<int>(P->d_occ_patch),
+                                          dp<int64_t>(P->d_occ_local), n, P->nsingle, P->hp[0].d == 2, dp<int>(counts), dp<int>(info),
+                                          nullptr, nullptr, s));
     }
     {
         KScope k(c, "pattern_scan");
         HIP_OK(c, gsx::launch_scan(dp<int>(counts), n, dp<int>(P->d_rowptr),
-                                   dp<long long>(P->d_scan_bsum), dp<long long>(P->d_scan_total), s));
+                                   dp<long long>(P->d_scan_bsum), dp<long long>(P->d_scan_total), dp<int>(info) + 1, s));
     }
-    int errh = 0;
+    int infoh[2] = {0, 0};
     long long total = 0;
-    HIP_OK(c, hipMemcpyAsync(&errh, errf.get(), sizeof(int), hipMemcpyDeviceToHost, s));
+    HIP_OK(c, hipMemcpyAsync(infoh, info.get(), sizeof(infoh), hipMemcpyDeviceToHost, s));
     HIP_OK(c, hipMemcpyAsync(&total, P->d_scan_total.get(), sizeof(long long), hipMemcpyDeviceToHost, s));
     HIP_OK(c, hipStreamSynchronize(s));
-    if (errh) return fail(c, GSX_ERR_ARG, "row of an interface DOF exceeds the pattern buffer");
+    if (infoh[0]) return fail(c, GSX_ERR_ARG, "row of an interface DOF exceeds the pattern buffer");
     if (total >= (long long)INT32_MAX) return fail(c, GSX_ERR_ARG, "nnz exceeds int32 indexing");
-    // max row length
-    std::vector<int> cnt(n);
-    HIP_OK(c, hipMemcpyAsync(cnt.data(), counts.get(), sizeof(int) * n, hipMemcpyDeviceToHost, s));
-    HIP_OK(c, hipStreamSynchronize(s));
-    P->maxrow = n ? *std::max_element(cnt.begin(), cnt.end()) : 0;
+    P->maxrow = infoh[1];
     P->nnz = total;
     P->d_col = dalloc(c, sizeof(int) * std::max<long long>(1, total));
     if (!P->d_col) return fail(c, GSX_ERR_OOM, "device allocation (col)");
     {
         KScope k(c, "pattern_fill");
-        if (P->npatch == 1 && P->d_f2g) {
-            const HostPatch &h = P->hp[0];
-            HIP_OK(c, gsx::launch_rowfill_patch(h.d, h.p[0], P->box_lo, P->box_hi, h.nb, h.nel,
-                                                P->grid_dims, n, dp<int>(P->d_f2g), dp<int>(P->d_rowptr),
-                                                dp<int>(P->d_col), s));
-        } else {
-            HIP_OK(c, gsx::launch_rowfill(dp<PatchDev>(P->d_patches), dp<int>(P->d_occ_ptr),
-                                          dp<int>(P->d_occ_patch), dp<int64_t>(P->d_occ_local), n,
+        HIP_OK(c, gsx::launch_row_pattern(dp<PatchDev>(P->d_patches), dp<int>(P->d_occ_ptr), dp<int>(P->d_occ_patch),
+                                          dp<int64_t>(P->d_occ_local), n, P->nsingle, P->hp[0].d == 2, nullptr, nullptr,
                                           dp<int>(P->d_rowptr), dp<int>(P->d_col), s));
-        }
     }
     P->have_pattern = true;
     return GSX_OK;
@@ -2887,7 +2894,7 @@ static gsx_status scan_counts(gsx_ctx *c, const int *counts, int n, DevPtr &rowp
     DevPtr bsum = dalloc(c, sizeof(long long) * ((n + 1023) / 1024 + 2));
     DevPtr tot = dalloc(c, sizeof(long long));
     if (!rowptr || !bsum || !tot) return fail(c, GSX_ERR_OOM, "device allocation (scan)");
-    HIP_OK(c, gsx::launch_scan(counts, n, dp<int>(rowptr), dp<long long>(bsum), dp<long long>(tot), s));
+    HIP_OK(c, gsx::launch_scan(counts, n, dp<int>(rowptr), dp<long long>(bsum), dp<long long>(tot), nullptr, s));
     long long t = 0;
     HIP_OK(c, hipMemcpyAsync(&t, tot.get(), sizeof(long long), hipMemcpyDeviceToHost, s));
     HIP_OK(c, hipStreamSynchronize(s));

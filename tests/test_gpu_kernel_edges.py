@@ -280,3 +280,56 @@ def test_row_assembly_2d(ctx, p, n, gx, gy):
     assert (r[5] != r[5].T).nnz == 0   # bitwise symmetric
     assert np.linalg.norm(r[3] - r[5] @ r[6]) <= 1.01e-10 * np.linalg.norm(r[3])
     gp.close()
+
+
+def _glued_boxes(d, p, n, g):
+    """g boxes per direction, glued; every outer side is a Dirichlet side."""
+    patches, sides, ifaces = [], [], []
+    at = {i: k for k, i in enumerate(np.ndindex(*g))}
+    for i, k in at.items():
+        patches.append(problems.box_patch(d, p, n, lo=[float(a) for a in i], hi=[a + 1.0 for a in i]))
+        for j in range(d):
+            t = [a for a in range(d) if a != j]
+            up = at.get(tuple(a + (b == j) for b, a in enumerate(i)))
+            if i[j] == 0:
+                sides.append((k, 2 * j + 1))
+            if up is None:
+                sides.append((k, 2 * j + 2))
+            else:
+                ifaces.append((k, 2 * j + 2, up, 2 * j + 1, t[0], 0) + ((t[1], 0) if d == 3 else (0, 0)))
+    return problems.Problem(patches, sides, ifaces)
+
+
+# pattern kernels: rows of one occurrence by 16 or 64 lanes, coupled rows by
+# merging windows (up to 8 patches at a corner), the closed form of a box in
+# segments of 32 rows
+@pytest.mark.parametrize("d,p,n,g", [(2, 1, (1, 2), (1, 1)), (2, 4, (3, 70), (1, 1)), (3, 1, (2, 1, 2), (1, 1, 1)),
+                                     (3, 4, (1, 34, 2), (1, 1, 1)), (3, 2, (65, 3, 2), (1, 1, 1)),
+                                     (2, 1, (1, 1), (2, 2)), (2, 3, (5, 2), (3, 2)), (2, 4, (33, 3), (2, 3)),
+                                     (3, 1, (2, 2, 1), (2, 2, 2)), (3, 3, (2, 3, 2), (2, 2, 1)), (3, 4, (2, 2, 2), (1, 1, 2))])
+@pytest.mark.parametrize("sides", [0, 1, 2])
+def test_row_patterns(ctx, d, p, n, g, sides):
+    """CSR patterns against the union of the functions' windows."""
+    prob = _glued_boxes(d, p, n, g)
+    prob.dir_sides = prob.dir_sides[::2] if sides == 1 else prob.dir_sides[:1] if sides == 2 else prob.dir_sides
+    gp = gsx.Problem(ctx, prob)
+    if gp.nfree == 0:
+        gp.close()
+        return
+    dofs_all, off = gp.dofs(), 0
+    want = [set() for _ in range(gp.nfree)]
+    for k, P in enumerate(prob.patches):
+        nb = [len(u) - P.p[0] - 1 for u in P.knots]
+        dofs = dofs_all[off:off + P.nbasis].reshape(nb[::-1])
+        off += P.nbasis
+        for loc in np.ndindex(*nb[::-1]):
+            r = dofs[loc]
+            if r < gp.nfree:
+                w = dofs[tuple(slice(max(0, i - p), i + p + 1) for i in loc)].ravel()
+                want[r].update(w[w < gp.nfree].tolist())
+    A, b = gp.assemble(gsx.PATTERN_FULL | gsx.ASM_REBUILD_PATTERN)
+    rp, ci, va = A.download()
+    assert np.array_equal(np.diff(rp), [len(w) for w in want])
+    assert np.array_equal(ci, np.concatenate([sorted(w) for w in want]) if gp.nfree else [])
+    for o in (A, b, gp):
+        o.close()
