@@ -456,56 +456,6 @@ __global__ void k_dense_scatter(int n, int npad, const int *__restrict__ rp, con
     for (int k = rp[r]; k < rp[r + 1]; ++k) D[(int64_t)r * npad + ci[k]] = v[k];
 }
 
-// invert the pivot block (kb) in LDS; result to Pinv (64x64, row-major).
-// In-place Gauss-Jordan over pairs of pivots: step p sweeps rows/columns
-// K = {p, p + 1} at once with the 2 x 2 inverse Q of M[K][K] (positive
-// determinant: the block is SPD),
-//   M'[K][K] = Q,  M'[K][c] = Q M[K][c],  M'[r][K] = -M[r][K] Q,
-//   M'[r][c] = M[r][c] - M[r][K] Q M[K][c],
-// which equals the two single sweeps in exact arithmetic and halves the
-// sequential steps.  Every entry is mapped from the old values (kept in
-// registers between the two barriers); 1024 threads, 4 entries each.
-constexpr int kPivThreads = 1024;
-__global__ __launch_bounds__(kPivThreads) void k_gj_pivot(double *__restrict__ D, int npad, int kb,
-                                                          double *__restrict__ Pinv)
-{
-    __shared__ double M[kGJ][kGJ + 1];
-    constexpr int PER = kGJ * kGJ / kPivThreads;
-    const int t = threadIdx.x;
-    for (int i = t; i < kGJ * kGJ; i += kPivThreads) M[i / kGJ][i % kGJ] = D[(int64_t)(kb + i / kGJ) * npad + kb + i % kGJ];
-    __syncthreads();
-    for (int p = 0; p < kGJ; p += 2) {
-        const double a = M[p][p], b = M[p][p + 1], c = M[p + 1][p], d = M[p + 1][p + 1];
-        const double id = 1.0 / (a * d - b * c);
-        const double q00 = d * id, q01 = -b * id, q10 = -c * id, q11 = a * id;
-        double nv[PER];
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const int i = t + kPivThreads * j, r = i / kGJ, col = i % kGJ;
-            const bool rin = (r >> 1) == (p >> 1), cin = (col >> 1) == (p >> 1);
-            const double m0 = M[p][col], m1 = M[p + 1][col];
-            double x;
-            if (rin) {
-                const double e0 = (r == p) ? q00 : q10, e1 = (r == p) ? q01 : q11;
-                x = cin ? ((col == p) ? e0 : e1) : e0 * m0 + e1 * m1;
-            } else {
-                const double u0 = M[r][p] * q00 + M[r][p + 1] * q10;
-                const double u1 = M[r][p] * q01 + M[r][p + 1] * q11;
-                x = cin ? -((col == p) ? u0 : u1) : M[r][col] - (u0 * m0 + u1 * m1);
-            }
-            nv[j] = x;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const int i = t + kPivThreads * j;
-            M[i / kGJ][i % kGJ] = nv[j];
-        }
-        __syncthreads();
-    }
-    for (int i = t; i < kGJ * kGJ; i += kPivThreads) Pinv[i] = M[i / kGJ][i % kGJ];
-}
-
 // Symmetric sweep (Gauss-Jordan in the form that keeps every intermediate
 // matrix symmetric).  Sweeping pivot block k of M:
 //   M'[k][k] = -B^-1,  M'[i][k] = M[i][k] B^-1,  M'[k][j] = B^-1 M[k][j],
@@ -513,59 +463,47 @@ __global__ __launch_bounds__(kPivThreads) void k_gj_pivot(double *__restrict__ D
 // after all blocks M = -A^-1.  Only the tiles I <= J are kept: a tile below
 // the diagonal is read as the transpose of its mirror.
 
-// W[J] = B^-1 M[k][J] for every column tile J != k; one block per tile
-__global__ __launch_bounds__(256) void k_gj_rowpanel(const double *__restrict__ D, int npad, int kb,
-                                                     const double *__restrict__ Pinv, double *__restrict__ W)
+// in-place sweep of the pair K = {p, p + 1} of a 4 x 4 block with the 2 x 2
+// inverse Q of m[K][K] (positive determinant: the block is SPD),
+//   m'[K][K] = Q,  m'[K][c] = Q m[K][c],  m'[r][K] = -m[r][K] Q,
+//   m'[r][c] = m[r][c] - m[r][K] Q m[K][c]
+template <int P>
+__device__ inline void gj_pair(double (&m)[4][4])
 {
-    __shared__ double sP[kGJ][kGJ + 1];
-    __shared__ double sR[kGJ][kGJ + 1];
-    const int t = threadIdx.x, j0 = blockIdx.x * kGJ;
-    if (j0 == kb) return;
-    for (int i = t; i < kGJ * kGJ; i += 256) {
-        const int r = i / kGJ, c = i % kGJ;
-        sP[r][c] = Pinv[i];
-        // M[k][J][r][c]: upper tile D[k][J], or the transpose of D[J][k]
-        // (read along D's rows, transposed into LDS)
-        if (j0 > kb) sR[r][c] = D[(int64_t)(kb + r) * npad + j0 + c];
-        else sR[c][r] = D[(int64_t)(j0 + r) * npad + kb + c];
+    const double id = 1.0 / (m[P][P] * m[P + 1][P + 1] - m[P][P + 1] * m[P + 1][P]);
+    const double q[2][2] = {{m[P + 1][P + 1] * id, -m[P][P + 1] * id}, {-m[P + 1][P] * id, m[P][P] * id}};
+    constexpr int O = 2 - P;   // the other pair
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const double u0 = m[O + r][P] * q[0][0] + m[O + r][P + 1] * q[1][0];
+        const double u1 = m[O + r][P] * q[0][1] + m[O + r][P + 1] * q[1][1];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) m[O + r][O + c] -= u0 * m[P][O + c] + u1 * m[P + 1][O + c];
+        m[O + r][P] = -u0;
+        m[O + r][P + 1] = -u1;
     }
-    __syncthreads();
-    for (int i = t; i < kGJ * kGJ; i += 256) {
-        const int r = i / kGJ, c = i % kGJ;
-        double s = 0.0;
-        for (int m = 0; m < kGJ; ++m) s += sP[r][m] * sR[m][c];
-        W[(int64_t)r * npad + j0 + c] = s;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const double w0 = q[0][0] * m[P][O + c] + q[0][1] * m[P + 1][O + c];
+        const double w1 = q[1][0] * m[P][O + c] + q[1][1] * m[P + 1][O + c];
+        m[P][O + c] = w0;
+        m[P + 1][O + c] = w1;
     }
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) m[P + r][P + c] = q[r][c];
 }
 
-// D[I][J] -= M[I][k] W[J] for the upper tiles I <= J, I, J != k.  FP64
-// matrix cores: each wavefront forms a 32x32 quadrant of the 64x64 tile as
-// 2x2 blocks of v_mfma_f64_16x16x4f64 over the 64-deep panel.  Operand
-// layout of that instruction: A[i][k] in lane i + 16 k, B[k][j] in lane
-// j + 16 k, D[i][j] in lane j + 16 (i % 4), element i / 4 (the rows of the
-// four result registers interleave).
+// 64 x 64 product of LDS tiles on the FP64 matrix cores: a wave's 32 x 32
+// quadrant as 2 x 2 blocks of v_mfma_f64_16x16x4f64 over the 64-deep panel.
+// Operand layout of that instruction: A[i][k] in lane i + 16 k, B[k][j] in
+// lane j + 16 k, D[i][j] in lane j + 16 (i % 4), element i / 4 (the rows of
+// the four result registers interleave).
 typedef double gj_d4 __attribute__((ext_vector_type(4)));
-__global__ __launch_bounds__(256) void k_gj_update(double *__restrict__ D, int npad, int kb,
-                                                   const double *__restrict__ W)
+__device__ inline void gj_product(const double (&A)[kGJ][kGJ + 1], const double (&B)[kGJ][kGJ + 1], int r0, int c0,
+                                  int li, int lk, gj_d4 (&acc)[2][2])
 {
-    const int I = blockIdx.y * kGJ, J = blockIdx.x * kGJ;
-    if (I == kb || J == kb || I > J) return;
-    __shared__ double sC[kGJ][kGJ + 1];
-    __shared__ double sW[kGJ][kGJ + 1];
-    const int t = threadIdx.x;
-    for (int i = t; i < kGJ * kGJ; i += 256) {
-        const int r = i / kGJ, c = i % kGJ;
-        // M[I][k]: upper tile D[I][k], or the transpose of D[k][I] (read
-        // along D's rows, transposed into LDS)
-        if (I < kb) sC[r][c] = D[(int64_t)(I + r) * npad + kb + c];
-        else sC[c][r] = D[(int64_t)(kb + r) * npad + I + c];
-        sW[r][c] = W[(int64_t)r * npad + J + c];
-    }
-    __syncthreads();
-    const int w = t / kWave, lane = t % kWave;
-    const int r0 = (w / 2) * 32, c0 = (w % 2) * 32;
-    const int li = lane % 16, lk = lane / 16;
-    gj_d4 acc[2][2];
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -573,57 +511,153 @@ __global__ __launch_bounds__(256) void k_gj_update(double *__restrict__ D, int n
 #pragma unroll 4
     for (int ks = 0; ks < kGJ / 4; ++ks) {
         const int m = 4 * ks + lk;
-        const double a0 = sC[r0 + li][m], a1 = sC[r0 + 16 + li][m];
-        const double b0 = sW[m][c0 + li], b1 = sW[m][c0 + 16 + li];
+        const double a0 = A[r0 + li][m], a1 = A[r0 + 16 + li][m];
+        const double b0 = B[m][c0 + li], b1 = B[m][c0 + 16 + li];
         acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
         acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
         acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
         acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
     }
+}
+
+// One sweep of the 64-block kb from S into T (both npad x npad), a block per
+// upper tile (I, J).  Every block inverts the pivot block itself, in
+// registers: 16 x 16 threads with 4 x 4 entries each, four pivots a step, whose
+// rows and columns go through LDS (two copies: one barrier a step); then
+// W = B^-1 M[k][J] and M[I][k] W on the matrix cores.  Bound by the chain of 16
+// steps: 29 us a sweep of a 256 x 256 pivot block (pivot, row panel, update and
+// swept panels in launches of their own: 70 us and three more gaps).
+__global__ __launch_bounds__(256) void k_gj_step(const double *__restrict__ S, double *__restrict__ T, int npad, int kb)
+{
+    const int J = blockIdx.x * kGJ, I = blockIdx.y * kGJ;
+    if (I > J) return;
+    __shared__ double sP[kGJ][kGJ + 1];
+    __shared__ double sA[kGJ][kGJ + 1];
+    __shared__ double sB[kGJ][kGJ + 1];
+    __shared__ double sR[2][4][kGJ], sC[2][4][kGJ];
+    constexpr int NQ = kGJ * kGJ / 256;
+    const int t = threadIdx.x, ty = t / 16, tx = t % 16;
+    double m[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) m[a][b] = S[(int64_t)(kb + 4 * ty + a) * npad + kb + 4 * tx + b];
+    // the panel tile M[k][X] that W is formed from, and M[I][k]: upper tiles,
+    // or the transposes of their mirrors (read along S's rows)
+    const int X = J == kb ? I : J;
+    const bool inner = I != kb && J != kb;
+    double ra[NQ], rb[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int r = (t + 256 * q) / kGJ, c = t % kGJ;
+        rb[q] = X > kb ? S[(int64_t)(kb + r) * npad + X + c] : S[(int64_t)(X + r) * npad + kb + c];
+        ra[q] = inner ? (I < kb ? S[(int64_t)(I + r) * npad + kb + c] : S[(int64_t)(kb + r) * npad + I + c]) : 0.0;
+    }
+    for (int k = 0; k < 16; ++k) {
+        double(&R)[4][kGJ] = sR[k & 1], (&C)[4][kGJ] = sC[k & 1];
+        if (ty == k)
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) R[a][4 * tx + b] = m[a][b];
+        if (tx == k)
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) C[b][4 * ty + a] = m[a][b];
+        __syncthreads();
+        double Q[4][4], c4[4][4];
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                Q[a][b] = R[a][4 * k + b];
+                c4[a][b] = C[b][4 * ty + a];
+            }
+        gj_pair<0>(Q);
+        gj_pair<2>(Q);
+        // the pivot columns take the same form with W = Q and nothing to
+        // subtract from
+        const bool pr = ty == k, pc = tx == k;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            double x[4], w[4];
+#pragma unroll
+            for (int a = 0; a < 4; ++a) x[a] = R[a][4 * tx + b];
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const double v = Q[a][0] * x[0] + Q[a][1] * x[1] + Q[a][2] * x[2] + Q[a][3] * x[3];
+                w[a] = pc ? Q[a][b] : v;
+            }
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const double u = c4[a][0] * w[0] + c4[a][1] * w[1] + c4[a][2] * w[2] + c4[a][3] * w[3];
+                m[a][b] = pr ? w[a] : (pc ? 0.0 : m[a][b]) - u;
+            }
+        }
+    }
+    if (I == kb && J == kb) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) T[(int64_t)(kb + 4 * ty + a) * npad + kb + 4 * tx + b] = -m[a][b];
+        return;
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) sP[4 * ty + a][4 * tx + b] = m[a][b];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int r = (t + 256 * q) / kGJ, c = t % kGJ;
+        if (X > kb) sB[r][c] = rb[q];
+        else sB[c][r] = rb[q];
+        if (I < kb) sA[r][c] = ra[q];
+        else sA[c][r] = ra[q];
+    }
+    __syncthreads();
+    const int w = t / kWave, lane = t % kWave;
+    const int r0 = (w / 2) * 32, c0 = (w % 2) * 32, li = lane % 16, lk = lane / 16;
+    gj_d4 acc[2][2];
+    gj_product(sP, sB, r0, c0, li, lk, acc);
+    __syncthreads();
+    // W into LDS, for J = k as the transpose: the tile M'[I][k]
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int v = 0; v < 2; ++v)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int row = I + r0 + 16 * u + lk + 4 * q, col = J + c0 + 16 * v + li;
-                D[(int64_t)row * npad + col] -= acc[u][v][q];
+                const int row = r0 + 16 * u + lk + 4 * q, col = c0 + 16 * v + li;
+                if (J == kb) sB[col][row] = acc[u][v][q];
+                else sB[row][col] = acc[u][v][q];
+            }
+    __syncthreads();
+    if (!inner) {
+        for (int i = t; i < kGJ * kGJ; i += 256) T[(int64_t)(I + i / kGJ) * npad + J + i % kGJ] = sB[i / kGJ][i % kGJ];
+        return;
+    }
+    gj_product(sA, sB, r0, c0, li, lk, acc);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int64_t at = (int64_t)(I + r0 + 16 * u + lk + 4 * q) * npad + J + c0 + 16 * v + li;
+                T[at] = S[at] - acc[u][v][q];
             }
 }
 
-// panels of the swept block: M'[I][k] = W[I]^T (I < k), M'[k][J] = W[J]
-// (J > k), M'[k][k] = -B^-1
-__global__ __launch_bounds__(256) void k_gj_panels(double *__restrict__ D, int npad, int kb,
-                                                   const double *__restrict__ W, const double *__restrict__ Pinv)
-{
-    const int I = blockIdx.x * kGJ;
-    const int t = threadIdx.x;
-    if (I < kb) {
-        // D[I][k] = W[I]^T through LDS, rows read and written contiguously
-        __shared__ double sT[kGJ][kGJ + 1];
-        for (int i = t; i < kGJ * kGJ; i += 256) sT[i / kGJ][i % kGJ] = W[(int64_t)(i / kGJ) * npad + I + i % kGJ];
-        __syncthreads();
-        for (int i = t; i < kGJ * kGJ; i += 256) {
-            const int r = i / kGJ, c = i % kGJ;
-            D[(int64_t)(I + r) * npad + kb + c] = sT[c][r];
-        }
-        return;
-    }
-    for (int i = t; i < kGJ * kGJ; i += 256) {
-        const int r = i / kGJ, c = i % kGJ;
-        if (I == kb) D[(int64_t)(kb + r) * npad + kb + c] = -Pinv[i];
-        else D[(int64_t)(kb + r) * npad + I + c] = W[(int64_t)r * npad + I + c];
-    }
-}
-
-// A^-1 = -M: negate the upper tiles and mirror them into the lower ones
-__global__ __launch_bounds__(256) void k_gj_finish(double *__restrict__ D, int npad)
+// A^-1 = -M: negate the upper tiles of S and mirror them into the lower ones of
+// D (may be S)
+__global__ __launch_bounds__(256) void k_gj_finish(const double *S, double *D, int npad)
 {
     const int I = blockIdx.y * kGJ, J = blockIdx.x * kGJ;
     if (I > J) return;
     __shared__ double sT[kGJ][kGJ + 1];
     const int t = threadIdx.x;
-    for (int i = t; i < kGJ * kGJ; i += 256) sT[i / kGJ][i % kGJ] = -D[(int64_t)(I + i / kGJ) * npad + J + i % kGJ];
+    for (int i = t; i < kGJ * kGJ; i += 256) sT[i / kGJ][i % kGJ] = -S[(int64_t)(I + i / kGJ) * npad + J + i % kGJ];
     __syncthreads();
     for (int i = t; i < kGJ * kGJ; i += 256) {
         const int r = i / kGJ, c = i % kGJ;
@@ -654,7 +688,7 @@ __global__ void k_gjb_take_block(const double *__restrict__ D, int npad, int kb,
 // MODE 1 (update): D[I][J] -= sum_c M[I][kb + 64 c + .] W[64 c + .][J]
 //   (grid: column tiles x row tiles, upper tiles outside the block)
 // Each 64 x 64 output tile accumulates the four 64-deep chunks on the FP64
-// matrix cores (the operand layout of k_gj_update) and is written once.
+// matrix cores (the operand layout of gj_product) and is written once.
 template <int MODE>
 __global__ __launch_bounds__(256) void k_gjb_gemm(double *__restrict__ D, int npad, int kb,
                                                   const double *__restrict__ Binv, double *__restrict__ W)
@@ -925,18 +959,16 @@ hipError_t launch_coarsen(int d, int p, const PatchDev *cpatches, const PatchDev
     return hipErrorInvalidValue;
 }
 
-// the 64-block symmetric sweep of the npad x npad matrix D (M = -A^-1 on
-// the upper tiles)
-static void gj_sweep64(double *D, int npad, double *W, double *Pinv, hipStream_t s)
+// the 64-block symmetric sweep of the npad x npad matrix D (M = -A^-1 on the
+// upper tiles), in turns between D and E; returns the one that holds M
+static double *gj_sweep64(double *D, double *E, int npad, hipStream_t s)
 {
     const int nb = npad / kGJ;
     for (int k = 0; k < nb; ++k) {
-        const int kb = k * kGJ;
-        hipLaunchKernelGGL(k_gj_pivot, dim3(1), dim3(kPivThreads), 0, s, D, npad, kb, Pinv);
-        hipLaunchKernelGGL(k_gj_rowpanel, dim3(nb), dim3(256), 0, s, D, npad, kb, Pinv, W);
-        hipLaunchKernelGGL(k_gj_update, dim3(nb, nb), dim3(256), 0, s, D, npad, kb, W);
-        hipLaunchKernelGGL(k_gj_panels, dim3(nb), dim3(256), 0, s, D, npad, kb, W, Pinv);
+        hipLaunchKernelGGL(k_gj_step, dim3(nb, nb), dim3(256), 0, s, D, E, npad, k * kGJ);
+        std::swap(D, E);
     }
+    return D;
 }
 
 int dense_inverse_npad(int n)
@@ -947,8 +979,8 @@ int dense_inverse_npad(int n)
 
 int64_t dense_inverse_work_doubles(int npad)
 {
-    if (npad <= kGJB) return (int64_t)kGJ * npad + kGJ * kGJ;
-    return (int64_t)kGJB * npad + kGJB * kGJB + kGJ * kGJB + kGJ * kGJ;
+    if (npad <= kGJB) return (int64_t)npad * npad;
+    return (int64_t)kGJB * npad + 2 * kGJB * kGJB;
 }
 
 hipError_t launch_dense_inverse(int n, int npad, const int *rp, const int *ci, const double *v, double *D,
@@ -957,22 +989,23 @@ hipError_t launch_dense_inverse(int n, int npad, const int *rp, const int *ci, c
     hipLaunchKernelGGL(k_dense_fill, g1((int64_t)npad * npad), dim3(256), 0, s, n, npad, D);
     if (n > 0) hipLaunchKernelGGL(k_dense_scatter, g1(n), dim3(256), 0, s, n, npad, rp, ci, v, D);
     const int nb = npad / kGJ;
+    double *M = D;
     if (npad <= kGJB) {
-        gj_sweep64(D, npad, work, work + (int64_t)kGJ * npad, s);
+        M = gj_sweep64(D, work, npad, s);
     } else {
-        double *W = work, *Bb = W + (int64_t)kGJB * npad, *Wi = Bb + kGJB * kGJB, *Pi = Wi + kGJ * kGJB;
+        double *W = work, *Bb = W + (int64_t)kGJB * npad, *Be = Bb + kGJB * kGJB;
         const int nbb = kGJB / kGJ;
         for (int kb = 0; kb < npad; kb += kGJB) {
             // B^-1 of the pivot block on its own copy
             hipLaunchKernelGGL(k_gjb_take_block, g1(kGJB * kGJB), dim3(256), 0, s, D, npad, kb, Bb);
-            gj_sweep64(Bb, kGJB, Wi, Pi, s);
-            hipLaunchKernelGGL(k_gj_finish, dim3(nbb, nbb), dim3(256), 0, s, Bb, kGJB);
+            double *Bm = gj_sweep64(Bb, Be, kGJB, s);
+            hipLaunchKernelGGL(k_gj_finish, dim3(nbb, nbb), dim3(256), 0, s, Bm, Bb, kGJB);
             hipLaunchKernelGGL(k_gjb_gemm<0>, dim3(nb, nbb), dim3(256), 0, s, D, npad, kb, Bb, W);
             hipLaunchKernelGGL(k_gjb_gemm<1>, dim3(nb, nb), dim3(256), 0, s, D, npad, kb, Bb, W);
             hipLaunchKernelGGL(k_gjb_panels, dim3(nb, nbb), dim3(256), 0, s, D, npad, kb, W, Bb);
         }
     }
-    hipLaunchKernelGGL(k_gj_finish, dim3(nb, nb), dim3(256), 0, s, D, npad);
+    hipLaunchKernelGGL(k_gj_finish, dim3(nb, nb), dim3(256), 0, s, M, D, npad);
     return hipGetLastError();
 }
 

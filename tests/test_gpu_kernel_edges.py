@@ -333,3 +333,24 @@ def test_row_patterns(ctx, d, p, n, g, sides):
     assert np.array_equal(ci, np.concatenate([sorted(w) for w in want]) if gp.nfree else [])
     for o in (A, b, gp):
         o.close()
+
+
+# dense inverse: below, at and above the 64 tiles and the 256 pivot blocks, odd
+# and even numbers of sweeps
+@pytest.mark.parametrize("n", [(2, 2), (8, 10), (9, 9), (6, 14), (4, 44), (13, 17), (17, 17), (2, 258), (17, 33),
+                               (25, 26), (34, 41)])
+def test_dense_coarse_inverse(ctx, n):
+    """A one-level multigrid applies the inverse of its matrix."""
+    prob = _noisy_box(2, 1, n)
+    gp = gsx.Problem(ctx, prob)
+    A, b = gp.assemble(gsx.PATTERN_FULL)
+    M = A.to_scipy().toarray()
+    mg = gsx.Multigrid(gp, A, 1, 1, 1, 1.0)
+    r = np.random.default_rng(3).standard_normal(gp.nfree)
+    rd, zd = ctx.to_device(r), ctx.array(gp.nfree)
+    mg.apply(rd, zd)
+    z, zs = zd.download(), np.linalg.solve(M, r)
+    # Gauss-Jordan on an SPD matrix: n eps cond
+    assert np.linalg.norm(z - zs) <= 1.2e-16 * max(16, gp.nfree) * np.linalg.cond(M) * np.linalg.norm(zs)
+    for o in (mg, rd, zd, A, b, gp):
+        o.close()
