@@ -369,4 +369,16 @@ hipError_t launch_sf2_gather(int p, const PatchDev *patches, const int *occ_ptr,
                              const double *raw, const double *rawf, double *val, double *rhs, int maxrow,
                              const double *fixed, int *err, hipStream_t s);
 
+// Galerkin product of raw rows: per patch of a group its first blocks in the two
+// kernels, the offset of its half-contracted lines and of its transfers
+// T[I][k] (p + 2 weights per coarse function) along x and y.
+struct Sf2Coarse {
+    int64_t bx, by, m_off, tx, ty;
+    int patch;
+};
+void sf2_galerkin_sizes(int p, const int *fnb, const int *cnb, int64_t *mid, int64_t *bx, int64_t *by);
+hipError_t launch_sf2_galerkin(int p, const PatchDev *cpatches, const PatchDev *fpatches, const Sf2Coarse *meta,
+                               int ng, int64_t nbx, int64_t nby, const double *T, const double *raw, double *mid,
+                               double *craw, hipStream_t s);
+
 }  // namespace gsx

@@ -292,7 +292,7 @@ struct gsx_problem {
     DevPtr d_fixed, d_neu;
     // element matrices of the last assembly (GSX_ASM_KEEP_ELEMENTS), laid
     // out at kmat_off, and the serial of that assembly
-    DevPtr kept_K;
+    DevPtr kept_K, kept_raw;   // element matrices, or raw rows of 2D patches
     uint64_t asm_serial = 0, kept_serial = 0;
     bool zero_kappa = false;        // some element has kappa exactly 0
     bool odd_glue = false;          // an interface joins a patch to itself or to one of another degree
@@ -1041,6 +1041,14 @@ struct gsx_matrix {
     std::vector<double> hist;
 };
 
+// 2D patches whose rows are assembled by sum factorisation
+static bool sf2_rows_ok(const gsx_problem *P)
+{
+    bool ok = P->d == 2 && !P->geo && !P->zero_kappa && !P->odd_glue;
+    for (const Group &g : P->groups) ok = ok && gsx::sf2_supported(g.p);
+    return ok;
+}
+
 static gsx_status pattern_build(gsx_problem *P)
 {
     gsx_ctx *c = P->ctx;
@@ -1126,6 +1134,7 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
     mode &= ~(GSX_ASM_REBUILD_PATTERN | GSX_ASM_CSR_ONLY | GSX_ASM_KEEP_ELEMENTS | GSX_ASM_ELEMENTWISE |
               GSX_ASM_ROWWISE);
     P->kept_K.reset();
+    P->kept_raw.reset();
     const uint64_t serial = ++P->asm_serial;
     if (!P->have_pattern || rebuild) {
         gsx_status st = pattern_build(P);
@@ -1150,9 +1159,7 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
     }
     // 2D patches of degrees 2 to 4: sum-factorised rows likewise (a row of a
     // patch glued to itself could meet a column twice in its window)
-    bool use_sf2 = P->d == 2 && P->nfree > 0 && !(elementwise_asked || P->geo) && !keep_elements &&
-                   !P->zero_kappa && !P->odd_glue;
-    for (const Group &g : P->groups) use_sf2 = use_sf2 && gsx::sf2_supported(g.p);
+    const bool use_sf2 = P->nfree > 0 && !elementwise_asked && sf2_rows_ok(P);
     const bool use_sf = single && !elementwise && !keep_elements && !P->zero_kappa && P->hp[0].d == 3 &&
                         P->hp[0].p[0] == P->hp[0].p[1] && P->hp[0].p[0] == P->hp[0].p[2] &&
                         gsx::sf_supported(3, P->hp[0].p[0]);
@@ -1365,7 +1372,10 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
     }
     // element matrices go back to the cache once the gathers have run, or
     // stay with the problem when asked for and formed in one pass
-    if (keep_elements && kcap == P->kdoubles) {
+    if (keep_elements && use_sf2) {
+        P->kept_raw = std::move(raw2);
+        P->kept_serial = serial;
+    } else if (keep_elements && kcap == P->kdoubles) {
         P->kept_K = std::move(Kbuf);
         P->kept_serial = serial;
     }
@@ -2975,7 +2985,10 @@ static gsx_status mg_sell(gsx_mg *mg, int l)
     hipStream_t s = c->stream;
     MGLevel &V = mg->L[l];
     const bool mixed = mg->precision == GSX_MIXED, finest = l == (int)mg->L.size() - 1;
-    if (V.n <= 0 || V.nnz <= 0) return GSX_OK;
+    // below 2^18 entries forming the slices costs more than a solve gains by
+    // them (2 x 2 patches of 28^2 elements p = 2, 78 K entries: set-up and solve
+    // 2.7 ms with slices, 2.5 without; from 3 M entries a step is twice as fast)
+    if (V.n <= 0 || V.nnz < (1 << 18)) return GSX_OK;
     const int nsl = (V.n + 63) / 64;
     DevPtr width = dalloc(c, sizeof(int) * nsl);
     if (!width) return fail(c, GSX_ERR_OOM, "device allocation (level slices)");
@@ -3096,6 +3109,57 @@ struct TransferCache {
         return items.back().T;
     }
 };
+
+// Raw rows of cp's functions from those of fp's (launch_sf2_galerkin).
+static gsx_status mg_galerkin_raw(gsx_ctx *c, gsx_problem *fp, gsx_problem *cp, TransferCache &tc, const double *Rf,
+                                  DevPtr &Rc)
+{
+    hipStream_t s = c->stream;
+    std::vector<double> T;
+    std::vector<gsx::Sf2Coarse> meta;
+    std::vector<int64_t> nbx, nby;
+    int64_t mid = 0;
+    for (const Group &g : cp->groups) {
+        int64_t bx = 0, by = 0;
+        for (int k : g.patches) {
+            int64_t to[2], m, x, y;
+            for (int j = 0; j < 2; ++j) {
+                int nf1 = 0, nc1 = 0;
+                const std::vector<double> &Tm =
+                    tc.get(cp->knots_h[(size_t)3 * k + j], fp->knots_h[(size_t)3 * k + j], g.p, nf1, nc1);
+                to[j] = (int64_t)T.size();
+                for (int I = 0; I < nc1; ++I)
+                    for (int q = 0; q < g.p + 2; ++q) {
+                        const int i = 2 * I - g.p + q;
+                        T.push_back(i >= 0 && i < nf1 ? Tm[(size_t)i * nc1 + I] : 0.0);
+                    }
+            }
+            gsx::sf2_galerkin_sizes(g.p, fp->hp[k].nb, cp->hp[k].nb, &m, &x, &y);
+            meta.push_back({bx, by, mid, to[0], to[1], k});
+            mid += m;
+            bx += x;
+            by += y;
+        }
+        nbx.push_back(bx);
+        nby.push_back(by);
+    }
+    Rc = dalloc(c, sizeof(double) * std::max<int64_t>(1, cp->rdoubles));
+    DevPtr d_mid = dalloc(c, sizeof(double) * std::max<int64_t>(1, mid));
+    DevPtr d_T = dalloc(c, sizeof(double) * std::max<size_t>(1, T.size()));
+    DevPtr d_meta = dalloc(c, sizeof(gsx::Sf2Coarse) * std::max<size_t>(1, meta.size()));
+    if (!Rc || !d_mid || !d_T || !d_meta) return fail(c, GSX_ERR_OOM, "device allocation (Galerkin product)");
+    HIP_OK(c, hipMemcpyAsync(d_T.get(), T.data(), sizeof(double) * T.size(), hipMemcpyHostToDevice, s));
+    HIP_OK(c, hipMemcpyAsync(d_meta.get(), meta.data(), sizeof(gsx::Sf2Coarse) * meta.size(), hipMemcpyHostToDevice, s));
+    size_t at = 0;
+    for (size_t q = 0; q < cp->groups.size(); ++q) {
+        const Group &g = cp->groups[q];
+        HIP_OK(c, gsx::launch_sf2_galerkin(g.p, dp<PatchDev>(cp->d_patches), dp<PatchDev>(fp->d_patches),
+                                           dp<gsx::Sf2Coarse>(d_meta) + at, (int)g.patches.size(), nbx[q], nby[q],
+                                           dp<double>(d_T), Rf, dp<double>(d_mid), dp<double>(Rc), s));
+        at += g.patches.size();
+    }
+    return GSX_OK;
+}
 
 // P: the knot-insertion transfer from the basis of cp to that of fp (same
 // degrees, cp's knots a subset of fp's) restricted to free DOFs, rows = fp's
@@ -3333,8 +3397,26 @@ extern "C" gsx_status gsx_mg_create(gsx_problem *fine, gsx_matrix *A, int32_t nl
         const int64_t kc = nlevels > 1 ? mg->L[nlevels - 2].prob->kdoubles : 0;
         elem_path = (fine->kdoubles + fine->fdoubles + kc) * (int64_t)sizeof(double) <= c->elem_budget;
     }
-    DevPtr Kf;
-    if (elem_path && fine->kept_K && fine->kept_serial == A->src_serial) {
+    // 2D patches of degrees 2 to 4: from raw rows instead, which are 1/8 of the
+    // element matrices' bytes at p = 3
+    const bool raw_path = elem_path && sf2_rows_ok(fine);
+    DevPtr Kf, Rf;
+    if (raw_path && fine->kept_raw && fine->kept_serial == A->src_serial) {
+        Rf = std::move(fine->kept_raw);
+    } else if (raw_path) {
+        KScope ke(c, "mg_elem");
+        Rf = dalloc(c, sizeof(double) * std::max<int64_t>(1, fine->rdoubles));
+        DevPtr Ff = dalloc(c, sizeof(double) * std::max<int64_t>(1, fine->nbasis));
+        if (!Rf || !Ff) return fail(c, GSX_ERR_OOM, "device allocation (row assembly)");
+        int64_t ndet = 0;
+        for (const Group &g : fine->groups) {
+            HIP_OK(c, gsx::launch_sf2_rows(g.p, dp<PatchDev>(fine->d_patches), dp<int>(g.d_gpatch),
+                                           dp<int64_t>(g.d_rprefix), (int)g.patches.size(), g.rprefix.back(),
+                                           g.rows_cy, c->gt, dp<double>(Rf), dp<double>(Ff),
+                                           dp<double>(fine->d_detmin) + ndet, s));
+            ndet += g.rprefix.back();
+        }
+    } else if (elem_path && fine->kept_K && fine->kept_serial == A->src_serial) {
         Kf = std::move(fine->kept_K);   // this matrix's own element matrices
     } else if (elem_path) {
         KScope ke(c, "mg_elem");
@@ -3355,7 +3437,7 @@ extern "C" gsx_status gsx_mg_create(gsx_problem *fine, gsx_matrix *A, int32_t nl
         gsx_problem *cp = C.prob;
         std::vector<double> tblk;
         std::vector<int64_t> toff;
-        GSX_TRY(mg_knot_transfer(c, fp, cp, F.n, C, tcache, elem_path ? &tblk : nullptr, &toff));
+        GSX_TRY(mg_knot_transfer(c, fp, cp, F.n, C, tcache, elem_path && !raw_path ? &tblk : nullptr, &toff));
         GSX_TRY(mg_transpose_transfer(c, C, F.n));
         DevPtr errf = dalloc(c, sizeof(int) * 2);
         if (!errf) return fail(c, GSX_ERR_OOM, "device allocation (transfer)");
@@ -3366,7 +3448,18 @@ extern "C" gsx_status gsx_mg_create(gsx_problem *fine, gsx_matrix *A, int32_t nl
         C.lpr = gsx::spmv_lpr(C.n ? (double)C.nnz / C.n : 1.0);
         C.val = dalloc(c, sizeof(double) * std::max<int64_t>(1, C.nnz));
         if (!C.val) return fail(c, GSX_ERR_OOM, "device allocation (Galerkin product)");
-        if (elem_path) {
+        if (raw_path) {
+            // coarse raw rows from the fine ones, then the coarse rows from them
+            KScope kg(c, "mg_galerkin");
+            DevPtr Rc;
+            GSX_TRY(mg_galerkin_raw(c, fp, cp, tcache, dp<double>(Rf), Rc));
+            for (const Group &g : cp->groups)
+                HIP_OK(c, gsx::launch_sf2_gather(g.p, dp<PatchDev>(cp->d_patches), dp<int>(cp->d_occ_ptr),
+                                                 dp<int>(cp->d_occ_patch), dp<int64_t>(cp->d_occ_local), C.n,
+                                                 dp<int>(C.rowptr), dp<int>(C.col), dp<double>(Rc), nullptr,
+                                                 dp<double>(C.val), nullptr, cp->maxrow, nullptr, dp<int>(errf), s));
+            Rf = std::move(Rc);
+        } else if (elem_path) {
             // coarse element matrices from the children's, then the coarse gather
             KScope kg(c, "mg_galerkin");
             DevPtr Kc = dalloc(c, sizeof(double) * std::max<int64_t>(1, cp->kdoubles));

@@ -45,7 +45,8 @@ typedef enum {
                                         solves only, e.g. batched members)    */
     GSX_ASM_KEEP_ELEMENTS = 0x400,   /* flag: the problem keeps this assembly's
                                         element matrices (when they were formed
-                                        in one pass) until its next assembly;
+                                        in one pass; of 2D patches assembled by
+                                        rows, the rows) until its next assembly;
                                         gsx_mg_create on the returned matrix
                                         takes them instead of recomputing      */
     GSX_ASM_ELEMENTWISE = 0x800,     /* flag: element matrices + row gather
@@ -262,7 +263,7 @@ gsx_status gsx_assemble_bdr(gsx_problem *prob, double *rhs_dev);
  * elements: values agree with the element path to rounding).  There no
  * entry is dropped by the exact-zero rule: an entry with only exact-zero
  * element contributions needs kappa = 0 on every element they share.  Other
- * problems, GSX_ASM_KEEP_ELEMENTS and GSX_ASM_ELEMENTWISE take the element
+ * problems, 3D ones with GSX_ASM_KEEP_ELEMENTS, and GSX_ASM_ELEMENTWISE take the element
  * path. */
 gsx_status gsx_assemble(gsx_problem *prob, int32_t pattern_mode,
                         int32_t precision, gsx_matrix **A_out,

@@ -154,11 +154,12 @@ def test_csr_products(ctx, n, lo, hi):
         o.close()
 
 
-# level operators in slices of 64 rows: several slices per wave block, four
+# level operators in slices of 64 rows from 2^18 entries up (CSR rows below):
+# several slices per wave block, four
 # waves per slice below 131,072 rows, uniform slices (inside a patch), a last
 # slice of one row, interface rows; against the cycle written out in scipy
 @pytest.mark.parametrize("gx,gy,n,p,levels", [(1, 1, 16, 2, 2), (2, 1, 12, 3, 2), (3, 2, 24, 3, 3), (2, 2, 8, 4, 2),
-                                              (1, 1, 374, 2, 2)])
+                                              (1, 1, 374, 2, 2), (2, 2, 60, 2, 3), (1, 1, 82, 3, 2), (2, 1, 52, 4, 2)])
 @pytest.mark.parametrize("prec", [gsx.FP64, gsx.MIXED])
 def test_multigrid_level_slices(ctx, gx, gy, n, p, levels, prec):
     prob = problems.square_grid(gx, gy, n, p)
@@ -353,4 +354,31 @@ def test_dense_coarse_inverse(ctx, n):
     # Gauss-Jordan on an SPD matrix: n eps cond
     assert np.linalg.norm(z - zs) <= 1.2e-16 * max(16, gp.nfree) * np.linalg.cond(M) * np.linalg.norm(zs)
     for o in (mg, rd, zd, A, b, gp):
+        o.close()
+
+
+# Galerkin levels from raw rows: one element per direction on the coarsest
+# level, lines ending inside a block, interfaces, several levels
+@pytest.mark.parametrize("p,n,g,levels", [(2, (2, 2), (1, 1), 2), (3, (2, 8), (1, 1), 2), (4, (4, 2), (1, 1), 2),
+                                          (2, (36, 132), (1, 1), 3), (3, (8, 4), (2, 3), 3), (4, (12, 20), (2, 2), 3)])
+@pytest.mark.parametrize("keep", [0, gsx.ASM_KEEP_ELEMENTS])
+def test_galerkin_rows(ctx, p, n, g, levels, keep):
+    """Every level's operator is P^T A P of the next finer one."""
+    prob = _glued_boxes(2, p, n, g)
+    for k, P in enumerate(prob.patches):
+        problems.perturb_interior(P, 0.1 / max(n), 50 + k)
+        P.kappa = problems.lognormal_kappa(P.nelem, 0.5, 60 + k)
+    gp = gsx.Problem(ctx, prob)
+    A, b = gp.assemble(gsx.PATTERN_FULL | keep)
+    mg = gsx.Multigrid(gp, A, levels, 1, 1, 0.7)
+    M = A.to_scipy()
+    for l in range(levels - 2, -1, -1):
+        Ac, P = mg.level(l)[:2]
+        want = (P.T @ M @ P).tocsr()
+        # (p + 2)^4 weighted terms per entry, weights at most 1
+        D = abs(Ac - want)
+        assert D.max() <= 1e-13 * (p + 2) ** 2 * abs(want).max()
+        assert (Ac != Ac.T).nnz == 0
+        M = Ac
+    for o in (mg, A, b, gp):
         o.close()
