@@ -115,7 +115,15 @@ __device__ inline void csr_rows(int n, const int *__restrict__ rowptr, const int
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
             const int e = min(kb - c0, m);
-            for (int o = max(ka - c0, 0) + lane % L; o < e; o += L) acc += buf[o];
+            // two sums a lane: half the chain, and half its rounding
+            Acc half = 0;
+            int o = max(ka - c0, 0) + lane % L;
+            for (; o + L < e; o += 2 * L) {
+                acc += buf[o];
+                half += buf[o + L];
+            }
+            if (o < e) acc += buf[o];
+            acc += half;
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
             if (k1 - c0 <= kCsrCap) break;

@@ -31,8 +31,12 @@ __global__ __launch_bounds__(256) void k_sell_width(int n, const int *__restrict
 }
 
 // A block per slice: columns (or, uniform slices, offsets) and values.  The
-// rows are taken 16 at a time through LDS, so the CSR arrays are read and the
-// slices written coalesced; longer rows are copied entry by entry.
+// values go through LDS, as many rows at a time as fit (all 64 up to 64 entries
+// each), so the CSR array is read and the slice written coalesced; longer rows
+// are copied entry by entry.  Whether a slice is uniform is tested over its
+// entries as one range, all loads independent; only other slices read their
+// columns again.  Bound by the bytes: 1.06 M rows of
+// 49 entries 374 us (16 rows at a time with their columns, row by row tests: 780).
 constexpr int kSellLds = 4096;
 template <typename VO>
 __global__ __launch_bounds__(256) void k_sell_fill(int n, const int *__restrict__ rowptr, const int *__restrict__ col,
@@ -41,50 +45,46 @@ __global__ __launch_bounds__(256) void k_sell_fill(int n, const int *__restrict_
                                                    VO *__restrict__ sval, double *__restrict__ sval64)
 {
     __shared__ double sv[kSellLds];
-    __shared__ int sc[kSellLds];
-    __shared__ int bad;
+    __shared__ int srp[65];
     const int sl = blockIdx.x, t = threadIdx.x, r0 = sl * 64, nr = min(64, n - r0);
     const int K = sptr[sl + 1] - sptr[sl];
     const int64_t base = (int64_t)sptr[sl] * 64;
-    if (t == 0) bad = nr < 64;
+    if (t < 65) srp[t] = rowptr[r0 + min(t, nr)];
     __syncthreads();
     // uniform: every row has K entries at the first row's offsets
-    const int a0 = rowptr[r0];
-    for (int i = t / 64; i < nr; i += 4) {
-        const int a = rowptr[r0 + i], len = rowptr[r0 + i + 1] - a;
-        bool ok = len == K;
-        for (int k = t & 63; ok && k < K; k += 64) ok = col[a + k] - i == col[a0 + k];
-        if (!ok) bad = 1;
+    const int a0 = srp[0];
+    int bad = nr < 64 || (t < 64 && srp[t + 1] - srp[t] != K);
+    bad = __syncthreads_count(bad);
+    if (!bad) {
+        int off = 0;
+#pragma unroll 4
+        for (int e = t; e < 64 * K; e += 256) {
+            const int i = e / K;
+            off |= col[a0 + e] - i - col[a0 + e - i * K];
+        }
+        bad = __syncthreads_count(off != 0);
     }
-    __syncthreads();
     const int uni = !bad;
     if (t == 0) uniform[sl] = uni;
     if (uni)
         for (int k = t; k < K; k += 256) scol[base + k] = col[a0 + k] - r0;
-    const bool lds = 16 * K <= kSellLds;
-    for (int q = 0; q < 64; q += 16) {
-        const int b0 = q < nr ? rowptr[r0 + q] : 0, b1 = q < nr ? rowptr[r0 + min(q + 16, nr)] : 0;
+    const int sh = 64 * K <= kSellLds ? 6 : 32 * K <= kSellLds ? 5 : 4, R = 1 << sh;   // rows at a time
+    const bool lds = R * K <= kSellLds;
+    for (int q = 0; q < 64; q += R) {
+        const int b0 = srp[q], b1 = srp[q + R];
         if (lds) {
             __syncthreads();
-            for (int k = b0 + t; k < b1; k += 256) {
-                sv[k - b0] = val[k];
-                sc[k - b0] = col[k];
-            }
+            for (int k = b0 + t; k < b1; k += 256) sv[k - b0] = val[k];
             __syncthreads();
         }
-        const int i = q + t % 16;
-        const int ra = i < nr ? rowptr[r0 + i] : 0, len = i < nr ? rowptr[r0 + i + 1] - ra : 0;
-        for (int k = t / 16; k < K; k += 16) {
-            double v = 0.0;
-            int cc = min(r0 + i, n - 1);
-            if (k < len) {
-                v = lds ? sv[ra + k - b0] : val[ra + k];
-                cc = lds ? sc[ra + k - b0] : col[ra + k];
-            }
+        const int i = q + (t & (R - 1));
+        const int ra = srp[i], len = srp[i + 1] - ra;   // 0 beyond the last row
+        for (int k = t >> sh; k < K; k += 256 >> sh) {
             const int64_t at = base + (int64_t)k * 64 + i;
+            const double v = k < len ? (lds ? sv[ra + k - b0] : val[ra + k]) : 0.0;
             sval[at] = (VO)v;
             if (sval64) sval64[at] = v;
-            if (!uni) scol[at] = cc;
+            if (!uni) scol[at] = k < len ? col[ra + k] : min(r0 + i, n - 1);
         }
     }
 }
@@ -100,6 +100,15 @@ __device__ inline double sell_sum(const SellOp &S, const V *__restrict__ sval, c
     const int *c = S.col + (int64_t)p0 * 64;
     double acc = 0.0;
     constexpr int U = 8;
+    // eight products in a tree: a row's sum rounds through a chain of K / 8
+    // chunks, not of K products
+    auto chunk = [](const V *a, const double *q) {
+        double h[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) h[u] = (double)a[u] * q[u] + (double)a[u + 4] * q[u + 4];
+        return (h[0] + h[1]) + (h[2] + h[3]);
+    };
+    double q[U];
     int k = part;
     if (S.uniform[sl]) {
         const T *xr = x + r;
@@ -112,7 +121,8 @@ __device__ inline double sell_sum(const SellOp &S, const V *__restrict__ sval, c
                 b[u] = xr[c[k + u * step]];
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u) acc += (double)a[u] * (double)b[u];
+            for (int u = 0; u < U; ++u) q[u] = (double)b[u];
+            acc += chunk(a, q);
         }
         for (; k < K; k += step) acc += (double)v[(int64_t)k * 64] * (double)xr[c[k]];
     } else {
@@ -126,7 +136,8 @@ __device__ inline double sell_sum(const SellOp &S, const V *__restrict__ sval, c
                 j[u] = c[(int64_t)(k + u * step) * 64];
             }
 #pragma unroll
-            for (int u = 0; u < U; ++u) acc += (double)a[u] * (double)x[j[u]];
+            for (int u = 0; u < U; ++u) q[u] = (double)x[j[u]];
+            acc += chunk(a, q);
         }
         for (; k < K; k += step) acc += (double)v[(int64_t)k * 64] * (double)x[c[(int64_t)k * 64]];
     }
