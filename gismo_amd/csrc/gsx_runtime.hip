@@ -285,6 +285,7 @@ struct gsx_problem {
     int box_lo[3] = {0, 0, 0}, box_hi[3] = {0, 0, 0};   // free functions per direction
     // element scratch
     DevPtr d_detmin, d_scan_bsum, d_scan_total;
+    int64_t ndet = 1;   // determinant minima of an assembly: one per element or per block of a row assembly
     int64_t kdoubles = 0, fdoubles = 0, rdoubles = 0;
     double min_det = 0.0;
     // boundary data: values of the eliminated DOFs (global index - nfree;
@@ -844,6 +845,13 @@ gsx_status gsx_problem_create(gsx_ctx *c, int32_t npatch, const gsx_patch_desc *
                                  hipMemcpyHostToDevice, s));
     }
 
+    // patches of few elements have more blocks of the 2D row assembly (which
+    // count rows of functions) than elements
+    int64_t row_blocks = 0;
+    for (const Group &g : P->groups) row_blocks += g.rprefix.empty() ? 0 : g.rprefix.back();
+    P->ndet = std::max({int64_t(1), P->nelem, row_blocks});
+    if (P->d == 3) P->ndet = std::max(P->ndet, gsx::sf_det_count(P->hp[0].p[0], P->hp[0].nel));
+
     // occurrences of every free DOF (patch order, then local order)
     std::vector<int> occ_cnt(nfree + 1, 0);
     for (int64_t i = 0; i < P->nbasis; ++i)
@@ -1049,6 +1057,23 @@ static bool sf2_rows_ok(const gsx_problem *P)
     return ok;
 }
 
+// Raw rows and their loads (launch_sf2_rows) of every patch; ndet: the
+// determinant minima written to d_detmin, one per block.
+static gsx_status sf2_assemble_rows(gsx_problem *P, double *raw, double *rawf, int64_t *ndet)
+{
+    gsx_ctx *c = P->ctx;
+    *ndet = 0;
+    for (const Group &g : P->groups) {
+        if (*ndet + g.rprefix.back() > P->ndet)
+            return fail(c, GSX_ERR_ARG, "row assembly: more blocks than determinant minima");
+        HIP_OK(c, gsx::launch_sf2_rows(g.p, dp<PatchDev>(P->d_patches), dp<int>(g.d_gpatch),
+                                       dp<int64_t>(g.d_rprefix), (int)g.patches.size(), g.rprefix.back(), g.rows_cy,
+                                       c->gt, raw, rawf, dp<double>(P->d_detmin) + *ndet, c->stream));
+        *ndet += g.rprefix.back();
+    }
+    return GSX_OK;
+}
+
 static gsx_status pattern_build(gsx_problem *P)
 {
     gsx_ctx *c = P->ctx;
@@ -1144,7 +1169,7 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
         return fail(c, GSX_ERR_ARG, "rows longer than 1024 entries are not supported");
     const bool single = P->npatch == 1 && P->d_f2g && P->nfree > 0;
     if (!P->d_detmin) {
-        P->d_detmin = dalloc(c, sizeof(double) * (std::max<int64_t>(1, P->nelem) + 260));
+        P->d_detmin = dalloc(c, sizeof(double) * (P->ndet + 260));   // then launch_min's slots
         if (!P->d_detmin) return fail(c, GSX_ERR_OOM, "device allocation (Jacobian check)");
     }
     // single 3D patch: sum-factorised rows, no element matrices
@@ -1206,13 +1231,7 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
         if (!raw2 || !err2) return fail(c, GSX_ERR_OOM, "device allocation (row assembly)");
         KScope k(c, "sf_assemble");
         HIP_OK(c, hipMemsetAsync(err2.get(), 0, sizeof(int), s));
-        for (const Group &g : P->groups) {
-            HIP_OK(c, gsx::launch_sf2_rows(g.p, dp<PatchDev>(P->d_patches), dp<int>(g.d_gpatch),
-                                           dp<int64_t>(g.d_rprefix), (int)g.patches.size(), g.rprefix.back(),
-                                           g.rows_cy, c->gt, dp<double>(raw2), dp<double>(Fbuf),
-                                           dp<double>(P->d_detmin) + ndet2, s));
-            ndet2 += g.rprefix.back();
-        }
+        GSX_TRY(sf2_assemble_rows(P, dp<double>(raw2), dp<double>(Fbuf), &ndet2));
     } else if (!single && P->geo) {
         KScope k(c, "geo_elem");
         for (int ip = 0; ip < P->npatch; ++ip)
@@ -1381,7 +1400,7 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
     }
     Kbuf.reset();
     Fbuf.reset();
-    double *dmin_slot = dp<double>(P->d_detmin) + std::max<int64_t>(1, P->nelem);
+    double *dmin_slot = dp<double>(P->d_detmin) + P->ndet;
     HIP_OK(c, gsx::launch_min(dp<double>(P->d_detmin),
                               use_sf    ? gsx::sf_det_count(h0.p[0], h0.nel)
                               : use_sf2 ? ndet2
@@ -3409,13 +3428,7 @@ extern "C" gsx_status gsx_mg_create(gsx_problem *fine, gsx_matrix *A, int32_t nl
         DevPtr Ff = dalloc(c, sizeof(double) * std::max<int64_t>(1, fine->nbasis));
         if (!Rf || !Ff) return fail(c, GSX_ERR_OOM, "device allocation (row assembly)");
         int64_t ndet = 0;
-        for (const Group &g : fine->groups) {
-            HIP_OK(c, gsx::launch_sf2_rows(g.p, dp<PatchDev>(fine->d_patches), dp<int>(g.d_gpatch),
-                                           dp<int64_t>(g.d_rprefix), (int)g.patches.size(), g.rprefix.back(),
-                                           g.rows_cy, c->gt, dp<double>(Rf), dp<double>(Ff),
-                                           dp<double>(fine->d_detmin) + ndet, s));
-            ndet += g.rprefix.back();
-        }
+        GSX_TRY(sf2_assemble_rows(fine, dp<double>(Rf), dp<double>(Ff), &ndet));
     } else if (elem_path && fine->kept_K && fine->kept_serial == A->src_serial) {
         Kf = std::move(fine->kept_K);   // this matrix's own element matrices
     } else if (elem_path) {

@@ -382,3 +382,40 @@ def test_galerkin_rows(ctx, p, n, g, levels, keep):
         M = Ac
     for o in (mg, A, b, gp):
         o.close()
+
+
+# patches of one element: more blocks of the row assembly (675, 800 and 768
+# determinant minima) than elements (225, 400 and 256), several blocks in the
+# reduction of the minima
+@pytest.mark.parametrize("p,g", [(4, 15), (2, 20), (3, 16)])
+def test_row_assembly_of_one_element_patches(ctx, p, g):
+    prob = problems.square_grid(g, g, 1, p)
+    for k, P in enumerate(prob.patches):
+        problems.perturb_interior(P, 0.1, 70 + k)
+    gp = gsx.Problem(ctx, prob)
+    out = []
+    for mode in (0, gsx.ASM_ELEMENTWISE):
+        A, b = gp.assemble(gsx.PATTERN_FULL | mode)
+        out.append((*A.download(), b.download()[:gp.nfree], gp.min_detj()))
+        A.close()
+        b.close()
+    r, e = out
+    assert np.array_equal(r[0], e[0]) and np.array_equal(r[1], e[1])
+    # as test_row_assembly_2d; the geometry's coordinates up to g multiply the
+    # element path's rounding of a Jacobian of size 1
+    scale = np.maximum.reduceat(np.abs(e[2]), e[0][:-1])
+    assert np.all(np.abs(r[2] - e[2]) <= 1e-12 * g * np.repeat(scale, np.diff(e[0])))
+    assert np.abs(r[3] - e[3]).max() <= 1e-12 * g * np.abs(e[3]).max()
+    assert r[4] == pytest.approx(e[4], rel=1e-12 * g)
+    gp.close()
+    # a folded patch is found wherever it lies among the blocks
+    for k in (0, g * g // 2, g * g - 1):
+        ctrl = prob.patches[k].ctrl
+        prob.patches[k].ctrl = ctrl.copy()
+        prob.patches[k].ctrl[p + 2] += 3.0   # the first interior control point
+        gp = gsx.Problem(ctx, prob)
+        with pytest.raises(gsx.GsxError) as err:
+            gp.assemble(gsx.PATTERN_FULL)
+        assert err.value.status == gsx.GSX_ERR_JACOBIAN
+        gp.close()
+        prob.patches[k].ctrl = ctrl
