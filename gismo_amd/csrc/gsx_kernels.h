@@ -80,7 +80,9 @@ hipError_t launch_min(const double *v, int64_t n, double *out, hipStream_t s);
 hipError_t launch_sum_arrays(const double *v, int narr, int64_t n, int64_t stride, double *out, hipStream_t s);
 
 // solve
+// class of a mean row length, and the lanes (8 to 64) that read a row of it
 int spmv_lpr(double avg_row);
+int spmv_lanes(int lpr);
 int spmv_blocks(int n, int lpr);
 hipError_t launch_spmv_f64(int lpr, int n, const int *rp, const int *ci, const double *v,
                            const double *x, double *y, const double *b, double *part, int mode,

@@ -4975,7 +4975,7 @@ static gsx_status batch_add(gsx_batch *B, gsx_matrix *A, int32_t row0, int32_t n
     g.tau = tau;
     g.tol = tol;
     g.maxit = maxit;
-    g.lpr = own ? 8 : gsx::spmv_lpr((double)(rp2[1] - rp2[0]) / nrows);
+    g.lpr = own ? 8 : gsx::spmv_lanes(gsx::spmv_lpr((double)(rp2[1] - rp2[0]) / nrows));
     g.row0 = row0;
     if (own) {
         const int d = box[0], p = box[1];

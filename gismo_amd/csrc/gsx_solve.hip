@@ -433,6 +433,8 @@ int spmv_lpr(double avg_row)
     return 8;
 }
 
+int spmv_lanes(int lpr) { return lpr == kCsrLong ? 64 : lpr; }
+
 int spmv_blocks(int n, int lpr) { return csr_blocks(n, lpr); }
 
 template <typename V, typename T, int MODE>
@@ -449,7 +451,7 @@ static hipError_t spmv_dispatch(int lpr, int n, const int *rowptr, const int *co
         else                                                                                                          \
             hipLaunchKernelGGL((k_spmv<LPR / 4, false, V, T, MODE>), grid, block, 0, s, n, rowptr, col, val, x, y, b, partial, st); \
         break;
-    switch (lpr == kCsrLong ? 64 : lpr) {
+    switch (spmv_lanes(lpr)) {
         GSX_L(8) GSX_L(16) GSX_L(32) GSX_L(64)
     default: return hipErrorInvalidValue;
     }
@@ -570,7 +572,7 @@ static hipError_t jacobi_dispatch(int lpr, int n, const int *rp, const int *ci, 
         else                                                                                                          \
             hipLaunchKernelGGL((k_jacobi_step<LPR / 4, false, V, T>), grid, block, 0, s, n, rp, ci, v, diag, b, xin, xout, tau); \
         break;
-    switch (lpr == kCsrLong ? 64 : lpr) {
+    switch (spmv_lanes(lpr)) {
         GSX_L(8) GSX_L(16) GSX_L(32) GSX_L(64)
     default: return hipErrorInvalidValue;
     }
@@ -612,7 +614,7 @@ static hipError_t residual_dispatch(int lpr, int n, const int *rp, const int *ci
         else                                                                                                          \
             hipLaunchKernelGGL((k_residual<LPR / 4, false, V, T>), grid, block, 0, s, n, rp, ci, v, x, b, r); \
         break;
-    switch (lpr == kCsrLong ? 64 : lpr) {
+    switch (spmv_lanes(lpr)) {
         GSX_L(8) GSX_L(16) GSX_L(32) GSX_L(64)
     default: return hipErrorInvalidValue;
     }

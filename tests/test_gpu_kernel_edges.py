@@ -419,3 +419,30 @@ def test_row_assembly_of_one_element_patches(ctx, p, g):
         assert err.value.status == gsx.GSX_ERR_JACOBIAN
         gp.close()
         prob.patches[k].ctrl = ctrl
+
+
+@pytest.mark.parametrize("prec", [gsx.FP64, gsx.MIXED])
+@pytest.mark.parametrize("per_row,lanes", [(60, 32), (150, 64), (300, 64), (700, 64)])
+def test_batch_lanes_of_csr_members(ctx, prec, per_row, lanes):
+    """A CSR member added without a tile shape sums its rows with the lanes of
+    its mean row length, 64 for the longest: its iterates are bitwise those of
+    the member given these lanes, and not those of 8 lanes."""
+    import scipy.sparse as sp
+    n = 900
+    rng = np.random.default_rng(per_row)
+    M = np.where(rng.random((n, n)) < per_row / n / 2, rng.standard_normal((n, n)), 0.0)
+    M = M + M.T
+    np.fill_diagonal(M, np.abs(M).sum(axis=1) + rng.uniform(0.5, 1.5, n))
+    M = sp.csr_matrix(M)
+    A = gsx.Matrix.from_csr(ctx, M.indptr, M.indices, M.data, with_fp32=True)
+    b = ctx.to_device(rng.standard_normal(n))
+    B = gsx.Batch(ctx, prec, 3)
+    xs = [ctx.array(n).zero() for _ in range(3)]
+    ids = [B.add(A, b, x, tol=1e-30, maxit=6, tile=t) for x, t in zip(xs, (None, (lanes, 1), (8, 1)))]
+    B.run(6)
+    got = [x.download() for x in xs]
+    assert all(B.result(i)[1] >= 6 for i in ids)
+    assert np.array_equal(got[0], got[1])
+    assert not np.array_equal(got[0], got[2])
+    for o in (B, b, A, *xs):
+        o.close()
