@@ -2319,7 +2319,8 @@ gsx_status gsx_cg_solve_noalloc(gsx_matrix *A, int32_t precond, double tau, cons
         if (relres) *relres = 0.0;
         return GSX_OK;
     }
-    const int rpb = 256 / A->lpr;   // the fixed array's documented share of partial sums: one per rpb rows
+    // the fixed array's documented share of partial sums: one per rpb rows
+    const int rpb = 256 / gsx::spmv_lanes(A->lpr);
     const int nparts = std::max((n + rpb - 1) / rpb, (n + 255) / 256) + 1;
     size_t off = 0;
     auto take = [&](size_t bytes) {

@@ -53,3 +53,29 @@ def test_noalloc_cg_refuses_oversized_requests(ctx):
     for a in (A, b, x):
         a.close()
     gp.close()
+
+
+@pytest.mark.parametrize("per_row,rows_per_part", [(30, 16), (200, 4), (400, 4)])
+def test_noalloc_cg_workspace_limit(ctx, per_row, rows_per_part):
+    """The workspace holds five vectors, four partial sums per 256 / lanes rows
+    (64 lanes for the longest rows) and the residual history: a request that
+    fills its 64 MiB runs, one history entry more than that is refused."""
+    import scipy.sparse as sp
+    n = 3000
+    k = per_row // 2
+    M = sp.diags([np.full(n - j, -1.0) for j in range(1, k + 1)], range(1, k + 1))
+    M = (M + M.T + sp.diags(np.full(n, 2.0 * k + 1.0))).tocsr()
+    A = gsx.Matrix.from_csr(ctx, M.indptr, M.indices, M.data)
+    b, x = ctx.to_device(np.ones(n)), ctx.array(n).zero()
+
+    def up(v):
+        return (v + 255) // 256 * 256
+    nparts = -(-n // rows_per_part) + 1
+    room = (64 << 20) - 5 * up(8 * n) - up(8 * 4 * nparts) - 256   # the state takes one piece of 256 bytes
+    maxit = room // 8 - 1
+    st, it, rr = _noalloc(A, b, x, gsx.PREC_JACOBI, 1.0, maxit=maxit)
+    assert st == 0 and rr < 1e-10, gsx.lib().gsx_last_error(ctx.h)
+    st, it, rr = _noalloc(A, b, x, gsx.PREC_JACOBI, 1.0, maxit=maxit + 1)
+    assert st == gsx.GSX_ERR_ARG
+    for a in (A, b, x):
+        a.close()
