@@ -296,7 +296,9 @@ struct gsx_problem {
     DevPtr kept_K, kept_raw;   // element matrices, or raw rows of 2D patches
     uint64_t asm_serial = 0, kept_serial = 0;
     bool zero_kappa = false;        // some element has kappa exactly 0
-    bool odd_glue = false;          // an interface joins a patch to itself or to one of another degree
+    // an interface joins a patch to itself or to one of another degree, or two
+    // functions of a patch are joined through its neighbours
+    bool odd_glue = false;
     // geometry, kappa and source of another problem (a level of a
     // p-multigrid hierarchy): this problem's patches give only the basis
     gsx_problem *geo = nullptr;
@@ -866,6 +868,7 @@ gsx_status gsx_problem_create(gsx_ctx *c, int32_t npatch, const gsx_patch_desc *
             const int g = P->dofs[P->boff[k] + l];
             if (g < nfree) {
                 const int o = fillp[g]++;
+                P->odd_glue = P->odd_glue || (o > occ_cnt[g] && occ_patch[o - 1] == k);
                 occ_patch[o] = k;
                 occ_local[o] = l;
             }
@@ -1183,7 +1186,8 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
         if (P->geo->npatch != P->npatch) return fail(c, GSX_ERR_ARG, "geometry problem changed");
     }
     // 2D patches of degrees 2 to 4: sum-factorised rows likewise (a row of a
-    // patch glued to itself could meet a column twice in its window)
+    // patch glued to itself, directly or around a corner of its neighbours,
+    // could meet a column twice in its window)
     const bool use_sf2 = P->nfree > 0 && !elementwise_asked && sf2_rows_ok(P);
     const bool use_sf = single && !elementwise && !keep_elements && !P->zero_kappa && P->hp[0].d == 3 &&
                         P->hp[0].p[0] == P->hp[0].p[1] && P->hp[0].p[0] == P->hp[0].p[2] &&

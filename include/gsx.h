@@ -258,7 +258,8 @@ gsx_status gsx_assemble_bdr(gsx_problem *prob, double *rhs_dev);
  * degree 1 with GSX_ASM_ROWWISE) whose kappa has no exact zero is assembled row by row by
  * sum factorisation on the FP64 matrix cores, without element matrices; so are
  * 2D patches of degree 2, 3 or 4 (equal in both directions; any number of
- * patches, none glued to itself or to one of another degree), on the vector units (the
+ * patches, none glued to itself, directly or around a corner of its
+ * neighbours, or to one of another degree), on the vector units (the
  * same sums over the same Gauss points, grouped by point columns instead of
  * elements: values agree with the element path to rounding).  There no
  * entry is dropped by the exact-zero rule: an entry with only exact-zero

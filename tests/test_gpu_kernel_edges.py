@@ -446,3 +446,25 @@ def test_batch_lanes_of_csr_members(ctx, prec, per_row, lanes):
     assert not np.array_equal(got[0], got[2])
     for o in (B, b, A, *xs):
         o.close()
+
+
+# patch 0's west and east sides on patch 1's south and west sides, so that the
+# ends of patch 0's south side are one function: rows whose window holds both
+# ends (up to p + 1 elements) meet that column twice
+@pytest.mark.parametrize("p,n", [(2, 2), (2, 3), (3, 2), (3, 4), (4, 3), (4, 5), (3, 6)])
+def test_patch_glued_to_itself_around_a_corner(ctx, p, n):
+    patches = [problems.box_patch(2, p, (n, 3)), problems.box_patch(2, p, (3, 3), lo=[2.0, 2.0], hi=[3.0, 3.0])]
+    for k, P in enumerate(patches):
+        problems.perturb_interior(P, 0.1 / n, 80 + k)
+        P.fkind = 1
+    prob = problems.Problem(patches, [(1, 2), (1, 4)], [(0, 1, 1, 3, 0, 0, 0, 0), (0, 2, 1, 1, 1, 0, 0, 0)])
+    dofs, nfree = O.mapper(prob.patches, prob.dir_sides, prob.ifaces)
+    assert dofs[0] == dofs[n + p - 1] < nfree
+    Ao, bo = O.assemble(prob.patches, dofs, nfree, 0)
+    gp = gsx.Problem(ctx, prob)
+    A, b = gp.assemble(gsx.PATTERN_EXPR)
+    # as test_row_assembly_2d; a column listed twice in a row counts once
+    assert np.abs(A.to_scipy().toarray() - Ao.toarray()).max() <= 1e-12 * np.abs(Ao.data).max()
+    assert np.abs(b.download() - bo).max() <= 1e-12 * np.abs(bo).max()
+    for o in (A, b, gp):
+        o.close()
