@@ -3422,10 +3422,11 @@ extern "C" gsx_status gsx_mg_create(gsx_problem *fine, gsx_matrix *A, int32_t nl
         elem_path = (fine->kdoubles + fine->fdoubles + kc) * (int64_t)sizeof(double) <= c->elem_budget;
     }
     // 2D patches of degrees 2 to 4: from raw rows instead, which are 1/8 of the
-    // element matrices' bytes at p = 3
-    const bool raw_path = elem_path && sf2_rows_ok(fine);
+    // element matrices' bytes at p = 3, unless A's element matrices were kept
+    const bool kept = fine->kept_serial == A->src_serial;
+    const bool raw_path = elem_path && sf2_rows_ok(fine) && !(kept && fine->kept_K);
     DevPtr Kf, Rf;
-    if (raw_path && fine->kept_raw && fine->kept_serial == A->src_serial) {
+    if (raw_path && kept && fine->kept_raw) {
         Rf = std::move(fine->kept_raw);
     } else if (raw_path) {
         KScope ke(c, "mg_elem");
@@ -3434,7 +3435,7 @@ extern "C" gsx_status gsx_mg_create(gsx_problem *fine, gsx_matrix *A, int32_t nl
         if (!Rf || !Ff) return fail(c, GSX_ERR_OOM, "device allocation (row assembly)");
         int64_t ndet = 0;
         GSX_TRY(sf2_assemble_rows(fine, dp<double>(Rf), dp<double>(Ff), &ndet));
-    } else if (elem_path && fine->kept_K && fine->kept_serial == A->src_serial) {
+    } else if (elem_path && kept && fine->kept_K) {
         Kf = std::move(fine->kept_K);   // this matrix's own element matrices
     } else if (elem_path) {
         KScope ke(c, "mg_elem");

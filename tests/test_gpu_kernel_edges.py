@@ -468,3 +468,24 @@ def test_patch_glued_to_itself_around_a_corner(ctx, p, n):
     assert np.abs(b.download() - bo).max() <= 1e-12 * np.abs(bo).max()
     for o in (A, b, gp):
         o.close()
+
+
+@pytest.mark.parametrize("mode", [0, gsx.ASM_ELEMENTWISE])
+def test_kept_elements_serve_the_multigrid_setup(ctx, mode):
+    """Element matrices or raw rows kept by an assembly are what the set-up
+    takes: it forms none of its own."""
+    prob = problems.square_grid(2, 2, 8, 3)
+    gp = gsx.Problem(ctx, prob)
+    for keep, formed in ((gsx.ASM_KEEP_ELEMENTS, 0), (0, 1)):
+        A, b = gp.assemble(gsx.PATTERN_FULL | mode | keep)
+        ctx.enable_timing(True)
+        ctx.reset_timing()
+        mg = gsx.Multigrid(gp, A, 2, 1, 1, 0.7)
+        ctx.enable_timing(False)
+        assert ctx.kernel_stats("mg_elem")[0] == formed
+        ops = [mg.level(l) for l in range(2)]
+        want = ops[0][1].T @ ops[1][0] @ ops[0][1]
+        assert abs(ops[0][0] - want).max() <= 1e-13 * 25 * abs(want).max()   # as test_galerkin_rows
+        for o in (mg, A, b):
+            o.close()
+    gp.close()
