@@ -1060,6 +1060,9 @@ static bool sf2_rows_ok(const gsx_problem *P)
     return ok;
 }
 
+// bytes of their raw rows and loads, which keep to the element budget
+static int64_t sf2_bytes(const gsx_problem *P) { return (P->rdoubles + P->nbasis) * (int64_t)sizeof(double); }
+
 // Raw rows and their loads (launch_sf2_rows) of every patch; ndet: the
 // determinant minima written to d_detmin, one per block.
 static gsx_status sf2_assemble_rows(gsx_problem *P, double *raw, double *rawf, int64_t *ndet)
@@ -1188,7 +1191,7 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
     // 2D patches of degrees 2 to 4: sum-factorised rows likewise (a row of a
     // patch glued to itself, directly or around a corner of its neighbours,
     // could meet a column twice in its window)
-    const bool use_sf2 = P->nfree > 0 && !elementwise_asked && sf2_rows_ok(P);
+    const bool use_sf2 = P->nfree > 0 && !elementwise_asked && sf2_rows_ok(P) && sf2_bytes(P) <= c->elem_budget;
     const bool use_sf = single && !elementwise && !keep_elements && !P->zero_kappa && P->hp[0].d == 3 &&
                         P->hp[0].p[0] == P->hp[0].p[1] && P->hp[0].p[0] == P->hp[0].p[2] &&
                         gsx::sf_supported(3, P->hp[0].p[0]);
@@ -1197,7 +1200,9 @@ gsx_status gsx_assemble(gsx_problem *P, int32_t mode, int32_t precision, gsx_mat
     // layers along its slowest direction (each slab recomputes the p element
     // layers its first rows share with the previous slab, so every entry is
     // still summed over all its elements in element order); several patches
-    // are assembled at once and must fit the budget.
+    // are assembled at once and must fit the budget.  The refusals hold for the
+    // 2D row path too: what an element-wise assembly of the problem refuses is
+    // refused whatever path it takes.
     const HostPatch &h0 = P->hp[0];
     const int sd = h0.d - 1;   // slowest direction
     int64_t layer_elems = 1;
@@ -3424,7 +3429,9 @@ extern "C" gsx_status gsx_mg_create(gsx_problem *fine, gsx_matrix *A, int32_t nl
     // 2D patches of degrees 2 to 4: from raw rows instead, which are 1/8 of the
     // element matrices' bytes at p = 3, unless A's element matrices were kept
     const bool kept = fine->kept_serial == A->src_serial;
-    const bool raw_path = elem_path && sf2_rows_ok(fine) && !(kept && fine->kept_K);
+    bool raw_path = elem_path && sf2_rows_ok(fine) && !(kept && fine->kept_K);
+    if (raw_path)   // two levels' rows and the half-contracted lines between them (fewer than the fine rows)
+        raw_path = 2 * sf2_bytes(fine) + sf2_bytes(mg->L[nlevels - 2].prob) <= c->elem_budget;
     DevPtr Kf, Rf;
     if (raw_path && kept && fine->kept_raw) {
         Rf = std::move(fine->kept_raw);

@@ -126,8 +126,10 @@ gsx_status gsx_ctx_memory(gsx_ctx *ctx, int64_t *bytes_in_use);
 /* Device bytes the element matrices of one assembly pass may occupy
  * (default 16 GiB).  A single patch larger than this is assembled in slabs
  * of element layers (the result is identical); a multipatch assembly that
- * does not fit fails with GSX_ERR_BUDGET.  No reference counterpart (the
- * reference assembles element by element on the host). */
+ * does not fit fails with GSX_ERR_BUDGET.  The row assembly of 2D patches
+ * (gsx_assemble) runs where its rows fit the budget too and refuses what the
+ * element path refuses.  No reference counterpart (the reference assembles
+ * element by element on the host). */
 gsx_status gsx_ctx_set_elem_budget(gsx_ctx *ctx, int64_t bytes);
 /* Largest coarsest multigrid level (rows, 1..32768, default 32768) solved
  * exactly through its dense FP64 inverse, one GEMV per coarse solve.  A

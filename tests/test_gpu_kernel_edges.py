@@ -489,3 +489,53 @@ def test_kept_elements_serve_the_multigrid_setup(ctx, mode):
         for o in (mg, A, b):
             o.close()
     gp.close()
+
+
+def _noisy_grid(g, n, p):
+    prob = problems.square_grid(g, g, n, p)
+    for k, P in enumerate(prob.patches):
+        problems.perturb_interior(P, 0.1 / n, 90 + k)
+        P.kappa = problems.lognormal_kappa(P.nelem, 0.5, 90 + k)
+    return prob
+
+
+# budgets in bytes that the element matrices fit (one patch: slabs of them) and
+# the raw rows of all patches do not
+@pytest.mark.parametrize("g,n,p,budget", [(1, 64, 2, 400_000), (1, 64, 4, 2_000_000), (4, 1, 4, 100_000)])
+def test_raw_rows_keep_to_the_element_budget(ctx, g, n, p, budget):
+    """Where the raw rows exceed the budget the element path runs: bitwise the
+    matrix and load of an assembly that asks for it."""
+    gp = gsx.Problem(ctx, _noisy_grid(g, n, p))
+    out = []
+    for b, mode in ((16 << 30, gsx.ASM_ELEMENTWISE), (budget, 0), (16 << 30, 0)):
+        try:
+            ctx.set_elem_budget(b)
+            A, rhs = gp.assemble(gsx.PATTERN_FULL | mode)
+        finally:
+            ctx.set_elem_budget(16 << 30)
+        out.append([*A.download(), rhs.download()])
+        for o in (A, rhs):
+            o.close()
+    assert all(np.array_equal(u, v) for u, v in zip(out[0], out[1]))
+    # the row path's sums round differently, so the comparison tells the paths
+    assert not np.array_equal(out[0][2], out[2][2])
+    gp.close()
+
+
+def test_galerkin_rows_keep_to_the_element_budget(ctx):
+    """Two levels' element matrices fit (233 KB), their raw rows and the lines
+    between them do not (up to 426 KB): the levels come from element matrices."""
+    gp = gsx.Problem(ctx, _noisy_grid(3, 2, 4))
+    out = []
+    for b, mode in ((16 << 30, gsx.ASM_ELEMENTWISE | gsx.ASM_KEEP_ELEMENTS), (270_000, 0), (16 << 30, 0)):
+        try:
+            ctx.set_elem_budget(b)
+            A, rhs = gp.assemble(gsx.PATTERN_FULL | mode)
+            mg = gsx.Multigrid(gp, A, 2, 1, 1, 0.7)
+        finally:
+            ctx.set_elem_budget(16 << 30)
+        out.append(mg.level(0)[0].data)
+        for o in (mg, A, rhs):
+            o.close()
+    assert np.array_equal(out[0], out[1]) and not np.array_equal(out[0], out[2])
+    gp.close()
