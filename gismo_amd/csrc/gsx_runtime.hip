@@ -95,6 +95,7 @@ struct gsx_ctx {
     GaussTab gt;
     int64_t elem_budget = int64_t(16) << 30;   // bytes of element matrices per assembly pass
     int64_t coarse_dense_max = 32768;          // largest coarsest level solved by its dense inverse
+    int64_t alloc_limit = 0;                   // device allocations above fail (0: none do)
     void *scratch = nullptr;   // this device's address of the allocation-free workspace
 };
 
@@ -123,6 +124,7 @@ gsx_status fail(gsx_ctx *c, gsx_status s, const std::string &msg)
 DevPtr dalloc(gsx_ctx *c, size_t bytes)
 {
     void *p = nullptr;
+    if (c->alloc_limit > 0 && bytes > (size_t)c->alloc_limit) return nullptr;
     bytes = Counter::round(bytes ? bytes : 16);
     auto mem = c->mem;
     p = mem->take(bytes);
@@ -523,6 +525,13 @@ gsx_status gsx_ctx_set_elem_budget(gsx_ctx *c, int64_t bytes)
 {
     if (!c || bytes <= 0) return GSX_ERR_ARG;
     c->elem_budget = bytes;
+    return GSX_OK;
+}
+
+gsx_status gsx_ctx_set_alloc_limit(gsx_ctx *c, int64_t bytes)
+{
+    if (!c || bytes < 0) return GSX_ERR_ARG;
+    c->alloc_limit = bytes;
     return GSX_OK;
 }
 
@@ -3002,12 +3011,10 @@ static int rcm_order(int n, const std::vector<int> &rp, const std::vector<int> &
     return b;
 }
 
-// Per-level diagonals, FP32 copies and vectors, then the exact coarse solve
-// (the dense inverse of the coarsest operator or, above the context's
-// coarse_dense_max rows, its banded FP64 Cholesky factor).
 // Slices of level l's operator, unless padding would add more than a quarter
-// of its entries (very uneven rows): FP32 values for the levels a mixed cycle
-// reads in FP32, FP64 values otherwise and on the finest level (the outer CG).
+// of its entries (very uneven rows) or they do not fit the device: FP32 values
+// for the levels a mixed cycle reads in FP32, FP64 values otherwise and on the
+// finest level (the outer CG).
 static gsx_status mg_sell(gsx_mg *mg, int l)
 {
     gsx_ctx *c = mg->ctx;
@@ -3020,26 +3027,78 @@ static gsx_status mg_sell(gsx_mg *mg, int l)
     if (V.n <= 0 || V.nnz < (1 << 18)) return GSX_OK;
     const int nsl = (V.n + 63) / 64;
     DevPtr width = dalloc(c, sizeof(int) * nsl);
-    if (!width) return fail(c, GSX_ERR_OOM, "device allocation (level slices)");
+    if (!width) return GSX_OK;
     HIP_OK(c, gsx::launch_sell_width(V.n, dp<int>(V.rowptr), dp<int>(width), s));
     DevPtr ptr;
     int64_t total = 0;
-    GSX_TRY(scan_counts(c, dp<int>(width), nsl, ptr, total));
+    const gsx_status st = scan_counts(c, dp<int>(width), nsl, ptr, total);
+    if (st != GSX_OK) return st == GSX_ERR_OOM ? GSX_OK : st;
     if ((double)total * 64 > 1.25 * (double)V.nnz + 65536.0) return GSX_OK;
     const size_t slots = (size_t)std::max<int64_t>(1, total) * 64;
-    V.sl_uni = dalloc(c, sizeof(int) * nsl);
-    V.sl_col = dalloc(c, sizeof(int) * slots);
-    if (mixed) V.sl_val32 = dalloc(c, sizeof(float) * slots);
-    if (!mixed || finest) V.sl_val = dalloc(c, sizeof(double) * slots);
-    if (!V.sl_uni || !V.sl_col || (mixed && !V.sl_val32) || ((!mixed || finest) && !V.sl_val))
-        return fail(c, GSX_ERR_OOM, "device allocation (level slices)");
+    DevPtr uni = dalloc(c, sizeof(int) * nsl), col = dalloc(c, sizeof(int) * slots), val32, val;
+    if (mixed) val32 = dalloc(c, sizeof(float) * slots);
+    if (!mixed || finest) val = dalloc(c, sizeof(double) * slots);
+    if (!uni || !col || (mixed && !val32) || ((!mixed || finest) && !val)) return GSX_OK;
     HIP_OK(c, gsx::launch_sell_fill(V.n, dp<int>(V.rowptr), dp<int>(V.col), dp<double>(V.val), dp<int>(ptr),
-                                    dp<int>(V.sl_uni), dp<int>(V.sl_col), dp<float>(V.sl_val32), dp<double>(V.sl_val),
-                                    s));
+                                    dp<int>(uni), dp<int>(col), dp<float>(val32), dp<double>(val), s));
     V.sl_ptr = ptr;
+    V.sl_uni = uni;
+    V.sl_col = col;
+    V.sl_val32 = val32;
+    V.sl_val = val;
     return GSX_OK;
 }
 
+// The exact coarse solve: the dense inverse up to coarse_dense_max rows (one
+// GEMV per solve); above, a banded FP64 Cholesky factor in reverse
+// Cuthill-McKee order (its two triangular solves run panel after panel, slower
+// than the GEMV where both fit).
+static gsx_status mg_coarse_solver(gsx_mg *mg)
+{
+    gsx_ctx *c = mg->ctx;
+    hipStream_t s = c->stream;
+    KScope ki(c, "mg_coarse_inverse");
+    MGLevel &C0 = mg->L[0];
+    const int n0 = C0.n;
+    if ((int64_t)n0 > c->coarse_dense_max) {
+        std::vector<int> rp((size_t)n0 + 1), ci((size_t)C0.nnz), pos;
+        HIP_OK(c, hipMemcpyAsync(rp.data(), C0.rowptr.get(), sizeof(int) * (n0 + 1), hipMemcpyDeviceToHost, s));
+        HIP_OK(c, hipMemcpyAsync(ci.data(), C0.col.get(), sizeof(int) * C0.nnz, hipMemcpyDeviceToHost, s));
+        HIP_OK(c, hipStreamSynchronize(s));
+        const int b = rcm_order(n0, rp, ci, pos);
+        if (b <= 4096) {
+            mg->band_b = b;
+            mg->band_pos = dalloc(c, sizeof(int) * n0);
+            mg->band_L = dalloc(c, sizeof(double) * (size_t)n0 * (b + 1));
+            mg->band_y = dalloc(c, sizeof(double) * n0);
+            DevPtr errf = dalloc(c, sizeof(int));
+            if (!mg->band_pos || !mg->band_L || !mg->band_y || !errf)
+                return fail(c, GSX_ERR_OOM, "device allocation (coarse factor)");
+            HIP_OK(c, hipMemcpyAsync(mg->band_pos.get(), pos.data(), sizeof(int) * n0, hipMemcpyHostToDevice, s));
+            HIP_OK(c, hipMemsetAsync(errf.get(), 0, sizeof(int), s));
+            HIP_OK(c, gsx::launch_band_factor(n0, b, dp<int>(C0.rowptr), dp<int>(C0.col), dp<double>(C0.val),
+                                              dp<int>(mg->band_pos), dp<double>(mg->band_L), dp<int>(errf), s));
+            int errh = 0;
+            HIP_OK(c, hipMemcpyAsync(&errh, errf.get(), sizeof(int), hipMemcpyDeviceToHost, s));
+            HIP_OK(c, hipStreamSynchronize(s));
+            if (errh) return fail(c, GSX_ERR_ARG, "coarsest operator is not positive definite (Cholesky pivot)");
+            return GSX_OK;
+        }
+    }
+    if ((int64_t)n0 > 32768)
+        return fail(c, GSX_ERR_ARG, "coarsest level too large for the dense inverse and its band too wide");
+    mg->npad = gsx::dense_inverse_npad(n0);
+    mg->Dinv = dalloc(c, sizeof(double) * (size_t)mg->npad * mg->npad);
+    DevPtr W = dalloc(c, sizeof(double) * (size_t)gsx::dense_inverse_work_doubles(mg->npad));
+    if (!mg->Dinv || !W) return fail(c, GSX_ERR_OOM, "device allocation (coarse inverse)");
+    HIP_OK(c, gsx::launch_dense_inverse(n0, mg->npad, dp<int>(C0.rowptr), dp<int>(C0.col), dp<double>(C0.val),
+                                        dp<double>(mg->Dinv), dp<double>(W), s));
+    HIP_OK(c, hipStreamSynchronize(s));
+    return GSX_OK;
+}
+
+// Per-level diagonals, FP32 copies and vectors, the exact coarse solve and, in
+// the memory that is left, the levels' slices.
 static gsx_status mg_finish(gsx_mg *mg)
 {
     gsx_ctx *c = mg->ctx;
@@ -3068,51 +3127,9 @@ static gsx_status mg_finish(gsx_mg *mg)
             }
         }
         GSX_TRY(mg_level_vectors(c, V, mixed));
-        if (l > 0) GSX_TRY(mg_sell(mg, l));
     }
-    // exact coarse solve: the dense inverse up to coarse_dense_max rows (one
-    // GEMV per solve); above, a banded FP64 Cholesky factor in reverse
-    // Cuthill-McKee order (its two triangular solves run panel after panel,
-    // slower than the GEMV where both fit)
-    {
-        KScope ki(c, "mg_coarse_inverse");
-        MGLevel &C0 = mg->L[0];
-        const int n0 = C0.n;
-        if ((int64_t)n0 > c->coarse_dense_max) {
-            std::vector<int> rp((size_t)n0 + 1), ci((size_t)C0.nnz), pos;
-            HIP_OK(c, hipMemcpyAsync(rp.data(), C0.rowptr.get(), sizeof(int) * (n0 + 1), hipMemcpyDeviceToHost, s));
-            HIP_OK(c, hipMemcpyAsync(ci.data(), C0.col.get(), sizeof(int) * C0.nnz, hipMemcpyDeviceToHost, s));
-            HIP_OK(c, hipStreamSynchronize(s));
-            const int b = rcm_order(n0, rp, ci, pos);
-            if (b <= 4096) {
-                mg->band_b = b;
-                mg->band_pos = dalloc(c, sizeof(int) * n0);
-                mg->band_L = dalloc(c, sizeof(double) * (size_t)n0 * (b + 1));
-                mg->band_y = dalloc(c, sizeof(double) * n0);
-                DevPtr errf = dalloc(c, sizeof(int));
-                if (!mg->band_pos || !mg->band_L || !mg->band_y || !errf)
-                    return fail(c, GSX_ERR_OOM, "device allocation (coarse factor)");
-                HIP_OK(c, hipMemcpyAsync(mg->band_pos.get(), pos.data(), sizeof(int) * n0, hipMemcpyHostToDevice, s));
-                HIP_OK(c, hipMemsetAsync(errf.get(), 0, sizeof(int), s));
-                HIP_OK(c, gsx::launch_band_factor(n0, b, dp<int>(C0.rowptr), dp<int>(C0.col), dp<double>(C0.val),
-                                                  dp<int>(mg->band_pos), dp<double>(mg->band_L), dp<int>(errf), s));
-                int errh = 0;
-                HIP_OK(c, hipMemcpyAsync(&errh, errf.get(), sizeof(int), hipMemcpyDeviceToHost, s));
-                HIP_OK(c, hipStreamSynchronize(s));
-                if (errh) return fail(c, GSX_ERR_ARG, "coarsest operator is not positive definite (Cholesky pivot)");
-                return GSX_OK;
-            }
-        }
-        if ((int64_t)n0 > 32768)
-            return fail(c, GSX_ERR_ARG, "coarsest level too large for the dense inverse and its band too wide");
-        mg->npad = gsx::dense_inverse_npad(n0);
-        mg->Dinv = dalloc(c, sizeof(double) * (size_t)mg->npad * mg->npad);
-        DevPtr W = dalloc(c, sizeof(double) * (size_t)gsx::dense_inverse_work_doubles(mg->npad));
-        if (!mg->Dinv || !W) return fail(c, GSX_ERR_OOM, "device allocation (coarse inverse)");
-        HIP_OK(c, gsx::launch_dense_inverse(n0, mg->npad, dp<int>(C0.rowptr), dp<int>(C0.col), dp<double>(C0.val),
-                                            dp<double>(mg->Dinv), dp<double>(W), s));
-        HIP_OK(c, hipStreamSynchronize(s));
-    }
+    GSX_TRY(mg_coarse_solver(mg));
+    for (int l = 1; l < nlevels; ++l) GSX_TRY(mg_sell(mg, l));
     return GSX_OK;
 }
 

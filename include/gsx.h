@@ -131,6 +131,10 @@ gsx_status gsx_ctx_memory(gsx_ctx *ctx, int64_t *bytes_in_use);
  * element path refuses.  No reference counterpart (the reference assembles
  * element by element on the host). */
 gsx_status gsx_ctx_set_elem_budget(gsx_ctx *ctx, int64_t bytes);
+/* Device allocations of the library above this many bytes fail as they do on
+ * a full device (0, the default: no limit).  For tests of what a program does
+ * when memory is short; no reference counterpart. */
+gsx_status gsx_ctx_set_alloc_limit(gsx_ctx *ctx, int64_t bytes);
 /* Largest coarsest multigrid level (rows, 1..32768, default 32768) solved
  * exactly through its dense FP64 inverse, one GEMV per coarse solve.  A
  * larger coarsest level is factored as a banded FP64 Cholesky in reverse

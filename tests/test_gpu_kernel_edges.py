@@ -539,3 +539,40 @@ def test_galerkin_rows_keep_to_the_element_budget(ctx):
             o.close()
     assert np.array_equal(out[0], out[1]) and not np.array_equal(out[0], out[2])
     gp.close()
+
+
+@pytest.mark.parametrize("prec", [gsx.FP64, gsx.MIXED])
+def test_hierarchy_without_room_for_its_slices(ctx, prec):
+    """Level slices are a second copy: where the finest one does not fit (an
+    allocation above the CSR values' size fails) that level runs on its CSR
+    arrays, and nothing is left of the slices."""
+    prob = problems.square_grid(2, 1, 56, 3)
+    gp = gsx.Problem(ctx, prob)
+    A, b = gp.assemble(gsx.PATTERN_FULL, prec)
+    assert A.nnz >= 1 << 18
+    r = ctx.to_device(np.random.default_rng(8).standard_normal(gp.nfree))
+    out, held = [], []
+    for limit in (0, 8 * A.nnz):
+        before = ctx.memory()
+        try:
+            ctx.set_alloc_limit(limit)
+            mg = gsx.Multigrid(gp, A, 4, 2, 2, 0.6, precision=prec)
+        finally:
+            ctx.set_alloc_limit(0)
+        held.append(ctx.memory() - before)
+        z, x = ctx.array(gp.nfree), ctx.array(gp.nfree).zero()
+        mg.apply(r, z)
+        it, rel, ok = gsx.mg_cg_solve(A, mg, b, x, tol=1e-9)
+        assert ok
+        out.append((z.download(), it, x.download()))
+        for o in (z, x, mg):
+            o.close()
+    # values and columns, of a mixed hierarchy FP32 and FP64 values and columns
+    assert held[0] - held[1] >= (16 if prec == gsx.MIXED else 12) * A.nnz
+    # both forms sum the same FP64 products of a row, in another order; the
+    # mixed cycle rounds its coarse vectors to FP32
+    assert np.linalg.norm(out[0][0] - out[1][0]) <= (1e-10 if prec == gsx.FP64 else 2e-5) * np.linalg.norm(out[0][0])
+    assert abs(out[0][1] - out[1][1]) <= 1
+    assert np.linalg.norm(out[0][2] - out[1][2]) <= 1e-6 * np.linalg.norm(out[0][2])
+    for o in (r, b, A, gp):
+        o.close()
