@@ -3015,16 +3015,19 @@ static int rcm_order(int n, const std::vector<int> &rp, const std::vector<int> &
 // of its entries (very uneven rows) or they do not fit the device: FP32 values
 // for the levels a mixed cycle reads in FP32, FP64 values otherwise and on the
 // finest level (the outer CG).
+constexpr int kSliceRows = 65536;
 static gsx_status mg_sell(gsx_mg *mg, int l)
 {
     gsx_ctx *c = mg->ctx;
     hipStream_t s = c->stream;
     MGLevel &V = mg->L[l];
     const bool mixed = mg->precision == GSX_MIXED, finest = l == (int)mg->L.size() - 1;
-    // below 2^18 entries forming the slices costs more than a solve gains by
-    // them (2 x 2 patches of 28^2 elements p = 2, 78 K entries: set-up and solve
-    // 2.7 ms with slices, 2.5 without; from 3 M entries a step is twice as fast)
-    if (V.n <= 0 || V.nnz < (1 << 18)) return GSX_OK;
+    // Fewer rows are too few slices for the chip, and rows of their own lanes
+    // (CSR) end sooner.  A cycle with slices on all levels of 2^18 entries / on
+    // none: 4.9 K rows of 250 (16^3 p = 3) 66 / 52 us, 8 K of 104 46 / 46, 14 K of
+    // 107 56 / 52, 36 K of 292 201 / 198 (mixed 166 / 174), 64 K of 114 219 / 214;
+    // 66 K of 48 124 / 132 (mixed 116 / 128), 263 K of 49 231 / 273 (189 / 245)
+    if (V.n < kSliceRows) return GSX_OK;
     const int nsl = (V.n + 63) / 64;
     DevPtr width = dalloc(c, sizeof(int) * nsl);
     if (!width) return GSX_OK;

@@ -154,12 +154,13 @@ def test_csr_products(ctx, n, lo, hi):
         o.close()
 
 
-# level operators in slices of 64 rows from 2^18 entries up (CSR rows below):
-# several slices per wave block, four
-# waves per slice below 131,072 rows, uniform slices (inside a patch), a last
-# slice of one row, interface rows; against the cycle written out in scipy
+# level operators in slices of 64 rows from 65,536 rows up (CSR rows below): four
+# waves per slice below 131,072 rows, several slices per block above, uniform
+# slices (inside a patch), a last slice of one row (257^2), rows next to
+# interfaces; against the cycle written out in scipy
 @pytest.mark.parametrize("gx,gy,n,p,levels", [(1, 1, 16, 2, 2), (2, 1, 12, 3, 2), (3, 2, 24, 3, 3), (2, 2, 8, 4, 2),
-                                              (1, 1, 374, 2, 2), (2, 2, 60, 2, 3), (1, 1, 82, 3, 2), (2, 1, 52, 4, 2)])
+                                              (1, 1, 374, 2, 2), (2, 2, 60, 2, 3), (1, 1, 82, 3, 2), (2, 1, 52, 4, 2),
+                                              (1, 1, 256, 3, 4), (2, 1, 184, 3, 4), (2, 2, 200, 2, 4), (2, 2, 136, 4, 4)])
 @pytest.mark.parametrize("prec", [gsx.FP64, gsx.MIXED])
 def test_multigrid_level_slices(ctx, gx, gy, n, p, levels, prec):
     prob = problems.square_grid(gx, gy, n, p)
@@ -546,10 +547,10 @@ def test_hierarchy_without_room_for_its_slices(ctx, prec):
     """Level slices are a second copy: where the finest one does not fit (an
     allocation above the CSR values' size fails) that level runs on its CSR
     arrays, and nothing is left of the slices."""
-    prob = problems.square_grid(2, 1, 56, 3)
+    prob = problems.square_grid(2, 1, 184, 3)
     gp = gsx.Problem(ctx, prob)
     A, b = gp.assemble(gsx.PATTERN_FULL, prec)
-    assert A.nnz >= 1 << 18
+    assert gp.nfree >= 65536
     r = ctx.to_device(np.random.default_rng(8).standard_normal(gp.nfree))
     out, held = [], []
     for limit in (0, 8 * A.nnz):
