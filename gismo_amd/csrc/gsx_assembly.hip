@@ -1130,14 +1130,25 @@ __global__ void k_min_stage(const double *__restrict__ v, int64_t n, double *__r
 // 108 us; one block of 128 threads per element took 2974 us, and the sum of
 // its per-element results another 1175 us.
 // ---------------------------------------------------------------------------
-constexpr int kNormChunk = 8;
+constexpr int kNormChunk = 8;   // at most
+
+// coefficients of every patch's functions, in the patches' order: k_norms then
+// waits for one load per row instead of two
+__global__ __launch_bounds__(256) void k_norm_coefs(const int *__restrict__ dofs, int64_t nbasis,
+                                                    const double *__restrict__ sol, int nfree,
+                                                    const double *__restrict__ fixed, double *__restrict__ out)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nbasis) return;
+    const int g = dofs[i];
+    out[i] = g < nfree ? sol[g] : (fixed ? fixed[g - nfree] : 0.0);
+}
 
 template <int D, int P>
 __global__ __launch_bounds__(256) void k_norms(const PatchDev *__restrict__ patches,
                                                const int *__restrict__ gpatch,
-                                               const int64_t *__restrict__ bprefix, int ng, GaussTab gt,
-                                               const double *__restrict__ sol, int nfree,
-                                               const double *__restrict__ fixed, double *__restrict__ out,
+                                               const int64_t *__restrict__ bprefix, int ng, int ch, GaussTab gt,
+                                               const double *__restrict__ coefs, double *__restrict__ out,
                                                double *__restrict__ out_h1)
 {
     constexpr int NB1 = P + 1, NF = D + 1, L = D - 1;   // fields: coordinates, then u_h
@@ -1146,11 +1157,12 @@ __global__ __launch_bounds__(256) void k_norms(const PatchDev *__restrict__ patc
     __shared__ double sR[2][4];
     const int gi = find_patch(bprefix, ng, blockIdx.x);
     const PatchDev &pd = patches[gpatch[gi]];
+    const double *coef = coefs + pd.b_off;
     const int lb = (int)(blockIdx.x - bprefix[gi]);
     const int G0 = pd.nel[0] * NB1;
     const int64_t ncol = D == 3 ? (int64_t)G0 * (pd.nel[1] * NB1) : G0;
     const int ncb = (int)((ncol + 255) / 256);
-    const int e0 = (lb / ncb) * kNormChunk, e1 = min(e0 + kNormChunk, pd.nel[L]);
+    const int e0 = (lb / ncb) * ch, e1 = min(e0 + ch, pd.nel[L]);
     const int t = threadIdx.x;
     if (t < (e1 - e0) * NB1) {
         const int span = P + e0 + t / NB1;
@@ -1201,8 +1213,7 @@ __global__ __launch_bounds__(256) void k_norms(const PatchDev *__restrict__ patc
                     double c[NF];
 #pragma unroll
                     for (int r = 0; r < D; ++r) c[r] = pd.ctrl[(base + bx) * D + r];
-                    const int g = pd.dofs[base + bx];
-                    c[D] = g < nfree ? sol[g] : (fixed ? fixed[g - nfree] : 0.0);
+                    c[D] = coef[base + bx];
 #pragma unroll
                     for (int f = 0; f < NF; ++f) {
                         a0[f] += c[f] * v[0][bx];
@@ -1571,20 +1582,30 @@ hipError_t launch_elem_range(int d, int p, const PatchDev *patches, const int *g
     return hipGetLastError();
 }
 
-int64_t norm_blocks(int d, int p, const int *nel)
+int64_t norm_blocks(int d, int p, const int *nel, int ch)
 {
     int64_t cols = (int64_t)nel[0] * (p + 1);
     if (d == 3) cols *= (int64_t)nel[1] * (p + 1);
-    return (cols + 255) / 256 * ((nel[d - 1] + kNormChunk - 1) / kNormChunk);
+    return (cols + 255) / 256 * ((nel[d - 1] + ch - 1) / ch);
+}
+
+hipError_t launch_norm_coefs(const int *dofs, int64_t nbasis, const double *sol, int nfree, const double *fixed,
+                             double *out, hipStream_t s)
+{
+    if (nbasis <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_norm_coefs, dim3((unsigned)((nbasis + 255) / 256)), dim3(256), 0, s, dofs, nbasis, sol, nfree,
+                       fixed, out);
+    return hipGetLastError();
 }
 
 hipError_t launch_norms(int d, int p, const PatchDev *patches, const int *gpatch, const int64_t *bprefix, int ng,
-                        int64_t nblocks, const GaussTab &gt, const double *sol, int nfree, double *out,
-                        double *out_h1, const double *fixed, hipStream_t s)
+                        int ch, int64_t nblocks, const GaussTab &gt, const double *coefs, double *out, double *out_h1,
+                        hipStream_t s)
 {
     if (nblocks <= 0) return hipSuccess;
+    if (ch < 1 || ch > kNormChunk) return hipErrorInvalidValue;
     const dim3 grid((unsigned)nblocks);
-#define GSX_L(D, P) if (d == D && p == P) { hipLaunchKernelGGL((k_norms<D, P>), grid, dim3(256), 0, s, patches, gpatch, bprefix, ng, gt, sol, nfree, fixed, out, out_h1); return hipGetLastError(); }
+#define GSX_L(D, P) if (d == D && p == P) { hipLaunchKernelGGL((k_norms<D, P>), grid, dim3(256), 0, s, patches, gpatch, bprefix, ng, ch, gt, coefs, out, out_h1); return hipGetLastError(); }
     GSX_L(2, 1) GSX_L(2, 2) GSX_L(2, 3) GSX_L(2, 4)
     GSX_L(3, 1) GSX_L(3, 2) GSX_L(3, 3) GSX_L(3, 4)
 #undef GSX_L

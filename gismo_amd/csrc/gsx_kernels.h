@@ -40,11 +40,16 @@ hipError_t launch_elem(int d, int p, const PatchDev *patches, const int *gpatch,
 hipError_t launch_elem_range(int d, int p, const PatchDev *patches, const int *gpatch,
                              const int64_t *gprefix, int ng, int64_t e0, int64_t e1, const GaussTab &gt,
                              double *Kbuf, double *Fbuf, double *detmin, hipStream_t s);
-// Blocks of launch_norms for one patch (each writes one partial per norm).
-int64_t norm_blocks(int d, int p, const int *nel);
+// coefficients of all patches' functions (nbasis) from the solution and the
+// eliminated values
+hipError_t launch_norm_coefs(const int *dofs, int64_t nbasis, const double *sol, int nfree, const double *fixed,
+                             double *out, hipStream_t s);
+// Blocks of launch_norms for one patch (each writes one partial per norm) in
+// chunks of ch elements (1 to 8) along the last direction.
+int64_t norm_blocks(int d, int p, const int *nel, int ch);
 hipError_t launch_norms(int d, int p, const PatchDev *patches, const int *gpatch, const int64_t *bprefix, int ng,
-                        int64_t nblocks, const GaussTab &gt, const double *sol, int nfree, double *out,
-                        double *out_h1, const double *fixed, hipStream_t s);
+                        int ch, int64_t nblocks, const GaussTab &gt, const double *coefs, double *out, double *out_h1,
+                        hipStream_t s);
 // CSR pattern: row counts (col null; overflow set where a row is too long) or
 // columns; rows [nsingle, nfree) have several occurrences; flat: 2D windows
 hipError_t launch_row_pattern(const PatchDev *patches, const int *occ_ptr, const int *occ_patch,

@@ -250,6 +250,7 @@ struct Group {
     std::vector<int> patches;
     std::vector<int64_t> prefix;
     std::vector<int64_t> nprefix;   // blocks of the error norm kernel per patch
+    int norm_ch = 8;                // and its elements per chunk
     int64_t nelem = 0;
     DevPtr d_gpatch, d_gprefix, d_nprefix;
     std::vector<int64_t> rprefix;   // blocks of the 2D row assembly per patch
@@ -837,10 +838,13 @@ gsx_status gsx_problem_create(gsx_ctx *c, int32_t npatch, const gsx_patch_desc *
                                      hipMemcpyHostToDevice, s));
         }
         g.prefix.assign(1, 0);
-        g.nprefix.assign(1, 0);
-        for (int k : g.patches) {
-            g.prefix.push_back(g.prefix.back() + P->hp[k].nelem);
-            g.nprefix.push_back(g.nprefix.back() + gsx::norm_blocks(g.d, g.p, P->hp[k].nel));
+        for (int k : g.patches) g.prefix.push_back(g.prefix.back() + P->hp[k].nelem);
+        // shorter chunks (p elements more each) until two blocks per CU run
+        for (g.norm_ch = 8;; g.norm_ch /= 2) {
+            g.nprefix.assign(1, 0);
+            for (int k : g.patches)
+                g.nprefix.push_back(g.nprefix.back() + gsx::norm_blocks(g.d, g.p, P->hp[k].nel, g.norm_ch));
+            if (g.norm_ch == 1 || g.nprefix.back() >= 512) break;
         }
         g.nelem = g.prefix.back();
         g.d_gpatch = dalloc(c, sizeof(int) * g.patches.size());
@@ -2710,14 +2714,16 @@ gsx_status gsx_error_norms(gsx_problem *P, const double *sol, double *l2, double
     int64_t nblk = 0;   // partial sums: one per block, then the two totals
     for (auto &g : P->groups) nblk += g.nprefix.back();
     DevPtr per = dalloc(c, sizeof(double) * (2 * nblk + 2));
-    if (!per) return fail(c, GSX_ERR_OOM, "device allocation (error norms)");
+    DevPtr coefs = dalloc(c, sizeof(double) * P->nbasis);
+    if (!per || !coefs) return fail(c, GSX_ERR_OOM, "device allocation (error norms)");
     double *pl2 = dp<double>(per), *ph1 = h1semi ? pl2 + nblk : nullptr, *ptot = pl2 + 2 * nblk;
+    HIP_OK(c, gsx::launch_norm_coefs(dp<int>(P->d_dofs), P->nbasis, sol, P->nfree,
+                                     P->d_fixed ? dp<double>(P->d_fixed) : nullptr, dp<double>(coefs), s));
     int64_t off = 0;
     for (auto &g : P->groups) {
         HIP_OK(c, gsx::launch_norms(g.d, g.p, dp<PatchDev>(P->d_patches), dp<int>(g.d_gpatch),
-                                    dp<int64_t>(g.d_nprefix), (int)g.patches.size(), g.nprefix.back(), c->gt, sol,
-                                    P->nfree, pl2 + off, ph1 ? ph1 + off : nullptr,
-                                    P->d_fixed ? dp<double>(P->d_fixed) : nullptr, s));
+                                    dp<int64_t>(g.d_nprefix), (int)g.patches.size(), g.norm_ch, g.nprefix.back(), c->gt,
+                                    dp<double>(coefs), pl2 + off, ph1 ? ph1 + off : nullptr, s));
         off += g.nprefix.back();
     }
     HIP_OK(c, gsx::launch_sum_arrays(pl2, h1semi ? 2 : 1, nblk, nblk, ptot, s));

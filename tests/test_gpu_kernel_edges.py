@@ -19,11 +19,12 @@ def _noisy_box(d, p, n, seed=3, kappa=True):
     return problems.Problem([P], problems.all_sides(d), [], name=f"box-d{d}-p{p}-n{n}")
 
 
-# one Gauss point column per thread (blocks of 256 columns), chunks of 8
-# elements along the last direction
+# one Gauss point column per thread (blocks of 256 columns), chunks of 1 to 8
+# elements along the last direction, longer ones the more columns there are
 @pytest.mark.parametrize("d,p,n", [(2, 1, (1, 1)), (2, 1, (128, 8)), (2, 2, (85, 9)), (2, 2, (86, 7)),
                                    (2, 3, (65, 17)), (2, 4, (3, 16)), (3, 1, (8, 17, 9)), (3, 2, (5, 6, 8)),
-                                   (3, 3, (4, 4, 1)), (3, 3, (5, 3, 10)), (3, 4, (2, 3, 9))])
+                                   (3, 3, (4, 4, 1)), (3, 3, (5, 3, 10)), (3, 4, (2, 3, 9)), (2, 1, (9000, 17)),
+                                   (2, 2, (5000, 70)), (3, 1, (60, 50, 21)), (3, 2, (60, 61, 13))])
 def test_error_norms_columns(ctx, d, p, n):
     prob = _noisy_box(d, p, n, kappa=False)
     dofs, nfree = O.mapper(prob.patches, prob.dir_sides, prob.ifaces)
