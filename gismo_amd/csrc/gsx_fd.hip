@@ -45,6 +45,49 @@ __global__ __launch_bounds__(256) void k_fd_mode(int m0, int m1, int m2, int dir
     y[yo + a + b * ys1 + c * ys2] = acc;
 }
 
+// Slab form (thin boxes, see fd_fused): the block stages the 2D slab of its fixed
+// third index (c for directions 0 and 1, b for direction 2; rows x m0 values) in
+// LDS and each thread computes one output of that slab from it: along direction
+// 0 y[c][b][j] = sum_i M[i][j] x[c][b][i] (the lanes share the slab row and read
+// consecutive columns of M), along directions 1 and 2 y[..][j][a] =
+// sum_i M[i][j] x[..][i][a] (the lanes read consecutive slab entries and share
+// the column of M).
+template <typename T, int DIR>
+__global__ __launch_bounds__(256) void k_fd_slab(int m0, int m1, int m2, const T *__restrict__ M,
+                                                 const T *__restrict__ x, int64_t xo, int64_t xs1, int64_t xs2,
+                                                 T *__restrict__ y, int64_t yo, int64_t ys1, int64_t ys2,
+                                                 const double *__restrict__ l0, const double *__restrict__ l1,
+                                                 const double *__restrict__ l2, double alpha,
+                                                 const CGState *__restrict__ st)
+{
+    extern __shared__ double fd_smem[];
+    T *sX = reinterpret_cast<T *>(fd_smem);
+    if (st && st->done) return;
+    const int fixed = blockIdx.y;
+    const int rows = DIR == 2 ? m2 : m1;
+    const int64_t base = xo + (DIR == 2 ? (int64_t)fixed * xs1 : (int64_t)fixed * xs2);
+    const int64_t rstride = DIR == 2 ? xs2 : xs1;
+    const int n = rows * m0;
+    for (int idx = threadIdx.x; idx < n; idx += 256) {
+        const int r = idx / m0, a = idx % m0;
+        sX[idx] = x[base + a + r * rstride];
+    }
+    __syncthreads();
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= n) return;
+    const int r = idx / m0, q = idx % m0;
+    T acc = 0;
+    if (DIR == 0) {
+        const T *xr = sX + r * m0;
+        for (int i = 0; i < m0; ++i) acc += M[(int64_t)i * m0 + q] * xr[i];
+    } else {
+        for (int i = 0; i < rows; ++i) acc += M[(int64_t)i * rows + r] * sX[i * m0 + q];
+    }
+    const int a = q, b = DIR == 2 ? fixed : r, c = DIR == 2 ? r : fixed;
+    if (l0) acc = (T)((double)acc / (alpha + l0[a] + l1[b] + (l2 ? l2[c] : 0.0)));
+    y[yo + a + (int64_t)b * ys1 + (int64_t)c * ys2] = acc;
+}
+
 // ---------------------------------------------------------------------------
 // Two mode products per launch on the matrix cores.  The products are small
 // GEMMs (65-deep at 64^3 p = 3) whose operands sit in the L2, so the apply is
@@ -209,14 +252,22 @@ __global__ __launch_bounds__(512) void k_fd_column(int m0, int m1, int m2, const
     }
 }
 
-constexpr size_t kFdLds = 64 * 1024;   // dynamic LDS a launch takes without opting in
+constexpr size_t kFdLds = 64 * 1024;       // dynamic LDS a launch takes without opting in
+constexpr size_t kFdSlabLds = 60 * 1024;   // of a slab
 
 bool fd_fused(int d, int m0, int m1, int m2, size_t esz)
 {
     // strips of 16 outputs in LDS; larger boxes take one mode product per launch
-    (void)m1;
-    return 16 * (size_t)fd_strip(m0) * esz <= kFdLds &&
-           (d < 3 || 16 * (size_t)((m2 + 15) / 16 * 16) * esz <= kFdLds);
+    if (16 * (size_t)fd_strip(m0) * esz > kFdLds || (d == 3 && 16 * (size_t)((m2 + 15) / 16 * 16) * esz > kFdLds))
+        return false;
+    // so do thin boxes, whose long sums fall to a few blocks of the fused kernels
+    // and to many of the slab form.  FP64 apply, fused / slabs: 4 x 4 x 128 21 / 32
+    // us, x 200 38 / 35, x 300 69 / 40; 12 x 12 x 300 71 / 50, 16 x 16 x 300 70 / 69;
+    // 200 x 4 x 4 29 / 37, 300 x 4 x 4 54 / 46, 300 x 8 x 8 56 / 57; 2D 200 x 4 25 /
+    // 28, 300 x 4 50 / 36, 300 x 16 53 / 54, 450 x 12 87 / 67
+    const bool slabs = (size_t)(m1 > m2 ? m1 : m2) * m0 * esz <= kFdSlabLds;
+    const int64_t pair_blocks = (int64_t)((m1 + 15) / 16) * m2, column_blocks = ((int64_t)m0 * m1 + 15) / 16;
+    return !(slabs && ((m2 >= 192 && column_blocks <= 16) || (m0 >= 256 && pair_blocks < (d == 3 ? 8 : 2))));
 }
 
 // waves of a block over nt tiles of 16: as many as share the tiles evenly
@@ -278,6 +329,18 @@ hipError_t launch_fd_mode_t(int m0, int m1, int m2, int dir, const T *M, const T
     const int64_t n = (int64_t)m0 * m1 * m2;
     if (n <= 0) return hipSuccess;
     if (dir < 0 || dir > 2) return hipErrorInvalidValue;
+    const int rows = dir == 2 ? m2 : m1;
+    const size_t lds = sizeof(T) * (size_t)rows * m0;
+    if (lds <= kFdSlabLds && (dir == 2 ? m1 : m2) <= 65535) {
+        const dim3 grid((unsigned)((rows * m0 + 255) / 256), (unsigned)(dir == 2 ? m1 : m2));
+#define GSX_SLAB(DIR)                                                                                                  \
+    if (dir == DIR)                                                                                                    \
+        hipLaunchKernelGGL((k_fd_slab<T, DIR>), grid, dim3(256), lds, s, m0, m1, m2, M, x, xo, xs1, xs2, y, yo, ys1,   \
+                           ys2, l0, l1, l2, alpha, st);
+        GSX_SLAB(0) GSX_SLAB(1) GSX_SLAB(2)
+#undef GSX_SLAB
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL((k_fd_mode<T>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, m0, m1, m2, dir, M, x,
                        xo, xs1, xs2, y, yo, ys1, ys2, l0, l1, l2, alpha, st);
     return hipGetLastError();
