@@ -109,10 +109,23 @@ struct CGStep {
     double *hist;
 };
 
+// How a row tile's input is staged in one plane: `entries` in LDS, consecutive
+// lines `line` entries apart, each reaching `halo` entries beyond the tile's
+// span; magic = 2^32 / line rounded up tells the line of an entry (exact below
+// 2^32 / line entries), or 0 where the whole window is one stretch.  plane: rows
+// of a plane of rows (at least 256) where a tile in two of them stages a window
+// for each, else 0.
+struct SpmvStage {
+    int entries, line, halo;
+    unsigned magic;
+    int plane;
+};
+
 // A structured operator's geometry: rows = the free box m0 x m1 x m2, vectors
-// on the padded grid with strides sy, sz; window: sspmv_window.
+// on the padded grid with strides sy, sz.
 struct SpmvGrid {
-    int d, p, nfree, sy, sz, m0, m1, window;
+    int d, p, nfree, sy, sz, m0, m1;
+    SpmvStage stage;
     const int *f2g;
 };
 

@@ -220,10 +220,8 @@ hipError_t launch_scatter_f64_to_grid(int nfree, const int *f2g, const double *s
                                       hipStream_t s);
 hipError_t launch_gather_f64_from_grid(int nfree, const int *f2g, const double *src, double *dst,
                                        hipStream_t s);
-// MODE 1 with st: skipped once the solve stopped or paused at iteration k
-// Grid entries staged for 256 rows: the largest span of a row tile plus its
-// halo in one plane.
-int sspmv_window(int p, int nfree, int m0, int m1, int sy, int sz);
+// How the inputs of the 256-row tiles are staged, for the widest of them.
+SpmvStage sspmv_stage(int d, int p, int nfree, int m0, int m1, int sy, int sz);
 hipError_t launch_sspmv_residual(const SpmvGrid &G, const double *sv, const double *x, double *y, const double *b,
                                  double *part, hipStream_t s);
 hipError_t launch_cg2_spmv_f64(const SpmvGrid &G, const double *sv, const double *z, const double *po, double *pn,

@@ -1046,7 +1046,7 @@ struct StencilOp {
     DevPtr diag64, diag32;
     DevPtr xg, rg, bg, zg, pg[2], tg;         // FP64 (directions by iteration parity)
     DevPtr r32, z32, p32[2], t32, xc32;       // FP32
-    int window = 0;                           // grid entries a row tile's input spans
+    gsx::SpmvStage stage{};                   // of a row tile's input
     DevPtr parts;
 };
 
@@ -1885,7 +1885,7 @@ static gsx_status stencil_prepare(gsx_matrix *A, bool mixed)
         HIP_OK(c, gsx::launch_stencil_diag(n, (int)K, dp<int>(S.f2g), dp<double>(S.s64), dp<double>(S.diag64), s));
         for (DevPtr *v : {&S.xg, &S.rg, &S.bg, &S.zg, &S.pg[0], &S.pg[1], &S.tg})
             HIP_OK(c, gsx::launch_fill_f64(dp<double>(*v), N, 0.0, s));
-        S.window = gsx::sspmv_window(S.p, n, S.m[0], S.m[1], S.nx, S.nx * S.ny);
+        S.stage = gsx::sspmv_stage(S.d, S.p, n, S.m[0], S.m[1], S.nx, S.nx * S.ny);
         S.built = true;
     }
     if (mixed && !S.r32) {
@@ -2134,7 +2134,7 @@ static gsx_status cg_grid(gsx_matrix *A, int precond, double tau, const double *
     double *hist = mixed ? nullptr : dp<double>(w.hist);
     const bool jac = precond == GSX_PREC_JACOBI;
     const int *f2g = dp<int>(S.f2g);
-    const gsx::SpmvGrid G{S.d, S.p, n, S.nx, S.nx * S.ny, S.m[0], S.m[1], S.window, f2g};
+    const gsx::SpmvGrid G{S.d, S.p, n, S.nx, S.nx * S.ny, S.m[0], S.m[1], S.stage, f2g};
     double *xg = dp<double>(S.xg), *rg = dp<double>(S.rg), *bg = dp<double>(S.bg);
     double *zg = dp<double>(S.zg), *tg = dp<double>(S.tg);
     const double *sv = dp<double>(S.s64), *dg = dp<double>(S.diag64);

@@ -152,23 +152,30 @@ __global__ void k_gather_from_grid(int nfree, const int *__restrict__ free2grid,
 // hits the L2.  Neighbours outside the free box contribute 0 (x is 0 there).
 // KIND 2 reads every slot from the row itself, with fewer index operations.
 //
-// The input of a block's 256 rows is staged in LDS, the window of grid entries
-// around them in planes dz and -dz (a few times the rows' number in entries):
-// it is read from memory once instead of once per coefficient, and in MODE 1
-// the direction is formed there, which saves its own launch.  Windows that do
-// not fit (STAGED = false) are read entry by entry.
+// The input of a block's 256 rows is staged in LDS, in planes dz and -dz: it is
+// read from memory once instead of once per coefficient, and in MODE 1 the
+// direction is formed there, which saves its own launch.  Staged is the window
+// of grid entries around the rows, lines -p .. p of them whole, or, where that
+// is less (lines longer than about 150 entries), the 2 p + 1 stretches of lines
+// that the rows reach (SpmvStage).  What does not fit (STAGED = false) is read
+// entry by entry.  With the whole windows alone 32 mixed CG iterations took 7.8
+// ms at 1800^2 elements p = 2 (now 4.3) and 24.8 ms at 2600^2 (8.4), FP64 ones
+// 15.0 (6.7) and 20.0 ms (13.2).
+// Entries are requested ahead of the barrier that they are waited for at: the
+// next tile's window before a tile's last plane is applied and, PLANES, the next
+// planes' first entries before a plane is.
 // Bound by the operator's bytes and the mirrored reads that miss the L2.  64^3
 // elements p = 3: FP32 46.1 us with the direction (49 us in two launches
 // before); FP64 residual 109 us (159 us reading all slots).  75^3 p = 2, FP64:
 // 54.5 us with the direction (89 + 7 us reading all slots).
 // ---------------------------------------------------------------------------
-template <int D, int P, typename V, typename T, int KIND, int MODE, bool STAGED, int Q>
+template <int D, int P, typename V, typename T, int KIND, int MODE, bool STAGED, int Q, int PLANES>
 __global__ __launch_bounds__(256 * Q) void k_cg2_spmv(int nfree, const int *__restrict__ free2grid, int sy, int sz,
                                                   int m0, int m1, const V *__restrict__ sval,
                                                   const T *__restrict__ x, const T *__restrict__ po,
                                                   T *__restrict__ pn, T *__restrict__ y, const T *__restrict__ b,
                                                   double *__restrict__ partial, CGStep cs,
-                                                  CGState *__restrict__ st, int wn)
+                                                  CGState *__restrict__ st, SpmvStage sg)
 {
     extern __shared__ double sp_smem[];
     __shared__ double s[8 * Q];
@@ -180,23 +187,52 @@ __global__ __launch_bounds__(256 * Q) void k_cg2_spmv(int nfree, const int *__re
     constexpr int C = NS / 2, SL = KIND == 0 ? stencil_half(NS) : NS;   // slots of the stored layout
     constexpr int UP = KIND == 0 ? 0 : C;                               // stored index of the centre slot
     static_assert(kStencilTile == 256, "one block applies one row tile");
+    constexpr int UNR = D == 2 && P <= 2 && sizeof(T) == 4 ? 2 : 1;   // lines whose loads are in flight together
     if (MODE == 1 && (st->done || (st->flag_next && st->flag_next <= cs.k))) return;
-    const int halo = P * sy + P;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
-    // the first tile's window is requested before the sums that give beta
-    constexpr int NPRE = MODE == 1 && STAGED ? (Q > 1 ? 1 : 4) : 0, NPA = NPRE ? NPRE : 1;
+    // staged entry i of a plane: entry j of line i / sg.line from w0 on (one line
+    // where sg.magic is 0); with sg.plane a tile's rows from `cut` on, which lie in
+    // the next plane of rows, have a window of their own (w1) behind the first
+    int w0 = 0, w1 = 0, l0 = 0, l1 = 0, behind = 0, total = 0, cut = 0;
+    auto window = [&](int r0) {
+        const int g0 = free2grid[r0], rb = min(r0 + 256, nfree);
+        cut = D == 3 && sg.plane ? min(rb, (r0 / sg.plane + 1) * sg.plane) : rb;
+        w0 = g0 - P * sy - P;
+        l0 = free2grid[cut - 1] - g0 + 1 + 2 * sg.halo;
+        behind = total = sg.magic ? W * sg.line : l0;
+        if (D == 3 && cut < rb) {
+            const int g1 = free2grid[cut];
+            w1 = g1 - P * sy - P;
+            l1 = free2grid[rb - 1] - g1 + 1 + 2 * sg.halo;
+            total += sg.magic ? W * sg.line : l1;
+        }
+    };
+    auto source = [&](int i, bool &in) {
+        const bool second = D == 3 && i >= behind;
+        if (second) i -= behind;
+        const int l = (int)__umulhi((unsigned)i, sg.magic), j = i - l * sg.line;
+        in = j < (second ? l1 : l0);
+        return (second ? w1 : w0) + l * sy + j;
+    };
+    // a tile's window is requested ahead: the first one's before the sums that
+    // give beta, the next one's before the tile's last plane is applied
+    constexpr int NB = D == 2 && sizeof(T) == 4 && P > 1 ? 6 : PLANES > 4 ? PLANES : 4;
+    constexpr int NPRE = MODE == 1 && STAGED ? (Q > 1 ? 1 : NB) : 0, NPA = NPRE ? NPRE : 1;
+    constexpr bool AHEAD = NPRE > 0 && (D == 2 || PLANES > 0);
     T prx[NPA], prp[NPA];
-    int w0 = 0, w1 = 0;
-    if (MODE == 1 && STAGED) {
-        w0 = free2grid[blk * 256] - halo;
-        w1 = free2grid[min(blk * 256 + 255, nfree - 1)] + halo + 1;
+    auto request = [&](int first) {
+        window(first);
 #pragma unroll
         for (int u = 0; u < NPRE; ++u) {
-            const int i = w0 + (int)threadIdx.x + NT * u;
-            prx[u] = i < w1 ? x[i] : (T)0;
-            prp[u] = i < w1 ? po[i] : (T)0;
+            const int i = (int)threadIdx.x + NT * u;
+            bool in;
+            const int g = source(i, in);
+            in = in && i < total;
+            prx[u] = in ? x[g] : (T)0;
+            prp[u] = in ? po[g] : (T)0;
         }
-    }
+    };
+    if (NPRE > 0) request(blk * 256);
     T tb = 0;
     if (MODE == 1) {
         double rr = 0.0, rzn = 0.0;
@@ -236,84 +272,129 @@ __global__ __launch_bounds__(256 * Q) void k_cg2_spmv(int nfree, const int *__re
         if (MODE == 2) return x[i];
         return first ? x[i] : x[i] + tb * po[i];
     };
-    T *sA = reinterpret_cast<T *>(sp_smem), *sB = sA + wn;
+    T *sA = reinterpret_cast<T *>(sp_smem), *sB = sA + sg.entries;
     double contrib = 0.0;
     for (int r0 = blk * 256; r0 < nfree; r0 += gridDim.x * 256) {
         const int r = r0 + t;
-        const bool act = r < nfree;
+        const bool act = r < nfree, pre = NPRE > 0 && (AHEAD || r0 == blk * 256);
+        if (STAGED && !pre) window(r0);
         const int g = act ? free2grid[r] : 0;
         const int ia = r % m0, ib = (r / m0) % m1, ic = (D == 3) ? r / (m0 * m1) : 0;
         const V *vb = sval + stencil_index(UP, r, SL);   // from the centre slot up
-        const bool pre = NPRE > 0 && r0 == blk * 256;
-        int c = 0;
-        if (STAGED) {
-            w0 = free2grid[r0] - halo;
-            w1 = free2grid[min(r0 + 255, nfree - 1)] + halo + 1;
-            c = g - w0;
-        }
+        // entry (dy, dx) around row r: c + dy sg.line + dx
+        const int c = g - P * sy + P * sg.line - (D == 3 && r >= cut ? w1 - behind : w0);
         T acc = 0, own = 0;
+        // the first entries of planes dz and -dz, requested before the plane
+        // before them is applied
+        constexpr int NPL = PLANES ? (Q > 1 ? 1 : PLANES) : 1;
+        T ax[NPL], ap[NPL], mx[NPL], mp[NPL];
+        auto request_plane = [&](int dz) {
+#pragma unroll
+            for (int u = 0; u < NPL; ++u) {
+                bool in;
+                const int i = (int)threadIdx.x + NT * u, from = source(i, in);
+                in = in && i < total;
+                ax[u] = in ? x[from + dz * sz] : (T)0;
+                mx[u] = in ? x[from - dz * sz] : (T)0;
+                if (MODE == 1) {
+                    ap[u] = in ? po[from + dz * sz] : (T)0;
+                    mp[u] = in ? po[from - dz * sz] : (T)0;
+                }
+            }
+        };
         auto plane = [&](int dz) {
             if (STAGED) {
                 __syncthreads();   // the readers of the last planes are done
-                int i = w0 + threadIdx.x;
+                int i = threadIdx.x;
                 if (pre && dz == 0) {
 #pragma unroll
                     for (int u = 0; u < NPRE; ++u, i += NT)
-                        if (i < w1) sA[i - w0] = first ? prx[u] : prx[u] + tb * prp[u];
+                        if (i < total) sA[i] = first ? prx[u] : prx[u] + tb * prp[u];
                 }
-                for (; i < w1; i += NT) {
-                    sA[i - w0] = input(i + dz * sz);
-                    if (D == 3 && dz > 0) sB[i - w0] = input(i - dz * sz);
+                if (PLANES && dz > 0) {
+#pragma unroll
+                    for (int u = 0; u < NPL; ++u, i += NT)
+                        if (i < total) {
+                            sA[i] = MODE == 2 || first ? ax[u] : ax[u] + tb * ap[u];
+                            sB[i] = MODE == 2 || first ? mx[u] : mx[u] + tb * mp[u];
+                        }
+                }
+                // loads in batches, all of one in flight
+                constexpr int U = Q > 1 ? 2 : 4;
+                for (; i < total; i += U * NT) {
+                    T a[U], m[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        bool in;
+                        const int from = source(i + u * NT, in);
+                        in = in && i + u * NT < total;
+                        a[u] = in ? input(from + dz * sz) : (T)0;
+                        m[u] = D == 3 && dz > 0 && in ? input(from - dz * sz) : (T)0;
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        if (i + u * NT >= total) break;
+                        sA[i + u * NT] = a[u];
+                        if (D == 3 && dz > 0) sB[i + u * NT] = m[u];
+                    }
                 }
                 __syncthreads();
             }
         };
-        // entry at grid offset o of plane +dz / -dz
-        auto xa = [&](int dz, int o) -> T { return STAGED ? sA[c + o] : input(g + dz * sz + o); };
-        auto xm = [&](int dz, int o) -> T {
-            return STAGED ? (D == 3 && dz > 0 ? sB[c + o] : sA[c + o]) : input(g - dz * sz + o);
+        // entry (dy, dx) around the row in plane +dz / -dz
+        auto xa = [&](int dz, int dy, int dx) -> T {
+            return STAGED ? sA[c + dy * sg.line + dx] : input(g + dz * sz + dy * sy + dx);
+        };
+        auto xm = [&](int dz, int dy, int dx) -> T {
+            if (!STAGED) return input(g - dz * sz + dy * sy + dx);
+            return D == 3 && dz > 0 ? sB[c + dy * sg.line + dx] : sA[c + dy * sg.line + dx];
         };
         // upper line (dz, dy) and its mirror (-dz, -dy)
         auto line = [&](int dz, int dy) {
             const int h0 = (D == 3 ? ((dz + P) * W + (dy + P)) * W : (dy + P) * W) - C;   // (dz, dy, -P) from the centre
 #pragma unroll
-            for (int dx = -P; dx <= P; ++dx) acc += (T)vb[(h0 + dx + P) * kStencilTile] * xa(dz, dy * sy + dx);
+            for (int dx = -P; dx <= P; ++dx) acc += (T)vb[(h0 + dx + P) * kStencilTile] * xa(dz, dy, dx);
             if (KIND == 2) {
 #pragma unroll
                 for (int dx = -P; dx <= P; ++dx)
-                    acc += (T)vb[-(h0 - dx + P) * kStencilTile] * xm(dz, dx - dy * sy);
+                    acc += (T)vb[-(h0 - dx + P) * kStencilTile] * xm(dz, -dy, dx);
             } else {
                 const bool okyz = ib - dy >= 0 && ib - dy < m1 && ic - dz >= 0;
                 const int rm = r - m0 * (dy + m1 * dz);
 #pragma unroll
                 for (int dx = -P; dx <= P; ++dx) {
                     const bool ok = okyz && ia + dx >= 0 && ia + dx < m0;
-                    acc += (T)(ok ? sval[stencil_index(UP + h0 - dx + P, rm + dx, SL)] : (V)0) * xm(dz, dx - dy * sy);
+                    acc += (T)(ok ? sval[stencil_index(UP + h0 - dx + P, rm + dx, SL)] : (V)0) * xm(dz, -dy, dx);
                 }
             }
         };
         plane(0);
+        const bool more = AHEAD && r0 + (int)gridDim.x * 256 < nfree;
+        if (D == 2 && more) request(r0 + gridDim.x * 256);
+        if (PLANES) request_plane(1);
         if (act) {
-            own = xa(0, 0);
+            own = xa(0, 0, 0);
             // centre line: own slots dx = 0..P, mirrors dx = -P..-1
             if (q == 0) {
 #pragma unroll
-                for (int dx = 0; dx <= P; ++dx) acc += (T)vb[dx * kStencilTile] * xa(0, dx);
+                for (int dx = 0; dx <= P; ++dx) acc += (T)vb[dx * kStencilTile] * xa(0, 0, dx);
 #pragma unroll
                 for (int dx = -P; dx < 0; ++dx) {
-                    if (KIND == 2) acc += (T)vb[dx * kStencilTile] * xa(0, dx);
-                    else acc += (T)(ia + dx >= 0 ? sval[stencil_index(UP - dx, r + dx, SL)] : (V)0) * xa(0, dx);
+                    if (KIND == 2) acc += (T)vb[dx * kStencilTile] * xa(0, 0, dx);
+                    else acc += (T)(ia + dx >= 0 ? sval[stencil_index(UP - dx, r + dx, SL)] : (V)0) * xa(0, 0, dx);
                 }
             }
-#pragma unroll 1
+#pragma unroll(UNR)
             for (int dy = Q > 1 && q == 0 ? Q : (Q > 1 ? q : 1); dy <= P; dy += Q) line(0, dy);
         }
         if (D == 3) {
 #pragma unroll 1
             for (int dz = 1; dz <= P; ++dz) {
                 plane(dz);
+                if (PLANES && dz < P) request_plane(dz + 1);
+                if (dz == P && more) request(r0 + gridDim.x * 256);
                 if (act) {
-#pragma unroll 1
+#pragma unroll(UNR)
                     for (int dy = -P + (q + dz) % Q; dy <= P; dy += Q) line(dz, dy);
                 }
             }
@@ -540,13 +621,35 @@ hipError_t launch_gather_f64_from_grid(int nfree, const int *f2g, const double *
     return hipGetLastError();
 }
 
-int sspmv_window(int p, int nfree, int m0, int m1, int sy, int sz)
+constexpr size_t kWindowLds = 64 * 1024;   // LDS of a tile's staged input
+
+SpmvStage sspmv_stage(int d, int p, int nfree, int m0, int m1, int sy, int sz)
 {
     auto grid = [&](int r) { return (int64_t)(r % m0) + (int64_t)sy * ((r / m0) % m1) + (int64_t)sz * (r / (m0 * m1)); };
-    int64_t w = 0;
-    for (int r0 = 0; r0 < nfree; r0 += 256) w = std::max(w, grid(std::min(r0 + 255, nfree - 1)) - grid(r0));
-    w += 1 + 2 * (int64_t)(p * sy + p);
-    return (int)std::min<int64_t>(w, INT32_MAX);
+    // span: grid entries that the rows of a tile in one plane reach over, whole:
+    // the sum over its planes
+    auto stage = [&](int plane) {
+        int64_t span = 0, whole = 0, parts = 1;
+        const int64_t halo = (int64_t)p * sy + p;
+        for (int64_t r0 = 0; r0 < nfree; r0 += 256) {
+            const int64_t e = std::min<int64_t>(r0 + 256, nfree);
+            int64_t cut = plane ? std::min(e, (r0 / plane + 1) * (int64_t)plane) : e;
+            const int64_t a = grid((int)cut - 1) - grid((int)r0) + 1;
+            const int64_t b = cut < e ? grid((int)e - 1) - grid((int)cut) + 1 : 0;
+            span = std::max({span, a, b});
+            whole = std::max(whole, a + 2 * halo + (b ? b + 2 * halo : 0));
+            if (b) parts = 2;
+        }
+        const int64_t line = span + 2 * p, lines = parts * line * (2 * p + 1);
+        if (lines < whole)
+            return SpmvStage{(int)std::min<int64_t>(lines, INT32_MAX), (int)line, p,
+                             (unsigned)(((uint64_t)1 << 32) / (uint64_t)line + 1), plane};
+        return SpmvStage{(int)std::min<int64_t>(whole, INT32_MAX), sy, (int)halo, 0u, plane};
+    };
+    SpmvStage g = stage(0);
+    const int plane = m0 * m1;
+    if (d == 3 && plane >= 256 && (size_t)g.entries * 2 * sizeof(double) > kWindowLds) g = stage(plane);
+    return g;
 }
 
 // An FP64 operator of at most this many bytes (all slots) is read whole: it
@@ -555,7 +658,6 @@ int sspmv_window(int p, int nfree, int m0, int m1, int sy, int sz)
 // 64^2 p = 2 (0.8 MB) 1788 / 1967 us, 18^3 p = 3 (20 MB) 3662 / 4392 us;
 // 75^3 p = 2 (422 MB) 12.5 / 7.4 ms.
 constexpr int64_t kMirrorBytes = (int64_t)24 << 20;
-constexpr size_t kWindowLds = 64 * 1024;
 
 // A 3D operator of at most a tile per CU leaves most of the chip idle: four
 // groups of 256 threads then share a tile's stencil lines and one sums the
@@ -566,23 +668,40 @@ constexpr size_t kWindowLds = 64 * 1024;
 // p = 2 1.50 / 1.66 ms, 300^2 p = 4 mixed 8.4 / 10.4.
 constexpr int kSplit = 4, kSplitTiles = 256;
 
+// Entries per thread requested ahead for the next planes of a 3D tile: they hide
+// two waits a plane, at registers.  Up to a tile for each of the four blocks a CU
+// holds, waits bound the kernel; with more tiles only the smallest stencils gain.
+// 32 CG iterations without / with them: 50^3 p = 3 mixed (518 tiles) 2.10 / 1.91
+// ms, 100 x 30 x 30 p = 2 mixed 1.20 / 1.10, 45^3 p = 2 FP64 1.05 / 0.96; 64^3 p =
+// 3 mixed (1073 tiles) 3.08 / 3.41, 64^3 p = 2 FP64 (1024) 1.55 / 1.73, mixed 1.60
+// / 1.49, 100^3 p = 1 mixed 2.11 / 1.96.  Six entries instead of four: 200 x 200 x
+// 3 p = 2 mixed 1.31 / 1.23, 64^3 p = 2 mixed 1.50 / 1.83.
+constexpr int kPlaneTiles = 1000;
+
 template <int D, int P, typename V, typename T, int KIND, int MODE>
 static hipError_t sspmv_launch(const SpmvGrid &G, const V *sv, const T *x, const T *po, T *pn, T *y, const T *b,
                                double *part, const CGStep &cs, CGState *st, hipStream_t s)
 {
     const dim3 grid(sspmv_blocks(G.nfree));
-    const size_t lds = (size_t)G.window * (D == 3 ? 2 : 1) * sizeof(T);
+    const size_t lds = (size_t)G.stage.entries * (D == 3 ? 2 : 1) * sizeof(T);
     const bool staged = lds <= kWindowLds;
-#define GSX_Q(STAGED, Q)                                                                                              \
-    hipLaunchKernelGGL((k_cg2_spmv<D, P, V, T, KIND, MODE, STAGED, Q>), grid, dim3(256 * Q), STAGED ? lds : 0, s,     \
-                       G.nfree, G.f2g, G.sy, G.sz, G.m0, G.m1, sv, x, po, pn, y, b, part, cs, st, STAGED ? G.window : 0)
+    constexpr bool f32 = sizeof(T) == 4;
+    constexpr int FEW = D == 2 ? 0 : f32 && P == 2 ? 6 : f32 || P <= 2 ? 4 : 0;
+    constexpr int MANY = D == 2 ? 0 : P == 1 ? 2 : f32 && P == 2 ? 4 : 0;
+#define GSX_Q(STAGED, Q, PLANES)                                                                                      \
+    hipLaunchKernelGGL((k_cg2_spmv<D, P, V, T, KIND, MODE, STAGED, Q, PLANES>), grid, dim3(256 * Q),                  \
+                       STAGED ? lds : 0, s, G.nfree, G.f2g, G.sy, G.sz, G.m0, G.m1, sv, x, po, pn, y, b, part, cs,    \
+                       st, G.stage)
     if (D == 3 && (int)grid.x <= kSplitTiles) {
         constexpr int Q = D == 3 ? kSplit : 1;
-        if (staged) GSX_Q(true, Q);
-        else GSX_Q(false, Q);
+        if (staged) GSX_Q(true, Q, FEW);
+        else GSX_Q(false, Q, 0);
+    } else if (!staged) {
+        GSX_Q(false, 1, 0);
+    } else if ((int)grid.x <= kPlaneTiles) {
+        GSX_Q(true, 1, FEW);
     } else {
-        if (staged) GSX_Q(true, 1);
-        else GSX_Q(false, 1);
+        GSX_Q(true, 1, MANY);
     }
 #undef GSX_Q
     return hipGetLastError();

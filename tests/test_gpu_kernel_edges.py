@@ -97,7 +97,10 @@ def test_fd_pcg_fp32_tiles(ctx, d, p, n):
 @pytest.mark.parametrize("d,p,n", [(2, 1, (2, 2)), (2, 2, (16, 17)), (2, 4, (300, 9)), (2, 1, (740, 731)),
                                    (3, 1, (9, 8, 7)), (3, 2, (3, 3, 600)), (3, 3, (2, 2, 450)), (3, 3, (19, 18, 19)),
                                    (3, 3, (21, 19, 20)), (3, 4, (13, 11, 12)), (3, 4, (2, 40, 3)),
-                                   (3, 1, (42, 41, 43)), (3, 2, (42, 40, 41))])
+                                   (3, 1, (42, 41, 43)), (3, 2, (42, 40, 41)),
+                                   (2, 2, (700, 40)), (2, 3, (1100, 500)), (2, 4, (160, 30)), (3, 1, (900, 5, 4)),
+                                   (3, 2, (700, 6, 5)), (3, 3, (130, 40, 3)), (3, 4, (300, 3, 2)),
+                                   (3, 2, (1500, 40, 3)), (3, 1, (700, 30, 30)), (3, 1, (100, 90, 80))])
 def test_structured_cg_tiles(ctx, d, p, n):
     """FP64 and mixed solves on the structured operator reach the CSR
     operator's solution in its iterations."""
