@@ -687,7 +687,8 @@ __global__ __launch_bounds__(256) void k_geo3d(const PatchDev *__restrict__ patc
     const int t = threadIdx.x;
     const int Gx = bx.g[0], Gy = bx.g[1], Gz = bx.g[2];
     const double *tx = tab + bx.toff[0], *ty = tab + bx.toff[1], *tz = tab + bx.toff[2];
-    const int e0 = blockIdx.y * ch, e1 = min(e0 + ch, bx.nel[2]);
+    const int ncb = (int)(((int64_t)Gx * Gy + 255) / 256), kz = blockIdx.x / ncb;   // chunks after columns
+    const int e0 = kz * ch, e1 = min(e0 + ch, bx.nel[2]);
     for (int k = t; k < (e1 - e0) * NB1 * NB1; k += 256) {
         const int q = k / NB1, m = k % NB1;
         const int64_t g = (int64_t)e0 * NB1 + q;
@@ -696,7 +697,7 @@ __global__ __launch_bounds__(256) void k_geo3d(const PatchDev *__restrict__ patc
         if (m == 0) sW[q] = tz[2 * (int64_t)Gz * NB1 + g];
     }
     __syncthreads();
-    const int64_t col = (int64_t)blockIdx.x * 256 + t;
+    const int64_t col = (int64_t)(blockIdx.x % ncb) * 256 + t;
     double dmin = 1e300;
     if (col < (int64_t)Gx * Gy) {
         const int gy = (int)(col % Gy), gx = (int)(col / Gy);
@@ -734,7 +735,7 @@ __global__ __launch_bounds__(256) void k_geo3d(const PatchDev *__restrict__ patc
                 }
             }
         };
-        double *r1 = R1 + ((int64_t)blockIdx.y * (ch + P) * Gx + gx) * Gy + gy;
+        double *r1 = R1 + ((int64_t)kz * (ch + P) * Gx + gx) * Gy + gy;
         const int64_t r1s = (int64_t)Gx * Gy;
 #pragma unroll
         for (int m = 0; m < NB1; ++m) acc[m] = 0.0;
@@ -812,7 +813,7 @@ __global__ __launch_bounds__(256) void k_geo3d(const PatchDev *__restrict__ patc
     for (int off = 32; off > 0; off >>= 1) dmin = fmin(dmin, __shfl_xor(dmin, off, 64));
     if ((t & 63) == 0) sMin[t >> 6] = dmin;
     __syncthreads();
-    if (t == 0) detmin[blockIdx.y * gridDim.x + blockIdx.x] = fmin(fmin(sMin[0], sMin[1]), fmin(sMin[2], sMin[3]));
+    if (t == 0) detmin[blockIdx.x] = fmin(fmin(sMin[0], sMin[1]), fmin(sMin[2], sMin[3]));
 }
 
 // Load vector of the free rows from k_geo3d's z sums: a block takes up to 64
@@ -1039,7 +1040,7 @@ hipError_t launch_sf_assemble(int p, const PatchDev *patches, const GaussTab &gt
     const int G = bx.g[0] + bx.g[1] + bx.g[2];
     const int ch = sf_chunk(p, bx.nel);
     const int64_t nload = (int64_t)((bx.m[0] + 63) / 64) * bx.m[1] * bx.m[2];
-    const dim3 ggeo((unsigned)(((int64_t)bx.g[0] * bx.g[1] + 255) / 256), (unsigned)((bx.nel[2] + ch - 1) / ch));
+    const dim3 ggeo((unsigned)sf_det_count(p, bx.nel));
 #define GSX_SF(PP)                                                                                              \
     if (p == PP) {                                                                                              \
         hipLaunchKernelGGL((k_sf_tables<PP>), dim3((G + 255) / 256), dim3(256), 0, s, patches, gt, tab, bx.g[0], \

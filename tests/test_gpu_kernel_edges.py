@@ -588,3 +588,27 @@ def test_hierarchy_without_room_for_its_slices(ctx, prec):
     assert np.linalg.norm(out[0][2] - out[1][2]) <= 1e-6 * np.linalg.norm(out[0][2])
     for o in (r, b, A, gp):
         o.close()
+
+
+def test_row_assembly_of_a_long_box(ctx):
+    """More chunks of elements along z (65,600 of 8) than a grid's second
+    dimension takes blocks."""
+    n = (1, 1, 524800)
+    P = problems.box_patch(3, 2, n, hi=[1.0, 1.0, 4100.0])
+    P.kappa = 1.0 + 0.5 * np.sin(np.arange(P.nelem))
+    P.fkind = 1
+    gp = gsx.Problem(ctx, problems.Problem([P], problems.all_sides(3), []))
+    out = []
+    for mode in (0, gsx.ASM_ELEMENTWISE):
+        A, b = gp.assemble(gsx.PATTERN_FULL | gsx.ASM_CSR_ONLY | mode)
+        out.append((*A.download(), b.download(), gp.min_detj()))
+        A.close()
+        b.close()
+    r, e = out
+    assert np.array_equal(r[0], e[0]) and np.array_equal(r[1], e[1])
+    # the Jacobian's z entries are differences of coordinates up to 4100 over an
+    # element of 1/128: 4100 128 eps = 1e-10 of them in either path
+    assert np.abs(r[2] - e[2]).max() <= 4e-10 * np.abs(e[2]).max()
+    assert np.abs(r[3] - e[3]).max() <= 4e-10 * np.abs(e[3]).max()
+    assert r[4] == pytest.approx(e[4], rel=4e-10)
+    gp.close()
