@@ -91,9 +91,11 @@ def test_fd_pcg_fp32_tiles(ctx, d, p, n):
 
 
 # the structured CG: row tiles of 256 with staged windows, all slots read below
-# 24 MB of operator and mirrored upper ones above, direct reads where a window
-# exceeds the LDS (the flat boxes), several tiles a block above 524,288 rows,
-# four groups of threads a tile for 3D operators of up to 256 tiles
+# 24 MB of operator and mirrored upper ones above, stretches of lines where these
+# are long, a window for each plane of a tile where one for both is too large,
+# direct reads where neither fits the LDS, several tiles a block above 524,288
+# rows, four groups of threads a tile for 3D operators of up to 256 tiles, planes
+# requested ahead in up to 1000
 @pytest.mark.parametrize("d,p,n", [(2, 1, (2, 2)), (2, 2, (16, 17)), (2, 4, (300, 9)), (2, 1, (740, 731)),
                                    (3, 1, (9, 8, 7)), (3, 2, (3, 3, 600)), (3, 3, (2, 2, 450)), (3, 3, (19, 18, 19)),
                                    (3, 3, (21, 19, 20)), (3, 4, (13, 11, 12)), (3, 4, (2, 40, 3)),
