@@ -881,11 +881,13 @@ gsx_status gsx_problem_create(gsx_ctx *c, int32_t npatch, const gsx_patch_desc *
             const int g = P->dofs[P->boff[k] + l];
             if (g < nfree) {
                 const int o = fillp[g]++;
-                P->odd_glue = P->odd_glue || (o > occ_cnt[g] && occ_patch[o - 1] == k);
                 occ_patch[o] = k;
                 occ_local[o] = l;
             }
         }
+    for (int g = P->nsingle; g < nfree; ++g)   // occurrences come in patch order
+        for (int o = occ_cnt[g] + 1; o < occ_cnt[g + 1]; ++o)
+            P->odd_glue = P->odd_glue || occ_patch[o - 1] == occ_patch[o];
     P->d_occ_ptr = dalloc(c, sizeof(int) * (nfree + 1));
     P->d_occ_patch = dalloc(c, sizeof(int) * std::max<size_t>(1, occ_patch.size()));
     P->d_occ_local = dalloc(c, sizeof(int64_t) * std::max<size_t>(1, occ_local.size()));

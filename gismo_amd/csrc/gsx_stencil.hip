@@ -157,7 +157,7 @@ __global__ void k_gather_from_grid(int nfree, const int *__restrict__ free2grid,
 // direction is formed there, which saves its own launch.  Staged is the window
 // of grid entries around the rows, lines -p .. p of them whole, or, where that
 // is less (lines longer than about 150 entries), the 2 p + 1 stretches of lines
-// that the rows reach (SpmvStage).  What does not fit (STAGED = false) is read
+// that the rows reach (SpmvStage).  What does not fit (STAGED = 0) is read
 // entry by entry.  With the whole windows alone 32 mixed CG iterations took 7.8
 // ms at 1800^2 elements p = 2 (now 4.3) and 24.8 ms at 2600^2 (8.4), FP64 ones
 // 15.0 (6.7) and 20.0 ms (13.2).
@@ -169,8 +169,9 @@ __global__ void k_gather_from_grid(int nfree, const int *__restrict__ free2grid,
 // before); FP64 residual 109 us (159 us reading all slots).  75^3 p = 2, FP64:
 // 54.5 us with the direction (89 + 7 us reading all slots).
 // ---------------------------------------------------------------------------
-template <int D, int P, typename V, typename T, int KIND, int MODE, bool STAGED, int Q, int PLANES>
-__global__ __launch_bounds__(256 * Q) void k_cg2_spmv(int nfree, const int *__restrict__ free2grid, int sy, int sz,
+template <int D, int P, typename V, typename T, int KIND, int MODE, int STAGED, int Q, int PLANES>
+// (windows of degree 4 in FP64: within the registers of four waves a SIMD)
+__global__ __launch_bounds__(256 * Q, D == 3 && P == 4 && sizeof(T) == 8 && STAGED < 2 ? 4 : 1) void k_cg2_spmv(int nfree, const int *__restrict__ free2grid, int sy, int sz,
                                                   int m0, int m1, const V *__restrict__ sval,
                                                   const T *__restrict__ x, const T *__restrict__ po,
                                                   T *__restrict__ pn, T *__restrict__ y, const T *__restrict__ b,
@@ -187,27 +188,32 @@ __global__ __launch_bounds__(256 * Q) void k_cg2_spmv(int nfree, const int *__re
     constexpr int C = NS / 2, SL = KIND == 0 ? stencil_half(NS) : NS;   // slots of the stored layout
     constexpr int UP = KIND == 0 ? 0 : C;                               // stored index of the centre slot
     static_assert(kStencilTile == 256, "one block applies one row tile");
-    constexpr int UNR = D == 2 && P <= 2 && sizeof(T) == 4 ? 2 : 1;   // lines whose loads are in flight together
+    constexpr int UNR = STAGED == 2 && D == 2 && PLANES && P <= 2 && sizeof(T) == 4 ? 2 : 1;   // lines whose loads are in flight together
     if (MODE == 1 && (st->done || (st->flag_next && st->flag_next <= cs.k))) return;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
-    // staged entry i of a plane: entry j of line i / sg.line from w0 on (one line
-    // where sg.magic is 0); with sg.plane a tile's rows from `cut` on, which lie in
-    // the next plane of rows, have a window of their own (w1) behind the first
+    // staged entry i of a plane: entry i from w0 on.  STAGED = 2: entry j of line
+    // i / sg.line from w0 on (one line where sg.magic is 0); with sg.plane a tile's
+    // rows from `cut` on, which lie in the next plane of rows, have a window of
+    // their own (w1) behind the first
+    constexpr bool LINES = STAGED == 2;
+    const int line_stride = LINES ? sg.line : sy, halo = LINES ? sg.halo : P * sy + P;
     int w0 = 0, w1 = 0, l0 = 0, l1 = 0, behind = 0, total = 0, cut = 0;
     auto window = [&](int r0) {
         const int g0 = free2grid[r0], rb = min(r0 + 256, nfree);
-        cut = D == 3 && sg.plane ? min(rb, (r0 / sg.plane + 1) * sg.plane) : rb;
+        cut = LINES && D == 3 && sg.plane ? min(rb, (r0 / sg.plane + 1) * sg.plane) : rb;
         w0 = g0 - P * sy - P;
-        l0 = free2grid[cut - 1] - g0 + 1 + 2 * sg.halo;
-        behind = total = sg.magic ? W * sg.line : l0;
-        if (D == 3 && cut < rb) {
+        l0 = free2grid[cut - 1] - g0 + 1 + 2 * halo;
+        behind = total = LINES && sg.magic ? W * sg.line : l0;
+        if (LINES && D == 3 && cut < rb) {
             const int g1 = free2grid[cut];
             w1 = g1 - P * sy - P;
-            l1 = free2grid[rb - 1] - g1 + 1 + 2 * sg.halo;
+            l1 = free2grid[rb - 1] - g1 + 1 + 2 * halo;
             total += sg.magic ? W * sg.line : l1;
         }
     };
     auto source = [&](int i, bool &in) {
+        in = true;
+        if (!LINES) return w0 + i;
         const bool second = D == 3 && i >= behind;
         if (second) i -= behind;
         const int l = (int)__umulhi((unsigned)i, sg.magic), j = i - l * sg.line;
@@ -216,9 +222,9 @@ __global__ __launch_bounds__(256 * Q) void k_cg2_spmv(int nfree, const int *__re
     };
     // a tile's window is requested ahead: the first one's before the sums that
     // give beta, the next one's before the tile's last plane is applied
-    constexpr int NB = D == 2 && sizeof(T) == 4 && P > 1 ? 6 : PLANES > 4 ? PLANES : 4;
+    constexpr int NB = LINES && D == 2 && PLANES && sizeof(T) == 4 && P > 1 ? 6 : PLANES > 4 ? PLANES : 4;
     constexpr int NPRE = MODE == 1 && STAGED ? (Q > 1 ? 1 : NB) : 0, NPA = NPRE ? NPRE : 1;
-    constexpr bool AHEAD = NPRE > 0 && (D == 2 || PLANES > 0);
+    constexpr bool AHEAD = NPRE > 0 && PLANES > 0 && (D == 3 || LINES);
     T prx[NPA], prp[NPA];
     auto request = [&](int first) {
         window(first);
@@ -281,8 +287,8 @@ __global__ __launch_bounds__(256 * Q) void k_cg2_spmv(int nfree, const int *__re
         const int g = act ? free2grid[r] : 0;
         const int ia = r % m0, ib = (r / m0) % m1, ic = (D == 3) ? r / (m0 * m1) : 0;
         const V *vb = sval + stencil_index(UP, r, SL);   // from the centre slot up
-        // entry (dy, dx) around row r: c + dy sg.line + dx
-        const int c = g - P * sy + P * sg.line - (D == 3 && r >= cut ? w1 - behind : w0);
+        // entry (dy, dx) around row r: c + dy line_stride + dx
+        const int c = g - P * sy + P * line_stride - (LINES && D == 3 && r >= cut ? w1 - behind : w0);
         T acc = 0, own = 0;
         // the first entries of planes dz and -dz, requested before the plane
         // before them is applied
@@ -319,8 +325,9 @@ __global__ __launch_bounds__(256 * Q) void k_cg2_spmv(int nfree, const int *__re
                             sB[i] = MODE == 2 || first ? mx[u] : mx[u] + tb * mp[u];
                         }
                 }
-                // loads in batches, all of one in flight
-                constexpr int U = Q > 1 ? 2 : 4;
+                // stretches of lines, more entries than a window has, in batches of
+                // loads; a window's without the registers of one
+                constexpr int U = !LINES ? 1 : Q > 1 ? 2 : 4;
                 for (; i < total; i += U * NT) {
                     T a[U], m[U];
 #pragma unroll
@@ -343,11 +350,11 @@ __global__ __launch_bounds__(256 * Q) void k_cg2_spmv(int nfree, const int *__re
         };
         // entry (dy, dx) around the row in plane +dz / -dz
         auto xa = [&](int dz, int dy, int dx) -> T {
-            return STAGED ? sA[c + dy * sg.line + dx] : input(g + dz * sz + dy * sy + dx);
+            return STAGED ? sA[c + dy * line_stride + dx] : input(g + dz * sz + dy * sy + dx);
         };
         auto xm = [&](int dz, int dy, int dx) -> T {
             if (!STAGED) return input(g - dz * sz + dy * sy + dx);
-            return D == 3 && dz > 0 ? sB[c + dy * sg.line + dx] : sA[c + dy * sg.line + dx];
+            return D == 3 && dz > 0 ? sB[c + dy * line_stride + dx] : sA[c + dy * line_stride + dx];
         };
         // upper line (dz, dy) and its mirror (-dz, -dy)
         auto line = [&](int dz, int dy) {
@@ -667,14 +674,18 @@ constexpr int64_t kMirrorBytes = (int64_t)24 << 20;
 // 6.5 / 7.5, 60^3 p = 3 mixed 8.6 / 12.0.  2D stencils have too few lines: 64^2
 // p = 2 1.50 / 1.66 ms, 300^2 p = 4 mixed 8.4 / 10.4.
 constexpr int kSplit = 4, kSplitTiles = 256;
+// One such block runs on a CU, so its window may take more LDS: 1 x 1 x 500 p = 4
+// FP64, 32 iterations, entry by entry 2.62 ms, staged 1.40; 1 x 1 x 600 p = 3 1.70
+// and 1.21.
+constexpr size_t kSplitLds = 128 * 1024;
 
 // Entries per thread requested ahead for the next planes of a 3D tile: they hide
 // two waits a plane, at registers.  Up to a tile for each of the four blocks a CU
-// holds, waits bound the kernel; with more tiles only the smallest stencils gain.
+// holds, waits bound the kernel; with more tiles only p = 2 in FP32 gains.
 // 32 CG iterations without / with them: 50^3 p = 3 mixed (518 tiles) 2.10 / 1.91
 // ms, 100 x 30 x 30 p = 2 mixed 1.20 / 1.10, 45^3 p = 2 FP64 1.05 / 0.96; 64^3 p =
 // 3 mixed (1073 tiles) 3.08 / 3.41, 64^3 p = 2 FP64 (1024) 1.55 / 1.73, mixed 1.60
-// / 1.49, 100^3 p = 1 mixed 2.11 / 1.96.  Six entries instead of four: 200 x 200 x
+// / 1.49, 100^3 p = 1 mixed 1.81 / 2.00.  Six entries instead of four: 200 x 200 x
 // 3 p = 2 mixed 1.31 / 1.23, 64^3 p = 2 mixed 1.50 / 1.83.
 constexpr int kPlaneTiles = 1000;
 
@@ -684,25 +695,34 @@ static hipError_t sspmv_launch(const SpmvGrid &G, const V *sv, const T *x, const
 {
     const dim3 grid(sspmv_blocks(G.nfree));
     const size_t lds = (size_t)G.stage.entries * (D == 3 ? 2 : 1) * sizeof(T);
-    const bool staged = lds <= kWindowLds;
+    // 0: entry by entry; 1: a window; 2: stretches of lines, or a window per plane
+    const bool split = D == 3 && (int)grid.x <= kSplitTiles;
+    const int staged = lds > (split ? kSplitLds : kWindowLds) ? 0 : G.stage.magic || G.stage.plane ? 2 : 1;
     constexpr bool f32 = sizeof(T) == 4;
     constexpr int FEW = D == 2 ? 0 : f32 && P == 2 ? 6 : f32 || P <= 2 ? 4 : 0;
-    constexpr int MANY = D == 2 ? 0 : P == 1 ? 2 : f32 && P == 2 ? 4 : 0;
+    // 2D: the next tile's stretches are requested where a block has further tiles
+    // (2600^2 p = 2 mixed 9.3 / 8.4 ms); below, the registers of it cost a wave per
+    // SIMD (600^2 p = 2 mixed 1.04 ms without, 1.12 with them)
+    constexpr int MANY = D == 2 ? 1 : f32 && P == 2 ? 4 : 0;
 #define GSX_Q(STAGED, Q, PLANES)                                                                                      \
     hipLaunchKernelGGL((k_cg2_spmv<D, P, V, T, KIND, MODE, STAGED, Q, PLANES>), grid, dim3(256 * Q),                  \
                        STAGED ? lds : 0, s, G.nfree, G.f2g, G.sy, G.sz, G.m0, G.m1, sv, x, po, pn, y, b, part, cs,    \
                        st, G.stage)
-    if (D == 3 && (int)grid.x <= kSplitTiles) {
-        constexpr int Q = D == 3 ? kSplit : 1;
-        if (staged) GSX_Q(true, Q, FEW);
-        else GSX_Q(false, Q, 0);
-    } else if (!staged) {
-        GSX_Q(false, 1, 0);
-    } else if ((int)grid.x <= kPlaneTiles) {
-        GSX_Q(true, 1, FEW);
-    } else {
-        GSX_Q(true, 1, MANY);
+#define GSX_ST(Q, PLANES)                                                                                             \
+    {                                                                                                                 \
+        if (staged == 2) GSX_Q(2, Q, PLANES);                                                                         \
+        else if (staged) GSX_Q(1, Q, PLANES);                                                                         \
+        else GSX_Q(0, Q, 0);                                                                                          \
     }
+    if (split) {
+        constexpr int Q = D == 3 ? kSplit : 1;
+        GSX_ST(Q, FEW)
+    } else if (D == 3 ? (int)grid.x <= kPlaneTiles : (G.nfree + 255) / 256 <= kMaxPartials) {
+        GSX_ST(1, FEW)
+    } else {
+        GSX_ST(1, MANY)
+    }
+#undef GSX_ST
 #undef GSX_Q
     return hipGetLastError();
 }
