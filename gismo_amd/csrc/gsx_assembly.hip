@@ -1119,15 +1119,18 @@ __global__ void k_min_stage(const double *__restrict__ v, int64_t n, double *__r
 // (gsExprEvaluator::integral, src/gsAssembler/gsExprEvaluator.h:382-450).
 //
 // A thread owns one Gauss point column (gx in 2D, (gx, gy) in 3D) and walks a
-// chunk of kNormChunk elements along the last direction.  It contracts each
+// chunk of up to kNormChunk elements along the last direction (shorter ones where
+// there are few columns).  It contracts each
 // new row (plane) of control points and coefficients with its own 1D basis
 // values once and keeps the last p + 1 contracted rows in registers, so a
 // point costs one (p + 1)-term sum per field and derivative instead of
 // (p + 1)^d terms, there is no LDS traffic but the 1D tables of the last
 // direction, and a row's loads are shared by the points of p + 1 elements.
-// Bound by FP64 arithmetic (the sines and the divisions among it).
-// 16 patches of 200^2 elements, 2D degree 3 (10.2 M points), both norms:
-// 108 us; one block of 128 threads per element took 2974 us, and the sum of
+// Bound by FP64 arithmetic (the sines and the divisions among it); the
+// coefficients come gathered (k_norm_coefs), as a load through the numbering
+// stalls a chunk's first rows.
+// 16 patches of 200^2 elements, 2D degree 3 (10.2 M points), both norms with the
+// gather: 113 us (122 us with chunks of 8 and loads through the numbering); one block of 128 threads per element took 2974 us, and the sum of
 // its per-element results another 1175 us.
 // ---------------------------------------------------------------------------
 constexpr int kNormChunk = 8;   // at most

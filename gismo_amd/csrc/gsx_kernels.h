@@ -17,15 +17,14 @@ bool sf_supported(int d, int p);
 bool sf_mfma(int p);   // degrees with the matrix-core variant (the default row assembly)
 int64_t sf_table_doubles(int p, const int *nel);
 // doubles of the per-Gauss-point D (6 per point) of the matrix-core variant
-// (degrees 2, 3), 0 for the others
+// (degrees 2 to 4), 0 for the others
 int64_t sf_dq_doubles(int p, const int *nel);
-// tables, element load vectors + det check (+ D), stencil rows (FP64, all
-// slots of free rows whose column is in the patch); the tiling (nty, ntz)
-// is chosen here
 // raw rows, z sums of the load and per-block determinant minima (doubles)
 int64_t sf_raw_doubles(int p, const int *nb);
 int64_t sf_load_doubles(int p, const int *nel);
 int64_t sf_det_count(int p, const int *nel);
+// tables, geometry (D, determinant minima, load) and the raw rows of all basis
+// functions (upper half of the stencil); the tiling (nty, ntz) is chosen here
 hipError_t launch_sf_assemble(int p, const PatchDev *patches, const GaussTab &gt, double *tab, SfBox bx, double *R1,
                               double *detmin, double *Dq, double *raw, double *rhs, hipStream_t s);
 hipError_t launch_sf_finish(int p, const SfBox &bx, int nfree, const int *rowptr, const double *raw, double *s64,
@@ -246,12 +245,8 @@ hipError_t launch_cg2_dot_f64(int n, const double *a, const double *b, double *p
                               hipStream_t s);
 hipError_t launch_cg2_dot_f32(int n, const float *a, const float *b, double *part, const CGState *st,
                               hipStream_t s);
-// fast diagonalization: one mode product y_a = sum_i M[i*m + a] x_i along
-// direction dir of the m0 x m1 x m2 box (element (a,b,c) of x at
-// xo + a + b xs1 + c xs2, of y at yo + a + b ys1 + c ys2); with l0 != null
-// the result is divided by alpha + l0[a] + l1[b] (+ l2[c])
 // Two mode products per launch on the matrix cores (gsx_fd.hip), where
-// fd_fused says the strips fit the LDS.
+// fd_fused says so: where the strips fit the LDS and the box is not too thin.
 bool fd_fused(int d, int m0, int m1, int m2, size_t esz);
 hipError_t launch_fd_pair_f64(int m0, int m1, int m2, const double *M0, const double *M1, const double *x, int64_t xo,
                               int64_t xs1, int64_t xs2, double *y, int64_t yo, int64_t ys1, int64_t ys2,
@@ -265,6 +260,10 @@ hipError_t launch_fd_column_f64(int m0, int m1, int m2, const double *Q, const d
 hipError_t launch_fd_column_f32(int m0, int m1, int m2, const float *Q, const float *QT, const float *x, float *y,
                                 const double *l0, const double *l1, const double *l2, double alpha,
                                 const CGState *st, hipStream_t s);
+// fast diagonalization: one mode product y_a = sum_i M[i*m + a] x_i along
+// direction dir of the m0 x m1 x m2 box (element (a,b,c) of x at
+// xo + a + b xs1 + c xs2, of y at yo + a + b ys1 + c ys2); with l0 != null
+// the result is divided by alpha + l0[a] + l1[b] (+ l2[c])
 hipError_t launch_fd_mode_f64(int m0, int m1, int m2, int dir, const double *M, const double *x, int64_t xo,
                               int64_t xs1, int64_t xs2, double *y, int64_t yo, int64_t ys1, int64_t ys2,
                               const double *l0, const double *l1, const double *l2, double alpha,

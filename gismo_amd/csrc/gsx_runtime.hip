@@ -4041,9 +4041,6 @@ static SmoothCoef smooth_coef(const gsx_mg *mg, const MGLevel &V, int k, double 
     return c;
 }
 
-// m smoothing sweeps on level V with FP64 vectors (matrix values FP64, or
-// FP32 when v32: the finest level of a mixed cycle).  Jacobi ping-pongs x
-// and t (x may come back as t); the polynomial smoothers update x in place.
 // r = b - A x and one damped Jacobi step of a level, on its slices or its CSR
 // arrays; v32: FP64 vectors on the FP32 values
 static hipError_t level_residual64(const MGLevel &V, bool v32, const double *x, const double *b, double *r,
@@ -4084,6 +4081,9 @@ static hipError_t level_jacobi32(const MGLevel &V, const float *b, const float *
                                        (float)V.tau, zero, s);
 }
 
+// m smoothing sweeps on level V with FP64 vectors (matrix values FP64, or
+// FP32 when v32: the finest level of a mixed cycle).  Jacobi ping-pongs x
+// and t (x may come back as t); the polynomial smoothers update x in place.
 static gsx_status smooth64(gsx_mg *mg, MGLevel &V, double *&x, double *&t, const double *b, bool &zero, int m,
                            bool v32, bool post)
 {

@@ -24,10 +24,10 @@
 // of their x flags), then x into the accumulators of the p + 1 rows
 // ix = e .. e + p that element e touches.  Row e is complete after element e
 // and leaves the registers.  Only the upper half of the stencil (o >= 0
-// lexicographically in (z, y, x)) is accumulated; each value is stored at
-// (i, o) and at its mirror (i + o, -o), so the FP64 stencil is bitwise
-// symmetric.  All basis rows are computed (eliminated ones too) so that every
-// mirror exists; only free rows are stored.
+// lexicographically in (z, y, x)) is accumulated, into raw rows (SfRaw) of all
+// basis functions, eliminated ones too: k_sf_finish3d takes the lower half of a
+// free row from the raw rows that mirror it, so the FP64 stencil is bitwise
+// symmetric.
 #include "gsx_common.h"
 #include "gsx_kernels.h"
 #include "gsx_basis.h"
@@ -368,7 +368,7 @@ __global__ __launch_bounds__(256) void k_sfasm3d(const PatchDev *__restrict__ pa
 // The same row assembly with the three contractions on the FP64 matrix cores
 // (v_mfma_f64_16x16x4f64; operand layout: A[i][k] in lane i + 16 k, B[k][j]
 // in lane j + 16 k, result [i][j] in lane j + 16 (i % 4), element i / 4).
-// D comes precomputed per Gauss point (k_load3d).  A block of 8 waves owns a
+// D comes precomputed per Gauss point (k_geo3d).  A block of 8 waves owns a
 // 4 x 4 tile of basis rows in (y, z); per Gauss point column gx:
 //   z:  T1_arr[gy][c]   = sum_gz D_s(arr)[gz][gy] Wz_f(arr)[gz][c]        (c = (izl, oz >= 0))
 //   y:  T3_cls[e][c]    = sum_(a,b) in cls sum_gy Wy_f(a,b)[e][gy] T1_arr(a,b)[gy][c]   (e = (iyl, oy))

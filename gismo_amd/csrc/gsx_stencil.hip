@@ -148,8 +148,9 @@ __global__ void k_gather_from_grid(int nfree, const int *__restrict__ free2grid,
 // together with its mirror line (-dz, -dy): both read the same slot plane, the
 // mirror one at the rows shifted by the offset, so a block reads the plane at
 // the same point of its loop as the blocks that own those rows (up to p
-// z-planes back, on the same XCD through xcd_block) and the second read mostly
-// hits the L2.  Neighbours outside the free box contribute 0 (x is 0 there).
+// z-planes back, on the same XCD through xcd_block) and part of the second
+// reads hit the L2 (64^3 elements p = 3: FP32 moves 1.40 times the upper half
+// and the vectors, FP64 1.73 times).  Neighbours outside the free box contribute 0 (x is 0 there).
 // KIND 2 reads every slot from the row itself, with fewer index operations.
 //
 // The input of a block's 256 rows is staged in LDS, in planes dz and -dz: it is
@@ -165,8 +166,8 @@ __global__ void k_gather_from_grid(int nfree, const int *__restrict__ free2grid,
 // next tile's window before a tile's last plane is applied and, PLANES, the next
 // planes' first entries before a plane is.
 // Bound by the operator's bytes and the mirrored reads that miss the L2.  64^3
-// elements p = 3: FP32 46.1 us with the direction (49 us in two launches
-// before); FP64 residual 109 us (159 us reading all slots).  75^3 p = 2, FP64:
+// elements p = 3: FP32 50 us with the direction (5.5 TB/s), FP64 118 us with it
+// (5.7 TB/s), FP64 residual 110 us (159 us reading all slots).  75^3 p = 2, FP64:
 // 54.5 us with the direction (89 + 7 us reading all slots).
 // ---------------------------------------------------------------------------
 template <int D, int P, typename V, typename T, int KIND, int MODE, int STAGED, int Q, int PLANES>
